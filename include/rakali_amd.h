@@ -194,17 +194,15 @@ int rkg_total_mass(rkg_grid *g, double *mass);
 /* Waits for all queued work of this grid. */
 int rkg_sync(rkg_grid *g);
 
-/* Rows per tile segment of the stage kernels (1..64; 0, the default,
- * chooses 16 for grids of at least 8192 such tiles and 8 below).  The get
- * call returns the rows in use. */
+/* Rows per tile of the stage kernels (1..64; 0, the default, chooses 16 for
+ * grids of at least 8192 such tiles and 8 below).  The get call returns the
+ * rows in use. */
 int rkg_set_tile_rows(rkg_grid *g, int rows);
 int rkg_get_tile_rows(rkg_grid *g, int *rows);
-/* Whether the stage kernels try their fast path (wavefronts whose faces
- * and cells are all wet and subsonic skip the dry and shock branches and
- * use cheaper exact sequences; any other wavefront takes the general code,
- * so results are the same bits either way): 0 (default) when the launch
- * has at least 6144 tiles, where it pays; 1 always; -1 never.  A tuning and
- * testing knob with no counterpart in the reference. */
+/* How the stage kernels evaluate their rows: 0 (default) and 1 take the row
+ * path (selects, shared reciprocals; rows with values of extreme size use
+ * plain divisions), -1 plain divisions for every row.  The results are the
+ * same bits.  A testing knob with no counterpart in the reference. */
 int rkg_set_fast_path(rkg_grid *g, int mode);
 /* Keeps U^n of every step in three extra planes (24 B per cell per step of
  * extra traffic) so that RKG_FIELD_H0..HV0 can be read; off by default. */

@@ -93,12 +93,16 @@ def _run(cmd: list[str], out: Path, verbose: bool) -> Path:
 
 
 def unit_flags(src: Path) -> list[str]:
-    """Extra flags of one translation unit: the stage kernels (stage_feat*)
-    use LLVM's ILP-first machine scheduler, which is about 1 % faster on the
-    4096x4096 step at the same occupancy (three waves per SIMD, no spills);
-    it changes the instruction order, not the arithmetic."""
-    if src.stem.startswith("stage_feat"):
-        return ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
+    """Extra flags of one translation unit: the units with the step's stage
+    kernels switch off LLVM's machine-level loop-invariant code motion.  It
+    hoists the row loop's double constants and addresses into more scalar
+    registers than there are and spills them to lanes of a vector register;
+    every row then reads them back with vector instructions (300 v_readlane
+    in a stage kernel, 40 without; 4096x4096 step 1065 -> 1025 us).  Made
+    again in the loop they are scalar instructions, which issue beside the
+    vector ones.  The arithmetic does not change."""
+    if src.stem.startswith(("stage_feat", "rkg_ensemble", "rkg_adjoint")):
+        return ["-mllvm", "-disable-machine-licm"]
     return []
 
 

@@ -43,19 +43,6 @@ constexpr unsigned ADJ_MAGIC = 0x72616B41u;  // 'rakA'
 constexpr unsigned ADJ_DEAD = 0xDEADBEEFu;
 constexpr int AW = 60;                        // own columns per workgroup of k_adj_x
 
-// Own range [lo, hi) of block `s` when [0, n) is cut into blocks of `w`,
-// the last block holding at least two cells (a boundary ghost maps onto
-// the two cells next to the edge, which must belong to one tile).
-__host__ __device__ __forceinline__ void block_range(int n, int w, int s, int& lo, int& hi) {
-    const int nb = (n + w - 1) / w;
-    lo = s * w;
-    hi = min(lo + w, n);
-    if (nb >= 2 && n - (nb - 1) * w == 1) {
-        if (s == nb - 1) lo = n - 2;
-        if (s == nb - 2) hi = n - 2;
-    }
-}
-
 struct AdjStage {
     GridDesc d;                 // geometry, physics, bed, n field; ah.. = stage input V
     const double* un;           // U^n (3 planes), stage 2
@@ -211,7 +198,7 @@ __device__ __forceinline__ adj::S3 load_ldiv(const AdjStage& a, int x, int y) {
 }
 
 __device__ __forceinline__ Cell vload(const GridDesc& d, int x, int y, double eta) {
-    return load_cell<true>(d, d.ah, d.ahu, d.ahv, x, y, eta);
+    return load_cell(d, d.ah, d.ahu, d.ahv, x, y, eta);
 }
 
 // Adjoint of the row-y ghost at column x onto interior cells (x-direction
@@ -265,7 +252,7 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, int blk) {
     const int sx = blk % nstr, sy = blk / nstr;
     const int c0 = sx * WAVE;
     int j0, j1;
-    block_range(d.ny, a.ty, sy, j0, j1);
+    tile_range(d.ny, a.ty, sy, j0, j1);
     const bool xin = c0 + lane < d.nx;
     const int x = xin ? c0 + lane : d.nx - 1;   // lanes past the edge repeat the last column, unwritten
     // rows j0 - 3 .. j1 + 2 are read; only ghost rows need the tide (whose
@@ -392,7 +379,7 @@ __device__ __forceinline__ void adj_x(const AdjStage& a, int blk) {
     const int nstr = (d.nx + AW - 1) / AW;
     const int sx = blk % nstr, sy = blk / nstr;
     int c0, c1;
-    block_range(d.nx, AW, sx, c0, c1);
+    tile_range(d.nx, AW, sx, c0, c1);
     const int r0 = sy * a.xrows, r1 = min(r0 + a.xrows, d.ny);
     const int x = c0 - 2 + lane;
     const bool own_col = x >= c0 && x < c1;
@@ -779,13 +766,13 @@ struct RecTileOf {
     __device__ int3 operator()(const GridDesc&) const { return make_int3(t.strip, t.seg, t.leader); }
 };
 
-template <int STAGE, bool HLLC, bool FASTK>
+template <int STAGE, bool HLLC>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_replay_batch(
     const GridDesc* __restrict__ descs, const RecTile* __restrict__ tiles, const int* __restrict__ parity) {
-    __shared__ TileLds L;
+    __shared__ TileRing ring;
     const RecTile t = tiles[blockIdx.x];
     const GridDesc& d = descs[t.member];
-    stage_tile<STAGE, HLLC, true, true, RecTileOf, 0, FASTK>(d, L, parity[t.member], MODE_STEP, d.t_end, RecTileOf{t});
+    stage_tile<STAGE, HLLC, true, true, RecTileOf>(d, ring, parity[t.member], MODE_STEP, d.t_end, RecTileOf{t});
 }
 
 __global__ __launch_bounds__(256) void k_gauge_seed_batch(const SeedArgs* __restrict__ sa,
@@ -915,12 +902,8 @@ template <int STAGE>
 void launch_rec(rkg_grid* g, const GridDesc& d, int p, hipStream_t st) {
     const int ntiles = d.nstrips * d.nsegs;
     const double tlim = g->cfg.t_end;
-    if (g->cfg.use_hllc && d.fast)
-        hipLaunchKernelGGL((k_stage<STAGE, true, true, true, 0, true>), dim3(ntiles), dim3(WAVE), 0, st, d, p, MODE_STEP, tlim);
-    else if (g->cfg.use_hllc)
+    if (g->cfg.use_hllc)
         hipLaunchKernelGGL((k_stage<STAGE, true, true, true>), dim3(ntiles), dim3(WAVE), 0, st, d, p, MODE_STEP, tlim);
-    else if (d.fast)
-        hipLaunchKernelGGL((k_stage<STAGE, false, true, true, 0, true>), dim3(ntiles), dim3(WAVE), 0, st, d, p, MODE_STEP, tlim);
     else
         hipLaunchKernelGGL((k_stage<STAGE, false, true, true>), dim3(ntiles), dim3(WAVE), 0, st, d, p, MODE_STEP, tlim);
 }
@@ -1615,20 +1598,12 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
             const GridDesc* r1 = (const GridDesc*)(d + oRec1);
             const GridDesc* r2 = (const GridDesc*)(d + oRec2);
             const int* par = (const int*)(d + oPar);
-            // one launch over every member: the fast path by the total tile count
-            const bool fk = (long long)nrec >= FAST_MIN_TILES;
-            if (hllc && fk) {
-                hipLaunchKernelGGL((k_replay_batch<1, true, true>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
-                hipLaunchKernelGGL((k_replay_batch<2, true, true>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
-            } else if (hllc) {
-                hipLaunchKernelGGL((k_replay_batch<1, true, false>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
-                hipLaunchKernelGGL((k_replay_batch<2, true, false>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
-            } else if (fk) {
-                hipLaunchKernelGGL((k_replay_batch<1, false, true>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
-                hipLaunchKernelGGL((k_replay_batch<2, false, true>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
+            if (hllc) {
+                hipLaunchKernelGGL((k_replay_batch<1, true>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
+                hipLaunchKernelGGL((k_replay_batch<2, true>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
             } else {
-                hipLaunchKernelGGL((k_replay_batch<1, false, false>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
-                hipLaunchKernelGGL((k_replay_batch<2, false, false>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
+                hipLaunchKernelGGL((k_replay_batch<1, false>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
+                hipLaunchKernelGGL((k_replay_batch<2, false>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
             }
         }
         for (int k = Ks - 1; k >= 0; --k) {

@@ -583,7 +583,7 @@ int rkg_set_mass_budget(rkg_grid* g, int enable) {
     if (enable && !g->mpart) {
         // room for the tiles of both stages at any tile height, for the
         // flux and the sponge sums
-        const long long cap = (long long)((g->cfg.nx + WAVE - 1) / WAVE) * g->cfg.ny;
+        const long long cap = (long long)((g->cfg.nx + OWN - 1) / OWN) * g->cfg.ny;
         HIP_TRY(hipMalloc((void**)&g->mpart, 4 * cap * sizeof(double)));
         g->mpart_cap = cap;
         CtrlSlot c;
@@ -756,7 +756,7 @@ int rkg_get_stream(rkg_grid* g, void** stream) {
 
 int rkg_set_fast_path(rkg_grid* g, int mode) {
     if (!valid(g)) return RKG_ERR_BAD_HANDLE;
-    if (mode < -1 || mode > 1) { set_error("fast path mode must be -1 (never), 0 (by tile count) or 1 (always)"); return RKG_ERR_RANGE; }
+    if (mode < -1 || mode > 1) { set_error("fast path mode must be -1 (plain divisions), 0 or 1 (the row path)"); return RKG_ERR_RANGE; }
     g->fast_mode = mode;
     return RKG_OK;
 }

@@ -43,16 +43,16 @@ struct TileOf {
 
 // The tile loop of the persistent variant needs about 250 VGPRs to keep
 // the tile body free of spills, so it runs at two waves per SIMD.
-template <int STAGE, bool HLLC, bool PERSISTENT, bool FASTK>
+template <int STAGE, bool HLLC, bool PERSISTENT>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(PERSISTENT ? 2 : RKG_WAVES_PER_EU, 8))) void k_stage_batch(
     const GridDesc* __restrict__ descs, const BatchTile* __restrict__ tiles, int ntiles, int p,
     unsigned* __restrict__ queue) {
-    __shared__ TileLds L;
+    __shared__ TileRing ring;
     if (!PERSISTENT) {
         const int t = xcd_tile(blockIdx.x, ntiles);
         const BatchTile bt = tiles[t];
-        stage_tile<STAGE, HLLC, false, false, TileOf, 0, FASTK>(descs[bt.member], L, p, MODE_STEP,
-                                                              descs[bt.member].t_end, TileOf{bt});
+        stage_tile<STAGE, HLLC, false, false, TileOf>(descs[bt.member], ring, p, MODE_STEP,
+                                                      descs[bt.member].t_end, TileOf{bt});
         return;
     }
     // The other stage's counter is idle during this launch: clear it for
@@ -65,9 +65,9 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(PERSISTENT
         const int t = __builtin_amdgcn_readfirstlane((int)slot);
         if (t >= ntiles) break;
         const BatchTile bt = tiles[t];
-        stage_tile<STAGE, HLLC, false, false, TileOf, 0, FASTK>(descs[bt.member], L, p, MODE_STEP,
-                                                              descs[bt.member].t_end, TileOf{bt});
-        __syncthreads();   // the next tile rewrites the LDS buffers and the slot
+        stage_tile<STAGE, HLLC, false, false, TileOf>(descs[bt.member], ring, p, MODE_STEP,
+                                                      descs[bt.member].t_end, TileOf{bt});
+        __syncthreads();   // the next tile rewrites the slot
     }
 }
 
@@ -116,6 +116,7 @@ GridDesc ens_desc(rkg_ensemble* e, int m) {
     const rkg_config& c = e->cfg[m];
     d.nx = c.nx; d.ny = c.ny; d.pitch = e->pitch[m];
     d.dx = c.dx; d.dy = c.dy;
+    d.sdx = spacing(c.dx); d.sdy = spacing(c.dy);
     d.ah = ens_plane(e, m, 0); d.ahu = ens_plane(e, m, 1); d.ahv = ens_plane(e, m, 2);
     d.bh = ens_plane(e, m, 3); d.bhu = ens_plane(e, m, 4); d.bhv = ens_plane(e, m, 5);
     d.bed = ens_plane(e, m, 6);
@@ -134,7 +135,7 @@ GridDesc ens_desc(rkg_ensemble* e, int m) {
     d.dt_fixed = c.dt_fixed; d.t_end = c.t_end;
     d.cfl_interval = c.cfl_interval;
     d.ty = e->ty;
-    d.nstrips = (c.nx + WAVE - 1) / WAVE;
+    d.nstrips = (c.nx + OWN - 1) / OWN;
     d.nsegs = (c.ny + e->ty - 1) / e->ty;
     d.ctrl = e->ctrl + 2 * m;
     d.ssp_coeff = 1.0;  // ensembles run SSP-RK2
@@ -190,21 +191,14 @@ int refresh_speeds(rkg_ensemble* e) {
     return RKG_OK;
 }
 
-template <int STAGE, bool HLLC, bool FASTK>
-void launch_one_k(rkg_ensemble* e, int p) {
-    if (e->schedule == 1)
-        hipLaunchKernelGGL((k_stage_batch<STAGE, HLLC, true, FASTK>), dim3(e->persistent_blocks), dim3(WAVE), 0,
-                           e->stream, e->descs, e->tiles, e->ntiles, p, e->queue);
-    else
-        hipLaunchKernelGGL((k_stage_batch<STAGE, HLLC, false, FASTK>), dim3(e->ntiles), dim3(WAVE), 0, e->stream,
-                           e->descs, e->tiles, e->ntiles, p, e->queue);
-}
-
-// The kernels with the fast path when the launch holds enough tiles.
 template <int STAGE, bool HLLC>
 void launch_one(rkg_ensemble* e, int p) {
-    if ((long long)e->ntiles >= FAST_MIN_TILES) launch_one_k<STAGE, HLLC, true>(e, p);
-    else launch_one_k<STAGE, HLLC, false>(e, p);
+    if (e->schedule == 1)
+        hipLaunchKernelGGL((k_stage_batch<STAGE, HLLC, true>), dim3(e->persistent_blocks), dim3(WAVE), 0,
+                           e->stream, e->descs, e->tiles, e->ntiles, p, e->queue);
+    else
+        hipLaunchKernelGGL((k_stage_batch<STAGE, HLLC, false>), dim3(e->ntiles), dim3(WAVE), 0, e->stream,
+                           e->descs, e->tiles, e->ntiles, p, e->queue);
 }
 
 void launch_stage(rkg_ensemble* e, int stage, int p) {

@@ -51,7 +51,7 @@ struct rkg_grid {
     double* mass_host;   // pinned [1]
     int parity;
     int ty;              // rows per stage tile, 0 = chosen from the grid size
-    int fast_mode;       // fast path: 0 by the launch's tile count, 1 always, -1 never
+    int fast_mode;       // rkg_set_fast_path: -1 runs every row with plain divisions
     bool speed_stale;
     bool prof;             // time each stage launch with events
     hipEvent_t ev[3];
@@ -133,20 +133,21 @@ inline double* field_ptr(rkg_grid* g, int field) {
     }
 }
 
-// Rows per stage tile: the set value, or (0) 16 rows when the grid has
-// at least 8192 tiles of 16 rows (several waves of tiles per wave slot, so
-// longer tiles waste less on halos), else 8 (smaller grids run one tile
-// per slot, and shorter tiles finish sooner).
 // Rows per stage tile by grid size: 16 once a grid has 8192 tiles of 16
 // rows, else 8 (a small grid needs more, shorter tiles to fill the chip).
 inline int default_tile_rows(int nx, int ny) {
-    const long long strips = (nx + 63) / 64;
+    const long long strips = (nx + OWN - 1) / OWN;
     return strips * ((ny + 15) / 16) >= 8192 ? 16 : 8;
 }
 
+// A tile next to a one-row tile at a south Chapman edge would read a ghost
+// row that depends on what the edge's tile overwrites: two rows at least
+// there (tile_range sees to the north edge).
 inline int tile_rows_of(const rkg_grid* g) {
-    if (g->ty > 0) return g->ty;
-    return default_tile_rows(g->cfg.nx, g->cfg.ny);
+    const int ty = g->ty > 0 ? g->ty : default_tile_rows(g->cfg.nx, g->cfg.ny);
+    bool chapman = false;
+    for (int s = 0; s < 4; ++s) chapman = chapman || g->cfg.bc[s] == RKG_BC_CHAPMAN;
+    return chapman && ty < 2 ? 2 : ty;
 }
 
 // apply_sponge does something (rki_kernel_sponge.F90:42-47 and a sponge edge).
@@ -164,6 +165,7 @@ inline GridDesc desc_of_config(const rkg_config& c, long long pitch, int ty) {
     memset(&d, 0, sizeof d);
     d.nx = c.nx; d.ny = c.ny; d.pitch = pitch;
     d.dx = c.dx; d.dy = c.dy;
+    d.sdx = spacing(c.dx); d.sdy = spacing(c.dy);
     d.plane = pitch * (long long)c.ny;
     d.g = c.g; d.cfl = c.cfl; d.manning_n = c.manning_n; d.coriolis_f = c.coriolis_f;
     d.use_hllc = c.use_hllc;
@@ -178,9 +180,8 @@ inline GridDesc desc_of_config(const rkg_config& c, long long pitch, int ty) {
     d.dt_fixed = c.dt_fixed; d.t_end = c.t_end;
     d.cfl_interval = c.cfl_interval;
     d.ty = ty;
-    d.nstrips = (c.nx + WAVE - 1) / WAVE;
+    d.nstrips = (c.nx + OWN - 1) / OWN;
     d.nsegs = (c.ny + d.ty - 1) / d.ty;
-    d.fast = (long long)d.nstrips * d.nsegs >= FAST_MIN_TILES ? 1 : 0;
     d.ssp_coeff = 1.0;
     return d;
 }
@@ -212,7 +213,7 @@ inline GridDesc make_desc(rkg_grid* g) {
         d.fdpy = g->frc + 5 * g->plane;
     }
     d.ssp_coeff = g->scheme == RKG_TIME_RK43 ? 2.0 : 1.0;  // rki_timestepper.F90:60-100
-    if (g->fast_mode != 0) d.fast = g->fast_mode > 0 ? 1 : 0;
+    d.plain_rows = g->fast_mode < 0 ? 1 : 0;
     return d;
 }
 

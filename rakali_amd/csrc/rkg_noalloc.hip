@@ -91,7 +91,10 @@ extern "C" int rkg_step_noalloc(const rkg_config* cfg, double* h, double* hu, do
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
 
-    GridDesc d = desc_of_config(*cfg, pitch, default_tile_rows(cfg->nx, cfg->ny));
+    bool chapman = false;
+    for (int k = 0; k < 4; ++k) chapman = chapman || cfg->bc[k] == RKG_BC_CHAPMAN;
+    const int ty = default_tile_rows(cfg->nx, cfg->ny);
+    GridDesc d = desc_of_config(*cfg, pitch, chapman && ty < 2 ? 2 : ty);
     d.ah = h; d.ahu = hu; d.ahv = hv;
     d.o2h = h; d.o2hu = hu; d.o2hv = hv;
     d.bed = b;
@@ -99,8 +102,6 @@ extern "C" int rkg_step_noalloc(const rkg_config* cfg, double* h, double* hu, do
     d.bhu = d.bh + cells;
     d.bhv = d.bhu + cells;
     d.ctrl = reinterpret_cast<CtrlSlot*>(s);
-    bool chapman = false;
-    for (int k = 0; k < 4; ++k) chapman = chapman || cfg->bc[k] == RKG_BC_CHAPMAN;
     const int ntiles = d.nstrips * d.nsegs;
     const bool hllc = cfg->use_hllc != 0;
 

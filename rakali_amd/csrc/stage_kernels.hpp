@@ -50,23 +50,29 @@ __device__ __forceinline__ SourceTerms make_src(const GridDesc& d, double dt) {
     return s;
 }
 
-__device__ __forceinline__ bool tile_is_interior(const GridDesc& d, int strip, int seg) {
-    const int c0 = strip * WAVE;
-    const int j0 = seg * d.ty;
-    const int j1 = min(j0 + d.ty, d.ny);
-    return c0 >= 2 && c0 + WAVE + 1 < d.nx && j0 >= 2 && j1 + 1 < d.ny;
-}
-
 // One tile of one stage of one grid.  `where(d)` gives the tile as
 // (strip, segment, leader); the leader is the single tile per grid and
 // launch that advances the control slot.  STAGE 1 and 2 are the fused
 // SSP-RK2 stages; STAGE 3 is one stage `gs` of a generic SSP scheme.
-template <int STAGE, bool HLLC, bool NF, bool REC, class Where, int FEAT = 0, bool FASTK = false>
-__device__ __forceinline__ void stage_tile(const GridDesc& d, TileLds& L, int p, int mode, double tlim,
-                                           Where where, const GenStage& gs = GenStage{}) {
+template <int STAGE, bool HLLC, bool NF, bool REC, class Where, int FEAT = 0>
+__device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, int p, int mode, double tlim, Where where, const GenStage& gs = GenStage{}) {
     const int3 w = where(d);
     const bool leader = w.z != 0;
+    const int strip = w.x, seg = w.y;
     StageCtx s;
+    int x0, x1;
+    tile_range(d.nx, OWN, strip, x0, x1);
+    tile_range(d.ny, d.ty, seg, s.row0, s.row1);
+    const bool west = x0 < HALO, east = x0 + OWN + HALO > d.nx;
+    const bool south = s.row0 < HALO, north = s.row1 + HALO > d.ny;
+    const bool edge = west || east || south || north;
+    // the stage's input and the first rows of the march, before the clock
+    if (STAGE == 1) { s.ih = d.ah; s.ihu = d.ahu; s.ihv = d.ahv; }
+    else if (STAGE == 2) { s.ih = d.bh; s.ihu = d.bhu; s.ihv = d.bhv; }
+    else { s.ih = gs.ih; s.ihu = gs.ihu; s.ihv = gs.ihv; }
+    const int c = x0 - HALO + (int)threadIdx.x;
+    const LaneSource lsrc = edge ? lane_source<true>(d, c) : lane_source<false>(d, c);
+    const FirstRows first = edge ? first_rows<true>(d, s, lsrc, s.row0) : first_rows<false>(d, s, lsrc, s.row0);
     s.alpha = 0.0; s.a_prev = 1.0;
     s.blend = false; s.first = false; s.last = false;
     s.radiate = false; s.prev_h = nullptr; s.bc_dt = 0.0;
@@ -100,11 +106,9 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileLds& L, int p,
         if (!active) return;
         s.bc_dt = dt;   // bc%dt = state%dt, rki_solver.F90:748
         if (STAGE == 1) {
-            s.ih = d.ah; s.ihu = d.ahu; s.ihv = d.ahv;
             s.oh = d.bh; s.ohu = d.bhu; s.ohv = d.bhv;
             s.dt = dt;
         } else {
-            s.ih = gs.ih; s.ihu = gs.ihu; s.ihv = gs.ihv;
             s.oh = gs.oh; s.ohu = gs.ohu; s.ohv = gs.ohv;
             s.dt = gs.beta * dt;
         }
@@ -113,7 +117,6 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileLds& L, int p,
         const CtrlSlot cp = d.ctrl[p];
         const CtrlSlot cq = d.ctrl[1 - p];
         if (!cq.active) return;
-        s.ih = gs.ih; s.ihu = gs.ihu; s.ihv = gs.ihv;
         s.oh = gs.oh; s.ohu = gs.ohu; s.ohv = gs.ohv;
         s.dt = gs.beta * cq.dt;
         t_tide = cp.t + gs.c * cq.dt;  // bc%time = t_base + c_i dt
@@ -123,7 +126,6 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileLds& L, int p,
     } else {
         const CtrlSlot cq = d.ctrl[1 - p];
         if (!cq.active) return;
-        s.ih = d.bh; s.ihu = d.bhu; s.ihv = d.bhv;
         s.oh = d.o2h; s.ohu = d.o2hu; s.ohv = d.o2hv;
         s.dt = cq.dt;
         t_tide = cq.t;  // bc%time = t + dt
@@ -139,19 +141,16 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileLds& L, int p,
         s.last = gs.last != 0;
     }
     s.src = make_src(d, s.dt);
-    s.rdx = recip(d.dx);
-    s.rdy = recip(d.dy);
-    const int strip = w.x, seg = w.y;
-    s.row0 = seg * d.ty;
-    s.row1 = min(s.row0 + d.ty, d.ny);
     double smax, fsum, ssum;
-    if (tile_is_interior(d, strip, seg)) {
-        // no ghost cells: the tide (a correctly rounded sine, a long
-        // dependent chain) is not needed
-        smax = process_tile<STAGE, HLLC, false, NF, REC, FEAT, FASTK>(d, s, L, strip, seg, fsum, ssum);
+    if (!edge) {
+        smax = process_tile<STAGE, HLLC, false, NF, REC, FEAT>(d, s, ring, lsrc, first, x0, x1, s.row0, s.row1, fsum, ssum);
     } else {
-        s.eta_tidal = tidal_eta(d, t_tide);
-        smax = process_tile<STAGE, HLLC, true, NF, REC, FEAT, FASTK>(d, s, L, strip, seg, fsum, ssum);
+        // the tide (a correctly rounded sine, a long dependent chain) only
+        // where the tile reads ghost cells of a tidal edge
+        if ((west && d.bc[0] == BC_TIDAL) || (east && d.bc[1] == BC_TIDAL) || (south && d.bc[2] == BC_TIDAL) ||
+            (north && d.bc[3] == BC_TIDAL))
+            s.eta_tidal = tidal_eta(d, t_tide);
+        smax = process_tile<STAGE, HLLC, true, NF, REC, FEAT>(d, s, ring, lsrc, first, x0, x1, s.row0, s.row1, fsum, ssum);
     }
     if (STAGE == 2 || STAGE == 3) {
         smax = wave_max(smax);
@@ -178,19 +177,18 @@ struct SingleGridTile {
     }
 };
 
-// FEAT: FEAT_FORCING / FEAT_SPONGE source terms.  FASTK: the fast path
-// compiled in (launches with d.fast set, FAST_MIN_TILES).
-template <int STAGE, bool HLLC, bool NF, bool REC, int FEAT = 0, bool FASTK = false>
+// FEAT: FEAT_FORCING / FEAT_SPONGE / FEAT_CHAPMAN source terms.
+template <int STAGE, bool HLLC, bool NF, bool REC, int FEAT = 0>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_stage(GridDesc d, int p, int mode, double tlim) {
-    __shared__ TileLds L;
-    stage_tile<STAGE, HLLC, NF, REC, SingleGridTile, FEAT, FASTK>(d, L, p, mode, tlim, SingleGridTile{});
+    __shared__ TileRing ring;
+    stage_tile<STAGE, HLLC, NF, REC, SingleGridTile, FEAT>(d, ring, p, mode, tlim, SingleGridTile{});
 }
 
 // One stage of a generic SSP scheme, single grid.
 template <bool HLLC, bool NF, int FEAT = 0>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_stage_gen(GridDesc d, GenStage gs, int p, int mode, double tlim) {
-    __shared__ TileLds L;
-    stage_tile<3, HLLC, NF, false, SingleGridTile, FEAT>(d, L, p, mode, tlim, SingleGridTile{}, gs);
+    __shared__ TileRing ring;
+    stage_tile<3, HLLC, NF, false, SingleGridTile, FEAT>(d, ring, p, mode, tlim, SingleGridTile{}, gs);
 }
 
 // Resets control slot p to time t / step count n with an empty speed max;
@@ -262,14 +260,13 @@ __global__ __launch_bounds__(256) void k_budget(CtrlSlot* ctrl, int p, const dou
 __global__ __launch_bounds__(256) void k_euler_finish(GridDesc d, int p) {
     if (!d.ctrl[1 - p].active) return;
     double m = 0.0;
-    const Recip rdx = recip(d.dx), rdy = recip(d.dy);
     const long long n = (long long)d.nx * d.ny;
     for (long long k = blockIdx.x * 256ll + threadIdx.x; k < n; k += (long long)gridDim.x * 256) {
         const int j = (int)(k / d.nx), i = (int)(k % d.nx);
         const long long o = (long long)j * d.pitch + i;
         const double h = d.bh[o], hu = d.bhu[o], hv = d.bhv[o];
         d.ah[o] = h; d.ahu[o] = hu; d.ahv[o] = hv;
-        m = dmax(m, cfl_speed<true>(d.g, rdx, rdy, h, hu, hv));
+        m = dmax(m, cfl_speed(d.g, d.dx, d.dy, h, hu, hv));
     }
     m = wave_max(m);
     if ((threadIdx.x & (WAVE - 1)) == 0 && m > 0.0)
@@ -280,12 +277,11 @@ __global__ __launch_bounds__(256) void k_euler_finish(GridDesc d, int p) {
 // rki_kernel_timestep.F90:53-70).
 __global__ __launch_bounds__(256) void k_init_speed(GridDesc d, int p) {
     double m = 0.0;
-    const Recip rdx = recip(d.dx), rdy = recip(d.dy);
     const long long n = (long long)d.nx * d.ny;
     for (long long k = blockIdx.x * 256ll + threadIdx.x; k < n; k += (long long)gridDim.x * 256) {
         const int j = (int)(k / d.nx), i = (int)(k % d.nx);
         const long long o = (long long)j * d.pitch + i;
-        m = dmax(m, cfl_speed<true>(d.g, rdx, rdy, d.ah[o], d.ahu[o], d.ahv[o]));
+        m = dmax(m, cfl_speed(d.g, d.dx, d.dy, d.ah[o], d.ahu[o], d.ahv[o]));
     }
     m = wave_max(m);
     if ((threadIdx.x & (WAVE - 1)) == 0 && m > 0.0)

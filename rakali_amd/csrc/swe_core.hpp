@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cstring>
+
 #include "crmath.hpp"
 
 namespace rk {
@@ -60,23 +62,26 @@ __device__ __forceinline__ double pow4(double x) { return ((x * x) * x) * x; }
 // from the exponent extremes), v_rcp, two Newton refinements of the
 // reciprocal, a product, a residual fma and the correction fma
 // (v_div_fmas), then v_div_fixup (identity for finite, non-zero operands).
-// Recip keeps the refined reciprocal so each further quotient by the same
+// Recip keeps the refined reciprocal, so each further quotient by the same
 // denominator costs a product and two fmas and returns the same bits as
 // `n / d`.  The residual is formed as -fma(d, q0, -n) so that zero
-// numerators keep their sign.  The unscaled sequence equals the IEEE
-// quotient while |n| >= 2^-969 (or n = 0) and the denominator lies in
-// [1e-8, 1e12]; callers guarantee the numerator bound by running a row
-// with EXACT = true (plain division) whenever a cell of its stencil holds
-// a non-zero h, hu, hv or b below 2^-300 in magnitude (see tiny()).
+// numerators keep their sign.  The refinement is one cubic step, an fma
+// fewer than two Newton steps: v_rcp_f64 is within 2^-24.3 (measured over
+// 6e9 operands), so y0 (1 + e + e^2) is 1 / d within 2^-72 before its
+// rounding, as close as two steps come in effect; the quotients agreed with
+// the division on all of those operands.  The unscaled sequence equals the
+// IEEE quotient while |n| >= 2^-969 (or n = 0) and the denominator is far
+// from the exponent extremes; callers guarantee the numerator bound by
+// running a row with EXACT = true (plain division) whenever a cell of its
+// stencil holds a value that is unbounded().
 struct Recip {
     double d, y;
 };
 
 __device__ __forceinline__ Recip recip(double d) {
     const double y0 = __builtin_amdgcn_rcp(d);
-    const double y1 = fma(y0, fma(-d, y0, 1.0), y0);
-    const double y2 = fma(y1, fma(-d, y1, 1.0), y1);
-    return Recip{d, y2};
+    const double e = fma(-d, y0, 1.0);
+    return Recip{d, fma(y0, fma(e, e, e), y0)};
 }
 
 template <bool EXACT>
@@ -87,16 +92,43 @@ __device__ __forceinline__ double rdiv(double n, const Recip& r) {
     return fma(-t, r.y, q0);
 }
 
-// Non-zero and below 2^-300 in magnitude: a value for which some quotient
-// of the step could leave the range where rdiv<false> is exact.
-__device__ __forceinline__ bool tiny(double x) { return fabs(x) < 0x1p-300 && x != 0.0; }
+// Division by a grid spacing.  Where the spacing has at most 50 significant
+// bits (`two_op`; 10, 20, 62.5 and the like), the quotient is
+// fma(n, yh, n yl) with 1/d = yh + yl: the value before its rounding is
+// within 2^-52 ulp of n / d, and such a quotient is at least 2^-51 ulp from
+// every rounding boundary (n 2^t - odd D is a non-zero integer, over D <
+// 2^50), so the result is the IEEE quotient at two operations instead of
+// three.  Another spacing takes rdiv.
+struct Spacing {
+    Recip r;
+    double yl;
+    bool two_op;
+};
 
-// Non-zero and outside [2^-300, 2^40] in magnitude, or not finite: besides
-// tiny values, the values for which the fast path's range arguments (below)
-// do not hold; the kernels that carry the fast path test their rows with it.
+inline Spacing spacing(double d) {   // on the host, once per launch
+    Spacing s;
+    uint64_t u;
+    memcpy(&u, &d, sizeof u);
+    s.r.d = d;
+    s.r.y = 1.0 / d;
+    s.yl = __builtin_fma(-d, s.r.y, 1.0) * s.r.y;   // the residual is exact
+    s.two_op = (u & 7) == 0;
+    return s;
+}
+
+template <bool TWO>
+__device__ __forceinline__ double sdiv(double n, const Spacing& s) {
+    return TWO ? fma(n, s.r.y, n * s.yl) : rdiv<false>(n, s.r);
+}
+
+// A depth or momentum that is non-zero and outside [2^-300, 2^40] in
+// magnitude, or a bed above 2^40, or a value that is not finite: one for which
+// some quotient of the step could leave the range where rdiv<false> is
+// exact, or another range argument of the row path (below) does not hold.  (A
+// tiny bed next to ordinary depths changes none of them.)
 __device__ __forceinline__ bool unbounded(double x) {
     const double a = fabs(x);
-    return x != 0.0 && !(a >= 0x1p-300 && a <= 0x1p40);
+    return (x != 0.0) & !((a >= 0x1p-300) & (a <= 0x1p40));
 }
 
 // Square root of a finite x >= 2^-767: the correctly rounded sequence the
@@ -116,11 +148,8 @@ __device__ __forceinline__ double sqrt_pos(double x) {
     d = fma(-g, g, x);
     return fma(d, h, g);
 }
-__device__ __forceinline__ bool tiny(const Cell& c) {
-    return tiny(c.h) || tiny(c.hu) || tiny(c.hv) || tiny(c.b);
-}
 __device__ __forceinline__ bool unbounded(const Cell& c) {
-    return unbounded(c.h) || unbounded(c.hu) || unbounded(c.hv) || unbounded(c.b);
+    return unbounded(c.h) | unbounded(c.hu) | unbounded(c.hv) | !(fabs(c.b) <= 0x1p40);
 }
 
 // minmod, rki_kernel_flux.F90:380-393
@@ -130,13 +159,13 @@ __device__ __forceinline__ double minmod(double a, double b) {
 }
 
 // HLL / HLLC normal flux in x: rki_kernel_flux.F90:410-495 and 584-684.
-template <bool HLLC, bool EXACT>
+template <bool HLLC>
 __device__ __forceinline__ void riemann_x(double g, double h_l, double hu_l, double hv_l,
                                           double h_r, double hu_r, double hv_r,
                                           double& f_h, double& f_hu, double& f_hv) {
     double u_l = 0.0, v_l = 0.0, u_r = 0.0, v_r = 0.0;
-    if (h_l > DRY_TOLERANCE) { const Recip r = recip(h_l); u_l = rdiv<EXACT>(hu_l, r); v_l = rdiv<EXACT>(hv_l, r); }
-    if (h_r > DRY_TOLERANCE) { const Recip r = recip(h_r); u_r = rdiv<EXACT>(hu_r, r); v_r = rdiv<EXACT>(hv_r, r); }
+    if (h_l > DRY_TOLERANCE) { u_l = hu_l / h_l; v_l = hv_l / h_l; }
+    if (h_r > DRY_TOLERANCE) { u_r = hu_r / h_r; v_r = hv_r / h_r; }
     const double a_l = sqrt(g * fmax0(h_l));
     const double a_r = sqrt(g * fmax0(h_r));
     double s_l, s_r;
@@ -177,13 +206,13 @@ __device__ __forceinline__ void riemann_x(double g, double h_l, double hu_l, dou
 
 // HLL / HLLC normal flux in y: rki_kernel_flux.F90:497-582 and 686-783.
 // Arguments are (h, hu, hv) of the bottom then the top state, as there.
-template <bool HLLC, bool EXACT>
+template <bool HLLC>
 __device__ __forceinline__ void riemann_y(double g, double h_b, double hu_b, double hv_b,
                                           double h_t, double hu_t, double hv_t,
                                           double& g_h, double& g_hu, double& g_hv) {
     double u_b = 0.0, v_b = 0.0, u_t = 0.0, v_t = 0.0;
-    if (h_b > DRY_TOLERANCE) { const Recip r = recip(h_b); u_b = rdiv<EXACT>(hu_b, r); v_b = rdiv<EXACT>(hv_b, r); }
-    if (h_t > DRY_TOLERANCE) { const Recip r = recip(h_t); u_t = rdiv<EXACT>(hu_t, r); v_t = rdiv<EXACT>(hv_t, r); }
+    if (h_b > DRY_TOLERANCE) { u_b = hu_b / h_b; v_b = hv_b / h_b; }
+    if (h_t > DRY_TOLERANCE) { u_t = hu_t / h_t; v_t = hv_t / h_t; }
     const double a_b = sqrt(g * fmax0(h_b));
     const double a_t = sqrt(g * fmax0(h_t));
     double s_l, s_r;
@@ -259,21 +288,21 @@ __device__ __forceinline__ void cell_states(const Cell& m, const Cell& c, const 
 // state R of its right cell (bed bR): Audusse hydrostatic reconstruction
 // (rki_kernel_flux.F90:208-210), velocities (extract_velocity, :395-408)
 // and the HLL/HLLC flux of the h_hyd-weighted momenta (:216-224).
-template <bool HLLC, bool YDIR, bool EXACT>
+template <bool HLLC, bool YDIR>
 __device__ __forceinline__ Face face_flux(double g, const FState& L, double bL, const FState& R,
                                           double bR) {
     const double b_max = dmax(bL, bR);
     const double h_hyd_l = fmax0(L.h + bL - b_max);
     const double h_hyd_r = fmax0(R.h + bR - b_max);
     double u_l = 0.0, v_l = 0.0, u_r = 0.0, v_r = 0.0;
-    if (L.h > DRY_TOLERANCE) { const Recip r = recip(L.h); u_l = rdiv<EXACT>(L.hu, r); v_l = rdiv<EXACT>(L.hv, r); }
-    if (R.h > DRY_TOLERANCE) { const Recip r = recip(R.h); u_r = rdiv<EXACT>(R.hu, r); v_r = rdiv<EXACT>(R.hv, r); }
+    if (L.h > DRY_TOLERANCE) { u_l = L.hu / L.h; v_l = L.hv / L.h; }
+    if (R.h > DRY_TOLERANCE) { u_r = R.hu / R.h; v_r = R.hv / R.h; }
     Face f;
     if (YDIR)
-        riemann_y<HLLC, EXACT>(g, h_hyd_l, h_hyd_l * u_l, h_hyd_l * v_l, h_hyd_r, h_hyd_r * u_r,
+        riemann_y<HLLC>(g, h_hyd_l, h_hyd_l * u_l, h_hyd_l * v_l, h_hyd_r, h_hyd_r * u_r,
                         h_hyd_r * v_r, f.fh, f.fhu, f.fhv);
     else
-        riemann_x<HLLC, EXACT>(g, h_hyd_l, h_hyd_l * u_l, h_hyd_l * v_l, h_hyd_r, h_hyd_r * u_r,
+        riemann_x<HLLC>(g, h_hyd_l, h_hyd_l * u_l, h_hyd_l * v_l, h_hyd_r, h_hyd_r * u_r,
                         h_hyd_r * v_r, f.fh, f.fhu, f.fhv);
     f.a = h_hyd_r * h_hyd_r - R.h * R.h;
     f.c = h_hyd_l * h_hyd_l;
@@ -282,145 +311,186 @@ __device__ __forceinline__ Face face_flux(double g, const FState& L, double bL, 
 }
 
 // ---------------------------------------------------------------------
-// The fast path.  Away from wet/dry fronts and shocks a wavefront's faces
-// and cells satisfy the assumptions below; each *_fast function performs
-// exactly the IEEE operations of its general counterpart for the branch
-// those assumptions select, and raises `bad` on a lane where one fails.
-// The callers test the assumptions they can before the work (wave-uniform
-// branches) and redo a piece on the general path when any lane that
-// matters raised `bad`, so results never depend on the path taken.  The
-// assumptions and what they remove:
-//  * every face state and hydrostatic depth exceeds DRY_TOLERANCE: the
-//    velocity quotients need no dry branch, the wave-speed arguments g h
-//    lie above 2^-767 and are finite (the row's inputs are bounded by
-//    unbounded()), so sqrt_pos gives sqrt's bits, and the speeds are Davis's;
-//  * s_l < 0 < s_r (the HLL star region) with s_r - s_l in [1e-8, 1e12]:
-//    1/(s_r - s_l) is the shared-reciprocal quotient of 1.0, the same bits
-//    as the division;
-//  * HLLC: |denom_star| > DRY_TOLERANCE and num = 0 or |num| >= 2^-900.
-//    Only the sign of s_star = num / denom_star is used; |denom_star| stays
-//    below 2^83 (depths below 2^41 for inputs bounded by unbounded(), and
-//    |u - s| <= 2 (s_r - s_l) <= 2e12), so the quotient does not underflow
-//    to zero and
-//    s_star >= 0 exactly when num is zero or num and denom_star have the
-//    same sign: no division;
-//  * updated cells: h >= DRY_TOLERANCE with h^4 >= DESING_EPS^4 (no clamp,
-//    no KP07) and speed^2 below the Froude backstop by a margin checked
-//    without the division; friction's x^(1/3) below 1e12 and its
-//    numerator g n^2 at least 2^-969, so its quotient is a shared-reciprocal
-//    one.
+// The row path.  Every row whose stencil passes unbounded() is evaluated by
+// the functions below (states_row, face_row, stage_body_row, ...); the
+// functions above, with plain divisions, take the others.  Both perform the
+// same rounded operations on every value that is used, so the bits do not
+// depend on the path.  The row path is written for a wavefront that is
+// bound by instruction issue (about 0.65 of the issue slots, three waves per
+// SIMD): branches are selects, and selects are few:
+//  * max(x, 0), max(a, b) and minmod are v_max_f64 / v_min_f64 (one
+//    instruction instead of a compare and two selects).  They differ from
+//    the compare-and-select forms only in the sign of a zero;
+//  * minmod(a, b) = max(min(a, b), 0) + min(max(a, b), 0): one of the two
+//    terms is the limited slope and the other is zero.  The reference zeroes
+//    the slope where a b <= 0; a and b are differences of values that are 0
+//    or at least 2^-300, hence 0 or at least 2^-352, and a b does not
+//    underflow;
+//  * c -+ 0.5 s is one fma: 0.5 s is exact.  Where the slopes are zeroed the
+//    factor 0.5 becomes 0, one select for the three slopes;
+//  * a dry side's velocities are zeroed through its reciprocal (n * 0), one
+//    select for both quotients.  A wavefront whose faces are wet takes a copy
+//    of the face without these selects;
+//  * square roots of g h take sqrt_pos: with h 0 or at least 2^-353 (a
+//    difference of bounded values) the argument is 0, where the result is
+//    selected, or above 2^-767;
+//  * 1 / (s_r - s_l) is a shared-reciprocal quotient: in the star region the
+//    span is at least 2^-180 and at most 2^45, far from the exponents where
+//    the division would scale;
+//  * HLLC needs only the sign of s_star.  In the star region u_r - s_r <= 0
+//    and u_l - s_l >= 0 (Davis or Ritter speeds), so denom_star <= 0 and
+//    s_star >= 0 where num <= 0.  With denom_star < -DRY_TOLERANCE a non-zero
+//    num is a rounded difference of terms whose larger one is at least 2^-89
+//    (|s| >= 2^-68 where a side has h > DRY_TOLERANCE and g >= 1e-3, depth
+//    times relative speed at least 2^-21), so |num| >= 2^-142; and
+//    |denom_star| is below 2^83: the quotient does not underflow.
 
-// riemann_x restricted to the HLL star region, rki_kernel_flux.F90:410-495
-// and 584-684 (Davis speeds, :463-466).
-template <bool HLLC>
-__device__ __forceinline__ void riemann_x_fast(double g, double h_l, double hu_l, double hv_l, double h_r,
-                                               double hu_r, double hv_r, double& f_h, double& f_hu,
-                                               double& f_hv, bool& bad) {
-    const Recip rl = recip(h_l), rr = recip(h_r);
-    const double u_l = rdiv<false>(hu_l, rl), v_l = rdiv<false>(hv_l, rl);
-    const double u_r = rdiv<false>(hu_r, rr), v_r = rdiv<false>(hv_r, rr);
-    const double a_l = sqrt_pos(g * h_l);
-    const double a_r = sqrt_pos(g * h_r);
-    const double s_l = dmin(u_l - a_l, u_r - a_r);
-    const double s_r = dmax(u_l + a_l, u_r + a_r);
-    const double fl_h = hu_l, fl_hu = hu_l * u_l + 0.5 * g * h_l * h_l, fl_hv = hu_l * v_l;
-    const double fr_h = hu_r, fr_hu = hu_r * u_r + 0.5 * g * h_r * h_r, fr_hv = hu_r * v_r;
-    const double span = s_r - s_l;
-    bad = bad || !(s_l < 0.0 && s_r > 0.0 && span >= 1.0e-8 && span <= 1.0e12);
-    const double denom = rdiv<false>(1.0, recip(span));
-    f_h = (s_r * fl_h - s_l * fr_h + s_l * s_r * (h_r - h_l)) * denom;
-    f_hu = (s_r * fl_hu - s_l * fr_hu + s_l * s_r * (hu_r - hu_l)) * denom;
-    if (!HLLC) {
-        f_hv = (s_r * fl_hv - s_l * fr_hv + s_l * s_r * (hv_r - hv_l)) * denom;
-    } else {
-        const double denom_star = h_r * (u_r - s_r) - h_l * (u_l - s_l);
-        const double num = s_l * h_r * (u_r - s_r) - s_r * h_l * (u_l - s_l);
-        bad = bad || !(fabs(denom_star) > DRY_TOLERANCE && (num == 0.0 || fabs(num) >= 0x1p-900));
-        const bool star_nonneg = num == 0.0 || ((num > 0.0) == (denom_star > 0.0));
-        f_hv = star_nonneg ? f_h * v_l : f_h * v_r;
-    }
+__device__ __forceinline__ double vmax(double a, double b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ double vmin(double a, double b) { return __builtin_fmin(a, b); }
+__device__ __forceinline__ double minmod_row(double a, double b) {
+    return vmax(vmin(a, b), 0.0) + vmin(vmax(a, b), 0.0);
 }
 
-// riemann_y restricted to the HLL star region, rki_kernel_flux.F90:497-582
-// and 686-783.
-template <bool HLLC>
-__device__ __forceinline__ void riemann_y_fast(double g, double h_b, double hu_b, double hv_b, double h_t,
-                                               double hu_t, double hv_t, double& g_h, double& g_hu,
-                                               double& g_hv, bool& bad) {
-    const Recip rb = recip(h_b), rt = recip(h_t);
-    const double u_b = rdiv<false>(hu_b, rb), v_b = rdiv<false>(hv_b, rb);
-    const double u_t = rdiv<false>(hu_t, rt), v_t = rdiv<false>(hv_t, rt);
-    const double a_b = sqrt_pos(g * h_b);
-    const double a_t = sqrt_pos(g * h_t);
-    const double s_l = dmin(v_b - a_b, v_t - a_t);
-    const double s_r = dmax(v_b + a_b, v_t + a_t);
-    const double gl_h = hv_b, gl_hu = hu_b * v_b, gl_hv = hv_b * v_b + 0.5 * g * h_b * h_b;
-    const double gr_h = hv_t, gr_hu = hu_t * v_t, gr_hv = hv_t * v_t + 0.5 * g * h_t * h_t;
-    const double span = s_r - s_l;
-    bad = bad || !(s_l < 0.0 && s_r > 0.0 && span >= 1.0e-8 && span <= 1.0e12);
-    const double denom = rdiv<false>(1.0, recip(span));
-    g_h = (s_r * gl_h - s_l * gr_h + s_l * s_r * (h_t - h_b)) * denom;
-    g_hv = (s_r * gl_hv - s_l * gr_hv + s_l * s_r * (hv_t - hv_b)) * denom;
-    if (!HLLC) {
-        g_hu = (s_r * gl_hu - s_l * gr_hu + s_l * s_r * (hu_t - hu_b)) * denom;
-    } else {
-        const double denom_star = h_t * (v_t - s_r) - h_b * (v_b - s_l);
-        const double num = s_l * h_t * (v_t - s_r) - s_r * h_b * (v_b - s_l);
-        bad = bad || !(fabs(denom_star) > DRY_TOLERANCE && (num == 0.0 || fabs(num) >= 0x1p-900));
-        const bool star_nonneg = num == 0.0 || ((num > 0.0) == (denom_star > 0.0));
-        g_hu = star_nonneg ? g_h * u_b : g_h * u_t;
-    }
+// cell_states from the surface and momenta (e, hu, hv) of the three cells and
+// the bed of the middle one; `flat` where the slopes are zeroed.
+struct Surf {
+    double e, hu, hv;
+};
+__device__ __forceinline__ Surf operator-(const Surf& a, const Surf& b) {
+    return Surf{a.e - b.e, a.hu - b.hu, a.hv - b.hv};
+}
+__device__ __forceinline__ void states_row(const Surf& dm, const Surf& dp, const Surf& c, double b, bool flat,
+                                           FState& lo, FState& hi) {
+    const double w = flat ? 0.0 : 0.5;
+    const double s_eta = minmod_row(dm.e, dp.e);
+    const double s_hu = minmod_row(dm.hu, dp.hu);
+    const double s_hv = minmod_row(dm.hv, dp.hv);
+    lo.h = vmax(fma(-w, s_eta, c.e) - b, 0.0);
+    lo.hu = fma(-w, s_hu, c.hu);
+    lo.hv = fma(-w, s_hv, c.hv);
+    hi.h = vmax(fma(w, s_eta, c.e) - b, 0.0);
+    hi.hu = fma(w, s_hu, c.hu);
+    hi.hv = fma(w, s_hv, c.hv);
 }
 
-// face_flux<HLLC, YDIR, false> on the fast path where the wavefront allows
-// it: when every lane that matters (`use`) has both face states and both
-// hydrostatic depths wet, the velocities need no dry branch and the Riemann
-// solver is riemann_*_fast; lanes outside its star region then take the
-// general solver on the same arguments.  Otherwise face_flux.
-template <bool HLLC, bool YDIR>
-__device__ __forceinline__ Face face_flux_auto(double g, const FState& L, double bL, const FState& R, double bR,
-                                               bool use) {
-    const double b_max = dmax(bL, bR);
-    const double h_hyd_l = fmax0(L.h + bL - b_max);
-    const double h_hyd_r = fmax0(R.h + bR - b_max);
-    const bool wet = L.h > DRY_TOLERANCE && R.h > DRY_TOLERANCE && h_hyd_l > DRY_TOLERANCE &&
-                     h_hyd_r > DRY_TOLERANCE;
-    if (__any(use && !wet)) return face_flux<HLLC, YDIR, false>(g, L, bL, R, bR);
-    const Recip rl = recip(L.h), rr = recip(R.h);
-    const double u_l = rdiv<false>(L.hu, rl), v_l = rdiv<false>(L.hv, rl);
-    const double u_r = rdiv<false>(R.hu, rr), v_r = rdiv<false>(R.hv, rr);
-    const double qu_l = h_hyd_l * u_l, qv_l = h_hyd_l * v_l, qu_r = h_hyd_r * u_r, qv_r = h_hyd_r * v_r;
+// face_flux of the row path.  DRY: some lane that matters has a dry side
+// (or hydrostatic depth); without it all four depths are wet.
+template <bool HLLC, bool YDIR, bool DRY>
+__device__ __forceinline__ Face face_row_as(double g, const FState& L, const FState& R, double h_l, double h_r,
+                                            bool use) {
+    Recip rL = recip(L.h), rR = recip(R.h), rl = recip(h_l), rr = recip(h_r);
+    const bool dry_l = h_l <= DRY_TOLERANCE, dry_r = h_r <= DRY_TOLERANCE;
+    if (DRY) {
+        rL.y = L.h > DRY_TOLERANCE ? rL.y : 0.0;
+        rR.y = R.h > DRY_TOLERANCE ? rR.y : 0.0;
+        rl.y = dry_l ? 0.0 : rl.y;
+        rr.y = dry_r ? 0.0 : rr.y;
+    }
+    const double q0_l = h_l * rdiv<false>(L.hu, rL), q1_l = h_l * rdiv<false>(L.hv, rL);
+    const double q0_r = h_r * rdiv<false>(R.hu, rR), q1_r = h_r * rdiv<false>(R.hv, rR);
+    // normal and tangential momentum of the hydrostatic states
+    const double n_l = YDIR ? q1_l : q0_l, t_l = YDIR ? q0_l : q1_l;
+    const double n_r = YDIR ? q1_r : q0_r, t_r = YDIR ? q0_r : q1_r;
+    const double u_l = rdiv<false>(n_l, rl), v_l = rdiv<false>(t_l, rl);
+    const double u_r = rdiv<false>(n_r, rr), v_r = rdiv<false>(t_r, rr);
+    double a_l = sqrt_pos(g * h_l), a_r = sqrt_pos(g * h_r);
+    if (DRY) {
+        a_l = h_l > 0.0 ? a_l : 0.0;
+        a_r = h_r > 0.0 ? a_r : 0.0;
+    }
+    double s_l = vmin(u_l - a_l, u_r - a_r);
+    double s_r = vmax(u_l + a_l, u_r + a_r);
+    if (DRY) {   // Ritter fronts
+        s_l = dry_r ? u_l - a_l : (dry_l ? fma(-2.0, a_r, u_r) : s_l);
+        s_r = dry_r ? fma(2.0, a_l, u_l) : (dry_l ? u_r + a_r : s_r);
+    }
+    const double half_g = 0.5 * g;
+    // x faces: fl_hv = hu_l v_l; y faces: gl_hu = hu_b v_b (the operand order of the reference)
+    const double fl_n = n_l * u_l + half_g * h_l * h_l, fr_n = n_r * u_r + half_g * h_r * h_r;
+    const double denom = rdiv<false>(1.0, recip(s_r - s_l));
+    const double ss = s_l * s_r;
     Face f;
-    bool bad = false;
-    if (YDIR) riemann_y_fast<HLLC>(g, h_hyd_l, qu_l, qv_l, h_hyd_r, qu_r, qv_r, f.fh, f.fhu, f.fhv, bad);
-    else riemann_x_fast<HLLC>(g, h_hyd_l, qu_l, qv_l, h_hyd_r, qu_r, qv_r, f.fh, f.fhu, f.fhv, bad);
-    if (__any(use && bad)) {
-        if (YDIR) riemann_y<HLLC, false>(g, h_hyd_l, qu_l, qv_l, h_hyd_r, qu_r, qv_r, f.fh, f.fhu, f.fhv);
-        else riemann_x<HLLC, false>(g, h_hyd_l, qu_l, qv_l, h_hyd_r, qu_r, qv_r, f.fh, f.fhu, f.fhv);
+    double fn, ft;
+    f.fh = (s_r * n_l - s_l * n_r + ss * (h_r - h_l)) * denom;
+    fn = (s_r * fl_n - s_l * fr_n + ss * (n_r - n_l)) * denom;
+    double fl_t = 0.0, fr_t = 0.0;
+    if (!HLLC) {
+        fl_t = YDIR ? t_l * u_l : n_l * v_l;
+        fr_t = YDIR ? t_r * u_r : n_r * v_r;
+        ft = (s_r * fl_t - s_l * fr_t + ss * (t_r - t_l)) * denom;
+    } else {
+        const double w_r = u_r - s_r, w_l = u_l - s_l;
+        const double denom_star = h_r * w_r - h_l * w_l;
+        const double num = s_l * h_r * w_r - s_r * h_l * w_l;
+        const bool big = denom_star < -DRY_TOLERANCE;
+        const bool left = (big & (num <= 0.0)) | (!big & (u_l + u_r >= 0.0));
+        ft = f.fh * (left ? v_l : v_r);
     }
-    f.a = h_hyd_r * h_hyd_r - R.h * R.h;
-    f.c = h_hyd_l * h_hyd_l;
+    // outside the star region the flux is that of the upwind state
+    if (DRY || __builtin_expect(__any(use & !((s_l < 0.0) & (s_r > 0.0))), 0)) {
+        if (HLLC) {
+            fl_t = YDIR ? t_l * u_l : n_l * v_l;
+            fr_t = YDIR ? t_r * u_r : n_r * v_r;
+        }
+        const bool left = s_l >= 0.0, right = s_r <= 0.0;
+        f.fh = left ? n_l : (right ? n_r : f.fh);
+        fn = left ? fl_n : (right ? fr_n : fn);
+        ft = left ? fl_t : (right ? fr_t : ft);
+    }
+    f.fhu = YDIR ? ft : fn;
+    f.fhv = YDIR ? fn : ft;
+    f.a = h_r * h_r - R.h * R.h;
+    f.c = h_l * h_l;
     f.d = L.h * L.h;
     return f;
 }
 
+// face_flux of the row path; `use`: the lanes whose face is used.
+template <bool HLLC, bool YDIR>
+__device__ __forceinline__ Face face_row(double g, const FState& L, double bL, const FState& R, double bR, bool use) {
+    const double b_max = vmax(bL, bR);
+    const double h_l = vmax(L.h + bL - b_max, 0.0);
+    const double h_r = vmax(R.h + bR - b_max, 0.0);
+    const double low = vmin(vmin(L.h, R.h), vmin(h_l, h_r));
+    if (__builtin_expect(__any(use & !(low > DRY_TOLERANCE)), 0)) return face_row_as<HLLC, YDIR, true>(g, L, R, h_l, h_r, use);
+    return face_row_as<HLLC, YDIR, false>(g, L, R, h_l, h_r, use);
+}
+
 // Net flux divergence of one cell from its four faces,
-// rki_kernel_flux.F90:358-369 (rdx, rdy: reciprocals of dx, dy).
-template <bool EXACT>
-__device__ __forceinline__ void divergence(double g, const Recip& rdx, const Recip& rdy,
-                                           const Face& xl, const Face& xr, const Face& yb,
-                                           const Face& yt, double& fh, double& fhu, double& fhv) {
+// rki_kernel_flux.F90:358-369 (rdx, rdy: reciprocals of dx, dy): the terms of
+// the y faces, then the sum.
+struct YPart {
+    double fh, fhu, fhv, press;
+};
+
+enum : int { DIV_PLAIN, DIV_SHARED, DIV_TWO_OP };   // how a quotient by the spacing is taken
+
+template <int MODE>
+__device__ __forceinline__ double over(double n, const Spacing& s) {
+    return MODE == DIV_PLAIN ? n / s.r.d : sdiv<MODE == DIV_TWO_OP>(n, s);
+}
+
+template <int MODE>
+__device__ __forceinline__ YPart divergence_y(double g, const Spacing& dy, const Face& yb, const Face& yt) {
+    YPart y;
+    y.fh = over<MODE>(yt.fh - yb.fh, dy);
+    y.fhu = over<MODE>(yt.fhu - yb.fhu, dy);
+    y.fhv = over<MODE>(yt.fhv - yb.fhv, dy);
+    y.press = over<MODE>(0.5 * g * (yb.a - yt.c + yt.d), dy);
+    return y;
+}
+
+template <int MODE>
+__device__ __forceinline__ void divergence(double g, const Spacing& dx, const Face& xl, const Face& xr, const YPart& y,
+                                           double& fh, double& fhu, double& fhv) {
     const double half_g = 0.5 * g;
-    fh = rdiv<EXACT>(-(xr.fh - xl.fh), rdx) - rdiv<EXACT>(yt.fh - yb.fh, rdy);
-    fhu = rdiv<EXACT>(-(xr.fhu - xl.fhu), rdx) - rdiv<EXACT>(yt.fhu - yb.fhu, rdy) -
-          rdiv<EXACT>(half_g * (xl.a - xr.c + xr.d), rdx);
-    fhv = rdiv<EXACT>(-(xr.fhv - xl.fhv), rdx) - rdiv<EXACT>(yt.fhv - yb.fhv, rdy) -
-          rdiv<EXACT>(half_g * (yb.a - yt.c + yt.d), rdy);
+    fh = over<MODE>(-(xr.fh - xl.fh), dx) - y.fh;
+    fhu = over<MODE>(-(xr.fhu - xl.fhu), dx) - y.fhu - over<MODE>(half_g * (xl.a - xr.c + xr.d), dx);
+    fhv = over<MODE>(-(xr.fhv - xl.fhv), dx) - y.fhv - y.press;
 }
 
 // Clamp + KP07 desingularization + Froude backstop,
 // rki_kernel_fused.F90:234-260 and :440-463.
-template <bool EXACT>
 __device__ __forceinline__ void clamp_desing(double g, double& h, double& hu, double& hv) {
     const double eps4 = 5.062499999999998e-16;  // DESING_EPS**4 folded (0x3CC23D5504170727)
     if (h < 0.0) {
@@ -430,9 +500,9 @@ __device__ __forceinline__ void clamp_desing(double g, double& h, double& hu, do
     } else {
         const double h4 = pow4(h);
         if (h4 < eps4) {
-            const Recip r = recip(sqrt(h4 + eps4));
-            const double u = rdiv<EXACT>(SQRT2 * h * hu, r);
-            const double v = rdiv<EXACT>(SQRT2 * h * hv, r);
+            const double r = sqrt(h4 + eps4);
+            const double u = SQRT2 * h * hu / r;
+            const double v = SQRT2 * h * hv / r;
             hu = h * u;
             hv = h * v;
         }
@@ -465,26 +535,25 @@ struct Frc {
 // rki_kernel_fused.F90:228-290.  With NF the Manning coefficient is the
 // cell's own n_cell (friction where n_cell > 0) instead of the scalar one;
 // FRC applies the surface forcing f (forcing_active).
-template <bool EXACT, bool NF, bool FRC = false>
+template <bool NF, bool FRC = false>
 __device__ __forceinline__ void stage_body(const SourceTerms& s, double dt, double fh, double fhu,
                                            double fhv, double& h, double& hu, double& hv, double n_cell,
                                            const Frc& f = Frc{}) {
     h = h + dt * fh;
     hu = hu + dt * fhu;
     hv = hv + dt * fhv;
-    clamp_desing<EXACT>(s.g, h, hu, hv);
+    clamp_desing(s.g, h, hu, hv);
     const bool friction = NF ? (n_cell > 0.0) : (s.has_friction != 0);
     const double n_sq = NF ? n_cell * n_cell : s.n_sq;
     if (h > DRY_TOLERANCE) {
         if (friction) {
-            const Recip rh = recip(h);
-            const double u = rdiv<EXACT>(hu, rh);
-            const double v = rdiv<EXACT>(hv, rh);
+            const double u = hu / h;
+            const double v = hv / h;
             const double speed = sqrt(u * u + v * v);
             const double cf = s.g * n_sq / crm::pow13(h);
-            const Recip rd = recip(1.0 + rdiv<EXACT>(dt * cf * speed, rh));
-            hu = rdiv<EXACT>(hu, rd);
-            hv = rdiv<EXACT>(hv, rd);
+            const double denom = 1.0 + dt * cf * speed / h;
+            hu = hu / denom;
+            hv = hv / denom;
         }
         if (FRC) {   // rki_kernel_fused.F90:273-280
             hu = hu + dt * f.wx / RHO_WATER;
@@ -501,90 +570,133 @@ __device__ __forceinline__ void stage_body(const SourceTerms& s, double dt, doub
     if (FRC) h = h + dt * f.rain;   // every cell, :286-289
 }
 
-// clamp_desing of the fast row path: the cell is wet (h >= DRY_TOLERANCE),
-// outside the KP07 band (h^4 >= DESING_EPS^4) and below the Froude
-// backstop, so the values pass unchanged.  The backstop test
-// (hu^2 + hv^2) / h^2 > fr_max_sq is decided without the quotient:
-// num < h^2 (fr_max_sq (1 - 2^-50)), rounded, implies num / h^2 < fr_max_sq
-// exactly, hence the rounded quotient is at most fr_max_sq (a double).
-__device__ __forceinline__ void clamp_fast(double g, double h, double hu, double hv, bool& bad) {
-    const double eps4 = 5.062499999999998e-16;
-    const double h4 = pow4(h);
+// clamp_desing of the row path: dry cells by selects, and clamp_desing itself
+// where a lane is in the KP07 band or near the Froude backstop.  The band,
+// ((h h) h) h < DESING_EPS^4, is h < KP07_DEPTH: the product is monotone in h,
+// also rounded.  The backstop test (hu^2 + hv^2) / h^2 > fr_max_sq is decided
+// without the quotient: num < h^2 (fr_max_sq (1 - 2^-50)), rounded, implies
+// num / h^2 < fr_max_sq exactly, hence the rounded quotient is at most
+// fr_max_sq (a double).  Returns true where the cell update has to be redone
+// with plain divisions: a lane's values are huge or not finite, or a depth is
+// the dry tolerance itself.
+constexpr double KP07_DEPTH = 0x1.3a92a30553261p-13;   // the smallest h with h^4, rounded, >= DESING_EPS^4
+
+__device__ __forceinline__ bool clamp_row(double g, double& h, double& hu, double& hv) {
     const double num = hu * hu + hv * hv;
     const double fr_max_sq = (FROUDE_BACKSTOP * FROUDE_BACKSTOP * g) * h;
     const double lim = (h * h) * (fr_max_sq * (1.0 - 0x1p-50));
-    bad = bad || !(h >= DRY_TOLERANCE && h4 >= eps4 && num < lim);
+    const bool dry = h < DRY_TOLERANCE;
+    if (__builtin_expect(__any(!(dry | ((h >= KP07_DEPTH) & (num < lim) & (h < 0x1p100)))), 0)) {
+        if (__any(!((h < 0x1p100) & (num < 0x1p200)) | (h == DRY_TOLERANCE))) return true;
+        clamp_desing(g, h, hu, hv);
+        return false;
+    }
+    h = vmax(h, 0.0);
+    hu = dry ? 0.0 : hu;
+    hv = dry ? 0.0 : hv;
+    return false;
 }
 
-// stage_body of the fast row path (clamp_fast above; friction's quotient
-// by x^(1/3) as a shared-reciprocal one while x^(1/3) <= 1e12 and
-// g n^2 >= 2^-969).
+// stage_body of the row path; returns true as clamp_row does.  A cell below
+// the dry tolerance has zero momenta and passes through friction and
+// Coriolis unchanged, the depth being raised to the tolerance for the
+// quotients.  The speed only enters 1 + dt cf speed / h, so raising u^2 + v^2
+// to 2^-700 leaves that sum as it is.  Friction's quotient by x^(1/3) (below
+// 2^34) is a shared-reciprocal one: with a scalar n the caller takes the row
+// path while g n^2 >= 2^-600, with a per-cell n this function asks for the
+// same.
 template <bool NF, bool FRC = false>
-__device__ __forceinline__ void stage_body_fast(const SourceTerms& s, double dt, double fh, double fhu, double fhv,
-                                                double& h, double& hu, double& hv, double n_cell, const Frc& f,
-                                                bool& bad) {
+__device__ __forceinline__ bool stage_body_row(const SourceTerms& s, double dt, double fh, double fhu, double fhv,
+                                               double& h, double& hu, double& hv, double n_cell, const Frc& f) {
     h = h + dt * fh;
     hu = hu + dt * fhu;
     hv = hv + dt * fhv;
-    clamp_fast(s.g, h, hu, hv, bad);
-    const bool friction = NF ? (n_cell > 0.0) : (s.has_friction != 0);
-    const double n_sq = NF ? n_cell * n_cell : s.n_sq;
-    if (friction) {
-        const Recip rh = recip(h);
+    if (clamp_row(s.g, h, hu, hv)) return true;
+    if (NF || s.has_friction) {
+        const double hs = vmax(h, DRY_TOLERANCE);
+        const Recip rh = recip(hs);
         const double u = rdiv<false>(hu, rh);
         const double v = rdiv<false>(hv, rh);
-        const double speed = sqrt(u * u + v * v);
-        const double p13 = crm::pow13(h);
-        const double gn2 = s.g * n_sq;
-        bad = bad || !(p13 <= 1.0e12 && gn2 >= 0x1p-969);
-        const double cf = rdiv<false>(gn2, recip(p13));
+        const double speed = sqrt_pos(vmax(u * u + v * v, 0x1p-700));
+        double gn2 = s.g * (NF ? n_cell * n_cell : s.n_sq);
+        if (NF) {
+            const bool friction = n_cell > 0.0;
+            if (__any(friction & !(gn2 >= 0x1p-600))) return true;
+            gn2 = friction ? gn2 : 0.0;
+        }
+        const double cf = rdiv<false>(gn2, recip(crm::pow13(hs)));
         const Recip rd = recip(1.0 + rdiv<false>(dt * cf * speed, rh));
         hu = rdiv<false>(hu, rd);
         hv = rdiv<false>(hv, rd);
     }
     if (FRC) {
-        hu = hu + dt * f.wx / RHO_WATER;
-        hv = hv + dt * f.wy / RHO_WATER;
-        hu = hu - dt * h * f.dpdx / RHO_WATER;
-        hv = hv - dt * h * f.dpdy / RHO_WATER;
+        const bool wet = h > DRY_TOLERANCE;
+        double qu = hu + dt * f.wx / RHO_WATER;
+        double qv = hv + dt * f.wy / RHO_WATER;
+        qu = qu - dt * h * f.dpdx / RHO_WATER;
+        qv = qv - dt * h * f.dpdy / RHO_WATER;
+        hu = wet ? qu : hu;
+        hv = wet ? qv : hv;
     }
     if (s.has_coriolis) {
         const double hu_old = hu, hv_old = hv;
         hu = hu_old * s.cosf + hv_old * s.sinf;
         hv = -hu_old * s.sinf + hv_old * s.cosf;
     }
-    if (FRC) h = h + dt * f.rain;
+    if (FRC) {
+        h = h + dt * f.rain;
+        if (__any(!((h < 0x1p100) & (fabs(hu) + fabs(hv) < 0x1p100)))) return true;
+    }
+    return false;
 }
 
-// cfl_speed for a cell that passed clamp_fast (h > DRY_TOLERANCE; g h and
-// h^4 + eps^4 are positive and finite, so sqrt_pos gives sqrt's bits).
-__device__ __forceinline__ double cfl_speed_fast(double g, const Recip& rdx, const Recip& rdy, double h, double hu,
-                                                 double hv) {
+// Largest |u| + a and |v| + a over the wet cells a lane has seen
+// (rki_kernel_timestep.F90:56-69 before the division by dx and dy).
+// Rounded division is monotone, so the largest of the per-cell speeds is
+// the larger of the two maxima divided by dx and dy (cfl_max).
+struct CflMax {
+    double u, v;
+};
+
+// `same`: dx = dy, where one maximum of max(|u|, |v|) + a does.
+__device__ __forceinline__ void cfl_row(double g, bool same, double h, double hu, double hv, CflMax& m) {
     const double eps4 = 5.062499999999998e-16;
-    const double wave_speed = sqrt_pos(g * h);
-    const double h4 = pow4(h);
+    const double hs = vmax(h, DRY_TOLERANCE);
+    const double wave_speed = sqrt_pos(g * hs);
+    const double h4 = pow4(hs);
     const Recip rd = recip(sqrt_pos(h4 + eps4));
-    const double u_abs = rdiv<false>(fabs(hu) * SQRT2 * h, rd);
-    const double v_abs = rdiv<false>(fabs(hv) * SQRT2 * h, rd);
-    const double sx = rdiv<false>(u_abs + wave_speed, rdx);
-    const double sy = rdiv<false>(v_abs + wave_speed, rdy);
-    return dmax(sx, sy);
+    const bool wet = h > DRY_TOLERANCE;
+    if (same) {
+        const double u_abs = rdiv<false>(vmax(fabs(hu), fabs(hv)) * SQRT2 * hs, rd);
+        m.u = vmax(m.u, wet ? u_abs + wave_speed : 0.0);
+    } else {
+        const double u_abs = rdiv<false>(fabs(hu) * SQRT2 * hs, rd);
+        const double v_abs = rdiv<false>(fabs(hv) * SQRT2 * hs, rd);
+        m.u = vmax(m.u, wet ? u_abs + wave_speed : 0.0);
+        m.v = vmax(m.v, wet ? v_abs + wave_speed : 0.0);
+    }
+}
+
+// The same with plain divisions.
+__device__ __forceinline__ void cfl_plain(double g, double h, double hu, double hv, CflMax& m) {
+    const double eps4 = 5.062499999999998e-16;
+    if (!(h > DRY_TOLERANCE)) return;
+    const double wave_speed = sqrt(g * h);
+    const double S = sqrt(pow4(h) + eps4);
+    m.u = dmax(m.u, fabs(hu) * SQRT2 * h / S + wave_speed);
+    m.v = dmax(m.v, fabs(hv) * SQRT2 * h / S + wave_speed);
+}
+
+__device__ __forceinline__ double cfl_max(const CflMax& m, bool same, double dx, double dy) {
+    if (same) return dmax(m.u, m.v) / dx;
+    return dmax(m.u / dx, m.v / dy);
 }
 
 // Per-cell CFL speed term, rki_kernel_timestep.F90:56-69; 0 for dry cells.
-template <bool EXACT>
-__device__ __forceinline__ double cfl_speed(double g, const Recip& rdx, const Recip& rdy, double h,
-                                            double hu, double hv) {
-    const double eps4 = 5.062499999999998e-16;
-    if (!(h > DRY_TOLERANCE)) return 0.0;
-    const double wave_speed = sqrt(g * h);
-    const double h4 = pow4(h);
-    const Recip rd = recip(sqrt(h4 + eps4));
-    const double u_abs = rdiv<EXACT>(fabs(hu) * SQRT2 * h, rd);
-    const double v_abs = rdiv<EXACT>(fabs(hv) * SQRT2 * h, rd);
-    const double sx = rdiv<EXACT>(u_abs + wave_speed, rdx);
-    const double sy = rdiv<EXACT>(v_abs + wave_speed, rdy);
-    return dmax(sx, sy);
+__device__ __forceinline__ double cfl_speed(double g, double dx, double dy, double h, double hu, double hv) {
+    CflMax m{0.0, 0.0};
+    cfl_plain(g, h, hu, hv, m);
+    return cfl_max(m, false, dx, dy);
 }
 
 }  // namespace rk

@@ -17,12 +17,6 @@ namespace rk {
 
 constexpr int WAVE = 64;        // wavefront width on CDNA
 constexpr int MAX_TC = 10;      // MAX_TIDAL_CONSTITUENTS
-// Tiles a stage launch needs before the fast path (swe_core.hpp) pays: its
-// wave-uniform tests and fallbacks cost latency, which a launch of a few
-// waves per SIMD cannot hide (at 2048 tiles, 1024^2 cells, the stage
-// kernels are 5 % slower with it; at 16384, 4096^2, 5 % faster).
-constexpr long long FAST_MIN_TILES = 6144;
-
 // Time-control slot.  Two slots ping-pong: a step reads slot p (state at
 // the start of the step) and its stage-1 kernel writes slot 1-p.
 struct alignas(64) CtrlSlot {
@@ -46,6 +40,7 @@ struct GridDesc {
     int nx, ny;
     long long pitch;              // elements per row
     double dx, dy;
+    Spacing sdx, sdy;             // dx and dy as divisors
     double* ah; double* ahu; double* ahv;   // A: U^n / U^{n+1}
     double* bh; double* bhu; double* bhv;   // B: U*
     double* sh; double* shu; double* shv;   // optional copy of U^n (RK save), or null
@@ -73,7 +68,7 @@ struct GridDesc {
     double dt_fixed, t_end;
     int cfl_interval;
     int ty;                       // rows per tile segment (<= 64)
-    int fast;                     // the launch may take the fast path (FAST_MIN_TILES)
+    int plain_rows;               // every row with plain divisions (rkg_set_fast_path(-1))
     int nstrips, nsegs;
     CtrlSlot* ctrl;               // [2]
 };
@@ -162,11 +157,9 @@ __host__ __device__ __forceinline__ Cell ghost_from(const GridDesc& d, int tag, 
 // Cell (c, j) of the state (h, hu, hv) with bed d.bed, synthesizing the
 // two ghost layers around the domain.  Corner cells and cells beyond the
 // second ghost layer are never read by the stencil; they return zeros.
-template <bool EDGE>
 __device__ __forceinline__ Cell load_cell(const GridDesc& d, const double* __restrict__ h,
                                           const double* __restrict__ hu, const double* __restrict__ hv,
                                           int c, int j, double eta_tidal) {
-    if (!EDGE) return load_direct(h, hu, hv, d.bed, d.pitch, c, j);
     const bool xin = (unsigned)c < (unsigned)d.nx;
     const bool yin = (unsigned)j < (unsigned)d.ny;
     if (xin && yin) return load_direct(h, hu, hv, d.bed, d.pitch, c, j);
@@ -205,20 +198,8 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 __device__ __forceinline__ double shfl_down1(double v) { return __shfl_down(v, 1, WAVE); }
 __device__ __forceinline__ double shfl_up1(double v) { return __shfl_up(v, 1, WAVE); }
 
-__device__ __forceinline__ Face shfl_down1(const Face& f) {
-    Face r;
-    r.fh = shfl_down1(f.fh); r.fhu = shfl_down1(f.fhu); r.fhv = shfl_down1(f.fhv);
-    r.a = shfl_down1(f.a); r.c = shfl_down1(f.c); r.d = shfl_down1(f.d);
-    return r;
-}
-__device__ __forceinline__ Cell shfl_up1(const Cell& x) {
-    return Cell{shfl_up1(x.h), shfl_up1(x.hu), shfl_up1(x.hv), shfl_up1(x.b)};
-}
-__device__ __forceinline__ Cell shfl_down1(const Cell& x) {
-    return Cell{shfl_down1(x.h), shfl_down1(x.hu), shfl_down1(x.hv), shfl_down1(x.b)};
-}
-__device__ __forceinline__ FState shfl_up1(const FState& x) {
-    return FState{shfl_up1(x.h), shfl_up1(x.hu), shfl_up1(x.hv)};
+__device__ __forceinline__ FState shfl_down1(const FState& x) {
+    return FState{shfl_down1(x.h), shfl_down1(x.hu), shfl_down1(x.hv)};
 }
 
 __device__ __forceinline__ double wave_max(double v) {
@@ -235,14 +216,14 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// Per-segment data of the two edge columns of a strip, one row per entry:
-// raw cells c0-1 and c0+64, the high x-state of c0-1, and the x-face
-// between c0+63 and c0+64.
-struct TileLds {
-    double hl[4][WAVE];
-    double hr[4][WAVE];
-    double ph[3][WAVE];
-    double pf[6][WAVE];
+// Three rows of the march, (h + b, hu, hv, b, h) of the wavefront's 64
+// columns, and what the row below hands up: its high y state (h, hu, hv), the
+// part of its upper face that the row above takes (fh, fhu, fhv, a) and the
+// differences across that face (h + b, hu, hv).  12.5 KB: 12 wavefronts, three
+// a SIMD, on a CU's 160 KB.
+struct TileRing {
+    double v[3][5][WAVE];
+    double up[10][WAVE];
 };
 
 struct StageCtx {
@@ -250,7 +231,6 @@ struct StageCtx {
     double* oh; double* ohu; double* ohv;                     // stage output
     double dt;
     double eta_tidal;
-    Recip rdx, rdy;
     SourceTerms src;
     // Chapman edges (FEAT_CHAPMAN): whether this boundary call radiates
     // (its state differs from the previous call's), the previous call's
@@ -331,16 +311,53 @@ __device__ __forceinline__ Cell chapman_ghost(const GridDesc& d, const StageCtx&
     return g;
 }
 
-template <bool EDGE, int FEAT = 0>
-__device__ __forceinline__ Cell ld(const GridDesc& d, const StageCtx& s, int c, int j) {
-    if constexpr (EDGE && (FEAT & FEAT_CHAPMAN) != 0) {
-        const bool xin = (unsigned)c < (unsigned)d.nx, yin = (unsigned)j < (unsigned)d.ny;
-        if (xin != yin) {
-            const int side = !xin ? (c < 0 ? 0 : 1) : (j < 0 ? 2 : 3);
-            if (d.bc[side] == BC_CHAPMAN) return chapman_ghost(d, s, side, c, j);
-        }
+// Where a tile's lane takes its cells from.  A ghost cell depends on one cell
+// of the grid, the mirror cell at a wall and the first interior cell at every
+// other edge (bc_wall_edge, bc_flather_edge, ..., rki_boundary.F90:281-464),
+// so each lane loads one cell a row whether it is a ghost or not, and the
+// edge's rule is arithmetic on that cell.
+struct LaneSource {
+    int c;      // column to load
+    int side;   // 0 W, 1 E: a ghost column; -1: a column of the grid; -2: beyond the ghosts
+};
+
+__device__ __forceinline__ bool mirrors(int tag) { return tag == BC_WALL || tag == BC_SPONGE; }
+
+template <bool EDGE>
+__device__ __forceinline__ LaneSource lane_source(const GridDesc& d, int c) {
+    if (!EDGE || ((unsigned)c < (unsigned)d.nx)) return LaneSource{c, -1};
+    const bool west = c < 0;
+    const int kk = west ? -c - 1 : c - d.nx;
+    if (kk > 1) return LaneSource{d.nx - 1, -2};
+    const int in = mirrors(d.bc[west ? 0 : 1]) ? kk : 0;
+    return LaneSource{west ? in : d.nx - 1 - in, west ? 0 : 1};
+}
+
+// The cells that row j of the march is made from: those of row j, or of the
+// source row of a ghost row.
+template <bool EDGE>
+__device__ __forceinline__ Cell row_source(const GridDesc& d, const StageCtx& s, const LaneSource& l, int j) {
+    int js = j;
+    if (EDGE) {
+        if (j < 0) js = mirrors(d.bc[2]) ? -j - 1 : 0;
+        else if (j >= d.ny) js = mirrors(d.bc[3]) ? 2 * d.ny - 1 - j : d.ny - 1;
     }
-    return load_cell<EDGE>(d, s.ih, s.ihu, s.ihv, c, j, s.eta_tidal);
+    return load_direct(s.ih, s.ihu, s.ihv, d.bed, d.pitch, l.c, js);
+}
+
+// Row j of the march at the lane's column from its source cell.
+template <bool EDGE, int FEAT>
+__device__ __forceinline__ Cell row_cell(const GridDesc& d, const StageCtx& s, const LaneSource& l, int c, int j,
+                                         const Cell& src) {
+    if (!EDGE) return src;
+    const int rs = j < 0 ? 2 : (j >= d.ny ? 3 : -1);
+    if (rs < 0 && l.side == -1) return src;
+    // corner cells and columns beyond the ghosts are not read by the stencil
+    const int side = rs >= 0 ? (l.side == -1 ? rs : -2) : l.side;
+    if (side < 0) return Cell{0.0, 0.0, 0.0, 0.0};
+    if constexpr ((FEAT & FEAT_CHAPMAN) != 0)
+        if (d.bc[side] == BC_CHAPMAN) return chapman_ghost(d, s, side, c, j);
+    return ghost_from(d, d.bc[side], s.eta_tidal, src, src, (side & 1) ? 1.0 : -1.0, side < 2);
 }
 
 template <bool B>
@@ -348,23 +365,40 @@ struct ExactTag {
     static constexpr bool value = B;
 };
 
-// One 64-column x d.ty-row tile of one RK stage, processed by one
-// wavefront marching down the rows; lane l owns column c = c0 + l.
-// Row j: the y-slope of row j+1 is formed from the raw rows j, j+1, j+2
-// held in registers, giving the face above row j together with the top
-// state of row j carried from the previous row; the x-slope of row j takes
-// the neighbouring columns by wave shuffles, the face left of each cell is
-// evaluated by its lane and the face right of it is the next lane's.  The
-// edge columns come from a per-segment batch (one row per lane) held in
-// LDS.  Every slope and every face of the tile is evaluated once.
-// A row whose stencil holds a non-zero value outside [2^-300, 2^40] in
-// magnitude, or a non-finite one (see tiny()), anywhere in the wavefront is
-// evaluated with plain divisions; every other row with the shared-reciprocal
-// quotients, its faces and cell updates on the fast path of swe_core.hpp
-// where the whole wavefront meets its assumptions.  All give the same bits
-// where they apply.
-// STAGE 1 writes U* to B; STAGE 2 reads U* and U^n, applies the RK2 average
-// and writes U^{n+1} over A, returning the lane's max CFL speed.
+// Columns of a strip that are owned and written: the wavefront's 64 lanes
+// less two halo lanes on each side.
+constexpr int HALO = 2;
+constexpr int OWN = WAVE - 2 * HALO;
+
+// Own range [lo, hi) of block s when [0, n) is cut into blocks of w, the
+// last block holding at least two cells: the halo of the block before it
+// then ends inside the grid, so a ghost cell (which may depend on what the
+// edge's own tile overwrites, see chapman_ghost) is read by the edge's own
+// tile only.  With w = 1 the block before the last one is empty.
+__host__ __device__ __forceinline__ void tile_range(int n, int w, int s, int& lo, int& hi) {
+    const int nb = (n + w - 1) / w;
+    lo = s * w;
+    hi = lo + w < n ? lo + w : n;
+    if (nb >= 2 && n - (nb - 1) * w == 1) {
+        if (s == nb - 1) lo = n - 2;
+        if (s == nb - 2) hi = n - 2;
+    }
+}
+
+// The source cells of rows j0-2 .. j0+1, loaded before the step's clock is
+// read (they do not depend on it): two memory round trips in one.
+struct FirstRows {
+    Cell r[4];
+};
+
+template <bool EDGE>
+__device__ __forceinline__ FirstRows first_rows(const GridDesc& d, const StageCtx& s, const LaneSource& l, int j0) {
+    FirstRows f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) f.r[q] = row_source<EDGE>(d, s, l, j0 - 2 + q);
+    return f;
+}
+
 // apply_sponge (rki_kernel_sponge.F90:16-88) on one interior cell (c, j),
 // 0-based: the distance to the nearest BC_SPONGE edge closer than the
 // width sets alpha = strength ((width - d) / width)^2.  dsum collects the
@@ -389,234 +423,246 @@ __device__ __forceinline__ void sponge_cell(const GridDesc& d, double dt, int c,
     }
 }
 
-template <int STAGE, bool HLLC, bool EDGE, bool NF, bool REC, int FEAT = 0, bool FASTK = false>
-__device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx& s, TileLds& L,
-                                               int strip, int seg, double& fsum, double& ssum) {
+// One tile of one RK stage: a strip of at most 60 owned columns x d.ty rows,
+// processed by one wavefront marching down the rows; lane l holds column
+// x0 - 2 + l, so the two columns each side that the stencil needs are lanes
+// of the same wavefront, and no column is treated apart.
+// Row j: the y-slope of row j+1 is formed from the raw rows j, j+1, j+2
+// held in registers, giving the face above row j together with the top
+// state of row j carried from the previous row; the march starts one row
+// early for the face below the first row.  The x-slope of row j takes the
+// neighbours' differences by wave shuffles, each lane evaluates the face on
+// its right and takes the face on its left from the lane before it.
+//
+// Bound by instruction issue: 60 of 64 lanes own a column (6 % of the work
+// is halo).  The former layout, 64 owned columns with the edge columns
+// batched one row per lane into LDS, spent 18 % of a 16-row tile in its
+// prologue (plain divisions, 4096^2) and read 34 selects a row from LDS.
+//
+// A row whose stencil holds a non-zero value outside [2^-300, 2^40] in
+// magnitude, or a non-finite one (unbounded()), anywhere in the wavefront is
+// evaluated with plain divisions and the branches of the reference; every
+// other row on the row path of swe_core.hpp.  Both give the same bits where
+// both apply.
+// STAGE 1 writes U* to B; STAGE 2 reads U* and U^n, applies the RK2 average
+// and writes U^{n+1} over A, returning the lane's max CFL speed.
+template <int STAGE, bool HLLC, bool EDGE, bool NF, bool REC, int FEAT = 0>
+__device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx& s, TileRing& ring,
+                                               const LaneSource& lsrc, const FirstRows& first, int x0, int x1, int j0,
+                                               int j1, double& fsum, double& ssum) {
     constexpr bool FRC = (FEAT & FEAT_FORCING) != 0;
     constexpr bool SPG = (FEAT & FEAT_SPONGE) != 0;
     const int lane = threadIdx.x;
-    const int c0 = strip * WAVE;
-    const int c = c0 + lane;
-    const int j0 = seg * d.ty;
-    const int j1 = min(j0 + d.ty, d.ny);
-    const int nrows = j1 - j0;
+    const int c = x0 - HALO + lane;
+    const bool own = lane >= HALO && c < x1;
+    const bool use_x = lane >= HALO - 1 && c < x1;   // lanes whose right face is used
     const double g = d.g;
     const long long pitch = d.pitch;
-    // the fast path's ranges assume a gravity of ordinary size
-    const bool try_fast = FASTK && g >= 1.0e-3 && g <= 1.0e6;
-    // the value test of the rows: kernels with the fast path also keep its
-    // range arguments (unbounded()), the others the division's (tiny())
-    auto odd = [](const Cell& x) { return FASTK ? unbounded(x) : tiny(x); };
-    double smax = 0.0;
+    // the row path's ranges assume a gravity and a friction of ordinary size
+    const bool plain = d.plain_rows || !(g >= 1.0e-3 && g <= 1.0e6) ||
+                       (!NF && s.src.has_friction && !(g * s.src.n_sq >= 0x1p-600));
+    CflMax smax{0.0, 0.0};
+    const bool same = d.dx == d.dy;
+    const bool two_op = d.sdx.two_op && d.sdy.two_op;
     double facc = 0.0;  // sum of the lane's flux_h, rows in order
     double sacc = 0.0;  // sum of the lane's sponge change of h
     const bool read_un = STAGE == 2 || (STAGE == 3 && s.blend);
 
-    // (1) edge columns of the segment, one row per lane
-    bool edge_tiny = false;
-    if (lane < nrows) {
-        const int j = j0 + lane;
-        const Cell a = ld<EDGE, FEAT>(d, s, c0 - 2, j);
-        const Cell bl = ld<EDGE, FEAT>(d, s, c0 - 1, j);
-        const Cell cc = ld<EDGE, FEAT>(d, s, c0, j);
-        FState lo, hi;
-        cell_states(a, bl, cc, lo, hi);
-        L.hl[0][lane] = bl.h; L.hl[1][lane] = bl.hu; L.hl[2][lane] = bl.hv; L.hl[3][lane] = bl.b;
-        L.ph[0][lane] = hi.h; L.ph[1][lane] = hi.hu; L.ph[2][lane] = hi.hv;
-        const Cell m1 = ld<EDGE, FEAT>(d, s, c0 + 63, j);
-        const Cell p0 = ld<EDGE, FEAT>(d, s, c0 + 64, j);
-        L.hr[0][lane] = p0.h; L.hr[1][lane] = p0.hu; L.hr[2][lane] = p0.hv; L.hr[3][lane] = p0.b;
-        edge_tiny = odd(a) || odd(bl) || odd(cc) || odd(m1) || odd(p0);
-        if (c0 + WAVE - 1 < d.nx) {
-            const Cell m2 = ld<EDGE, FEAT>(d, s, c0 + 62, j);
-            const Cell p1 = ld<EDGE, FEAT>(d, s, c0 + 65, j);
-            FState lo1, hi1, lo2, hi2;
-            cell_states(m2, m1, p0, lo1, hi1);
-            cell_states(m1, p0, p1, lo2, hi2);
-            const Face f = face_flux<HLLC, false, true>(g, hi1, m1.b, lo2, p0.b);
-            L.pf[0][lane] = f.fh; L.pf[1][lane] = f.fhu; L.pf[2][lane] = f.fhv;
-            L.pf[3][lane] = f.a; L.pf[4][lane] = f.c; L.pf[5][lane] = f.d;
-        }
-    }
-    // rows of the segment whose edge cells hold tiny values
-    const unsigned long long edge_rows = __ballot(edge_tiny);
-
-    // (2) y pipeline: top state of row j0-1, face below row j0
-    Cell rc, rn, rnn;
-    FState tc;
-    Face fyb;
-    bool t_prev, t_rc, t_rn, t_rnn;
+    // the rows j, j+1 and j+2 of the march, in LDS; a lane's neighbours by
+    // their lane, the wavefront's ends repeating themselves (unused)
+    const int lane_m = max(lane - 1, 0), lane_p = min(lane + 1, WAVE - 1);
+    auto surf = [&](int slot, int l) { return Surf{ring.v[slot][0][l], ring.v[slot][1][l], ring.v[slot][2][l]}; };
+    auto cell = [&](int slot, int l) {
+        return Cell{ring.v[slot][4][l], ring.v[slot][1][l], ring.v[slot][2][l], ring.v[slot][3][l]};
+    };
+    auto put = [&](int slot, const Cell& x) {
+        ring.v[slot][0][lane] = x.h + x.b; ring.v[slot][1][lane] = x.hu; ring.v[slot][2][lane] = x.hv;
+        ring.v[slot][3][lane] = x.b; ring.v[slot][4][lane] = x.h;
+    };
+    auto hand_up = [&](const FState& hi, const Face& f, const Surf& dm) {
+        ring.up[0][lane] = hi.h; ring.up[1][lane] = hi.hu; ring.up[2][lane] = hi.hv;
+        ring.up[3][lane] = f.fh; ring.up[4][lane] = f.fhu; ring.up[5][lane] = f.fhv; ring.up[6][lane] = f.a;
+        ring.up[7][lane] = dm.e; ring.up[8][lane] = dm.hu; ring.up[9][lane] = dm.hv;
+    };
+    // per row of the ring, over the wavefront: a value out of the row path's
+    // bounds; the lanes below the dry tolerance; those in a thin layer
+    struct RowBits {
+        bool odd;
+        unsigned long long dry, thin;
+    };
+    auto bits = [&](const Cell& x) {
+        return RowBits{(bool)__any(unbounded(x)), __ballot(x.h < DRY_TOLERANCE), __ballot(x.h < THIN_LAYER_THRESHOLD)};
+    };
+    int sc = 0, sn = 1, snn = 2;
+    bool odd_prev;
+    RowBits bc, bn, bnn;
     {
-        const Cell a = ld<EDGE, FEAT>(d, s, c, j0 - 2);
-        const Cell bm = ld<EDGE, FEAT>(d, s, c, j0 - 1);
-        rc = ld<EDGE, FEAT>(d, s, c, j0);
-        rn = ld<EDGE, FEAT>(d, s, c, j0 + 1);
-        rnn = ld<EDGE, FEAT>(d, s, c, j0 + 2);
-        FState lo, tm;
-        cell_states(a, bm, rc, lo, tm);
-        FState bc;
-        cell_states(bm, rc, rn, bc, tc);
-        fyb = face_flux<HLLC, true, true>(g, tm, bm.b, bc, rc.b);
-        t_prev = odd(bm);
-        t_rc = odd(rc);
-        t_rn = odd(rn);
-        t_rnn = odd(rnn);
+        const Cell a = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0 - 2, first.r[0]);
+        const Cell rc = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0 - 1, first.r[1]);
+        const Cell rn = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0, first.r[2]);
+        const Cell rnn = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0 + 1, first.r[3]);
+        FState lo, hi;
+        cell_states(a, rc, rn, lo, hi);
+        odd_prev = __any(unbounded(a));
+        bc = bits(rc);
+        bn = bits(rn);
+        bnn = bits(rnn);
+        put(0, rc);
+        put(1, rn);
+        put(2, rnn);
+        hand_up(hi, Face{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, surf(1, lane) - surf(0, lane));
     }
-    const bool own = c < d.nx;
-    Cell un;   // U^n at (c, j) for the RK2 average
-    un.h = 0.0; un.hu = 0.0; un.hv = 0.0; un.b = 0.0;
-    if (!FASTK && read_un && own) {
-        const long long k = (long long)j0 * pitch + c;
-        un.h = d.ah[k]; un.hu = d.ahu[k]; un.hv = d.ahv[k];
-    }
-    __syncthreads();
+    // a column of the grid for the lanes that own none: their loads of U^n are not used
+    const int c_in = min(max(c, 0), d.nx - 1);
 
-    for (int j = j0; j < j1; ++j) {
-        const int r = j - j0;
-        const bool more = j + 1 < j1;
-        Cell nxt, nun;
-        if (more) nxt = ld<EDGE, FEAT>(d, s, c, j + 3);
-        // U^n at (c, j) for the RK2 average, needed at the end of the row.
-        // Kernels with the fast path load it here (its load hides behind the
-        // faces, and it saves the registers of a second row); the others
-        // fetch it a row ahead, which a launch of few waves needs.
-        if constexpr (FASTK) {
-            if (read_un && own) {
-                const long long k = (long long)j * pitch + c;
-                un.h = d.ah[k]; un.hu = d.ahu[k]; un.hv = d.ahv[k];
-            }
-        } else if (more && read_un && own) {
-            const long long k = (long long)(j + 1) * pitch + c;
-            nun.h = d.ah[k]; nun.hu = d.ahu[k]; nun.hv = d.ahv[k];
-        }
-        FState tn;
-        Face fyt;
-        auto row = [&](auto exact) {
+    for (int j = j0 - 1; j < j1; ++j) {
+        const bool inner = j >= j0;   // the row before the first only gives its upper face
+        const bool plain_row = plain || odd_prev || bc.odd || bn.odd || bnn.odd;
+        double fh = 0.0, fhu = 0.0, fhv = 0.0;   // the row's flux divergence
+        auto faces = [&](auto exact) {
             constexpr bool EX = decltype(exact)::value;
-            // faces and cells take the fast path (swe_core.hpp) where the
-            // wavefront allows it; lanes up to the first column past the
-            // grid feed an owned cell through their x-face
-            const bool fast = FASTK && !EX && try_fast;
-            const bool use_x = c <= d.nx;
             // y: slope of row j+1 and the face between rows j and j+1
-            FState bn;
-            cell_states(rc, rn, rnn, bn, tn);
-            if (fast) fyt = face_flux_auto<HLLC, true>(g, tc, rc.b, bn, rn.b, own);
-            else fyt = face_flux<HLLC, true, EX>(g, tc, rc.b, bn, rn.b);
+            YPart y;
+            {
+                const FState tc{ring.up[0][lane], ring.up[1][lane], ring.up[2][lane]};
+                const double b_c = ring.v[sc][3][lane], b_n = ring.v[sn][3][lane];
+                const Surf n = surf(sn, lane), dp = surf(snn, lane) - n;
+                FState lo, tn;
+                Face fyt;
+                if (EX) {
+                    cell_states(cell(sc, lane), cell(sn, lane), cell(snn, lane), lo, tn);
+                    fyt = face_flux<HLLC, true>(g, tc, b_c, lo, b_n);
+                } else {
+                    const Surf dm{ring.up[7][lane], ring.up[8][lane], ring.up[9][lane]};
+                    states_row(dm, dp, n, b_n, __builtin_amdgcn_inverse_ballot_w64(bn.thin | bc.dry | bnn.dry), lo,
+                               tn);
+                    fyt = face_row<HLLC, true>(g, tc, b_c, lo, b_n, own);
+                }
+                const Face fyb{ring.up[3][lane], ring.up[4][lane], ring.up[5][lane], ring.up[6][lane], 0.0, 0.0};
+                if (EX) y = divergence_y<DIV_PLAIN>(g, d.sdy, fyb, fyt);
+                else if (two_op) y = divergence_y<DIV_TWO_OP>(g, d.sdy, fyb, fyt);
+                else y = divergence_y<DIV_SHARED>(g, d.sdy, fyb, fyt);
+                hand_up(tn, fyt, dp);
+            }
+            if (!inner) return;
 
-            // x: slope of row j, face left of each cell, face right from the next lane
-            Cell xm = shfl_up1(rc);
-            Cell xp = shfl_down1(rc);
-            if (lane == 0) xm = Cell{L.hl[0][r], L.hl[1][r], L.hl[2][r], L.hl[3][r]};
-            if (lane == WAVE - 1) xp = Cell{L.hr[0][r], L.hr[1][r], L.hr[2][r], L.hr[3][r]};
-            FState xlo, xhi;
-            cell_states(xm, rc, xp, xlo, xhi);
-            FState rprev = shfl_up1(xhi);
-            if (lane == 0) rprev = FState{L.ph[0][r], L.ph[1][r], L.ph[2][r]};
-            Face fxl;
-            if (fast) fxl = face_flux_auto<HLLC, false>(g, rprev, xm.b, xlo, rc.b, use_x);
-            else fxl = face_flux<HLLC, false, EX>(g, rprev, xm.b, xlo, rc.b);
-            Face fxr = shfl_down1(fxl);
-            if (lane == WAVE - 1)
-                fxr = Face{L.pf[0][r], L.pf[1][r], L.pf[2][r], L.pf[3][r], L.pf[4][r], L.pf[5][r]};
+            // x: slope of row j, the face right of each cell, the face left of it from the lane before
+            const double b_c = ring.v[sc][3][lane], b_p = ring.v[sc][3][lane_p];
+            FState lo, hi;
+            Face fxl, fxr;
+            if (EX) {
+                cell_states(cell(sc, lane_m), cell(sc, lane), cell(sc, lane_p), lo, hi);
+                fxr = face_flux<HLLC, false>(g, hi, b_c, shfl_down1(lo), b_p);
+            } else {
+                const Surf q = surf(sc, lane);
+                states_row(q - surf(sc, lane_m), surf(sc, lane_p) - q, q, b_c,
+                           __builtin_amdgcn_inverse_ballot_w64(bc.thin | (bc.dry << 1) | (bc.dry >> 1)), lo, hi);
+                fxr = face_row<HLLC, false>(g, hi, b_c, shfl_down1(lo), b_p, use_x);
+            }
+            fxl.fh = shfl_up1(fxr.fh); fxl.fhu = shfl_up1(fxr.fhu); fxl.fhv = shfl_up1(fxr.fhv);
+            fxl.a = shfl_up1(fxr.a);
+            fxl.c = 0.0; fxl.d = 0.0;
+            if (EX) divergence<DIV_PLAIN>(g, d.sdx, fxl, fxr, y, fh, fhu, fhv);
+            else if (two_op) divergence<DIV_TWO_OP>(g, d.sdx, fxl, fxr, y, fh, fhu, fhv);
+            else divergence<DIV_SHARED>(g, d.sdx, fxl, fxr, y, fh, fhu, fhv);
+        };
+        if (__builtin_expect(plain_row, 0)) faces(ExactTag<true>{});
+        else faces(ExactTag<false>{});
 
-            if (own) {
-                double fh, fhu, fhv;
-                divergence<EX>(g, s.rdx, s.rdy, fxl, fxr, fyb, fyt, fh, fhu, fhv);
-                facc = facc + fh;
-                const long long k = (long long)j * pitch + c;
-                if (REC) {
-                    d.rec[k] = fh; d.rec[d.plane + k] = fhu; d.rec[2 * d.plane + k] = fhv;
-                }
-                double h = rc.h, hu = rc.hu, hv = rc.hv;
-                Frc fr{0.0, 0.0, 0.0, 0.0, 0.0};
-                if (FRC) {
-                    fr.wx = d.fwx[k];
-                    fr.wy = d.fwy[k];
-                    fr.dpdx = d.fdpx[k];
-                    fr.dpdy = d.fdpy[k];
-                    fr.rain = d.frain[k];
-                }
-                const double n_cell = NF ? d.nfield[k] : 0.0;
-                bool body_fast = fast;
-                if (fast) {
-                    bool bad = false;
-                    double h1 = h, hu1 = hu, hv1 = hv;
-                    stage_body_fast<NF, FRC>(s.src, s.dt, fh, fhu, fhv, h1, hu1, hv1, n_cell, fr, bad);
-                    if (__any(bad)) body_fast = false;
-                    else { h = h1; hu = hu1; hv = hv1; }
-                }
-                if (!body_fast) stage_body<EX, NF, FRC>(s.src, s.dt, fh, fhu, fhv, h, hu, hv, n_cell, fr);
+        // Row j+3 and U^n at (c, j), both needed at the end of the row: the
+        // cell update hides them, and the faces keep their registers.  The
+        // loads are unconditional (the last row of the halo again, a cell of
+        // the grid): under a condition the compiler waits for everything in
+        // flight where the paths join.
+        const int jn = min(j + 3, j1 + 1);
+        const Cell src = row_source<EDGE>(d, s, lsrc, jn);
+        Cell un{0.0, 0.0, 0.0, 0.0};
+        if (read_un) {
+            const long long k = (long long)max(j, 0) * pitch + c_in;
+            un.h = d.ah[k]; un.hu = d.ahu[k]; un.hv = d.ahv[k];
+        }
+
+        double h = 0.0, hu = 0.0, hv = 0.0;   // the row's result
+        if (inner && own) {
+            const long long k = (long long)j * pitch + c;
+            if (REC) {
+                d.rec[k] = fh; d.rec[d.plane + k] = fhu; d.rec[2 * d.plane + k] = fhv;
+            }
+            Frc fr{0.0, 0.0, 0.0, 0.0, 0.0};
+            if (FRC) {
+                fr.wx = d.fwx[k];
+                fr.wy = d.fwy[k];
+                fr.dpdx = d.fdpx[k];
+                fr.dpdy = d.fdpy[k];
+                fr.rain = d.frain[k];
+            }
+            const double n_cell = NF ? d.nfield[k] : 0.0;
+            double relax = 0.0;
+            // the cell update; true where it has to be redone with plain divisions
+            auto update = [&](auto exact) -> bool {
+                constexpr bool EX = decltype(exact)::value;
+                relax = 0.0;
+                h = ring.v[sc][4][lane]; hu = ring.v[sc][1][lane]; hv = ring.v[sc][2][lane];
+                if (EX) stage_body<NF, FRC>(s.src, s.dt, fh, fhu, fhv, h, hu, hv, n_cell, fr);
+                else if (stage_body_row<NF, FRC>(s.src, s.dt, fh, fhu, fhv, h, hu, hv, n_cell, fr)) return true;
                 // the sponge follows each fused stage (rki_solver.F90:787,814)
-                if (STAGE == 1 && SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, sacc);
-                // U^n with a tiny value in any lane: the rest of the cell
-                // update with plain divisions
-                const bool ex_un = EX || (read_un && __any(odd(un)));
+                if (STAGE == 1 && SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, relax);
                 if (STAGE == 2) {
                     // rki_kernel_fused.F90:435-463
                     h = 0.5 * (un.h + h);
                     hu = 0.5 * (un.hu + hu);
                     hv = 0.5 * (un.hv + hv);
-                    if (ex_un) {
-                        clamp_desing<true>(g, h, hu, hv);
-                        if (SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, sacc);
-                        smax = dmax(smax, cfl_speed<true>(g, s.rdx, s.rdy, h, hu, hv));
-                    } else {
-                        bool cell_fast = fast;
-                        if (fast) {
-                            bool bad = false;
-                            clamp_fast(g, h, hu, hv, bad);   // passes the values unchanged
-                            cell_fast = !__any(bad);
-                        }
-                        if (!cell_fast) clamp_desing<false>(g, h, hu, hv);
-                        if (SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, sacc);
-                        if (cell_fast && !SPG) smax = dmax(smax, cfl_speed_fast(g, s.rdx, s.rdy, h, hu, hv));
-                        else smax = dmax(smax, cfl_speed<false>(g, s.rdx, s.rdy, h, hu, hv));
-                    }
                 }
-                if (STAGE == 3) {
-                    if (s.blend) {  // compute_ssp_combine, rki_kernel_update.F90:183-206
-                        h = s.alpha * un.h + s.a_prev * h;
-                        hu = s.alpha * un.hu + s.a_prev * hu;
-                        hv = s.alpha * un.hv + s.a_prev * hv;
-                        if (ex_un) clamp_desing<true>(g, h, hu, hv);
-                        else clamp_desing<false>(g, h, hu, hv);
-                    }
-                    if (SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, sacc);   // :919-920, at beta_i dt
-                    if (s.last) {
-                        if (ex_un) smax = dmax(smax, cfl_speed<true>(g, s.rdx, s.rdy, h, hu, hv));
-                        else smax = dmax(smax, cfl_speed<false>(g, s.rdx, s.rdy, h, hu, hv));
-                    }
+                if (STAGE == 3 && s.blend) {  // compute_ssp_combine, rki_kernel_update.F90:183-206
+                    h = s.alpha * un.h + s.a_prev * h;
+                    hu = s.alpha * un.hu + s.a_prev * hu;
+                    hv = s.alpha * un.hv + s.a_prev * hv;
                 }
-                s.oh[k] = h; s.ohu[k] = hu; s.ohv[k] = hv;
-                if ((STAGE == 1 || (STAGE == 3 && s.first)) && d.sh != nullptr) {
-                    // h0, hu0, hv0 (rki_kernel_fused.F90:224-226, rki_solver.F90:879-881)
-                    d.sh[k] = rc.h; d.shu[k] = rc.hu; d.shv[k] = rc.hv;
+                if (STAGE == 2 || (STAGE == 3 && s.blend)) {
+                    if (EX) clamp_desing(g, h, hu, hv);
+                    else if (clamp_row(g, h, hu, hv)) return true;
                 }
-            }
-        };
-        const bool lane_tiny = t_prev || t_rc || t_rn || t_rnn;
-        if (__any(lane_tiny) || ((edge_rows >> r) & 1ull))
-            row(ExactTag<true>{});
-        else
-            row(ExactTag<false>{});
-
-        fyb = fyt;
-        tc = tn;
-        rc = rn;
-        rn = rnn;
-        t_prev = t_rc;
-        t_rc = t_rn;
-        t_rn = t_rnn;
-        if (more) {
-            rnn = nxt;
-            t_rnn = odd(nxt);
-            if (!FASTK && read_un) un = nun;
+                // :919-920, at beta_i dt in the generic schemes
+                if (STAGE != 1 && SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, relax);
+                if (STAGE == 2 || (STAGE == 3 && s.last)) {
+                    if (EX) cfl_plain(g, h, hu, hv, smax);
+                    else cfl_row(g, same, h, hu, hv, smax);
+                }
+                return false;
+            };
+            if (__builtin_expect(plain_row, 0) || __builtin_expect(update(ExactTag<false>{}), 0))
+                update(ExactTag<true>{});
+            facc = facc + fh;
+            sacc = sacc + relax;
         }
+
+        // The prefetched row is waited for before the stores are issued:
+        // loads and stores share one in-order counter, and a wait after the
+        // stores waits for them too (a quarter of a row's time, 4096^2).
+        Cell nxt{0.0, 0.0, 0.0, 0.0};
+        odd_prev = bc.odd;
+        bc = bn;
+        bn = bnn;
+        if (j + 1 < j1) {
+            nxt = row_cell<EDGE, FEAT>(d, s, lsrc, c, jn, src);
+            bnn = bits(nxt);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (inner && own) {
+            const long long k = (long long)j * pitch + c;
+            if ((STAGE == 1 || (STAGE == 3 && s.first)) && d.sh != nullptr) {
+                // h0, hu0, hv0 (rki_kernel_fused.F90:224-226, rki_solver.F90:879-881)
+                d.sh[k] = ring.v[sc][4][lane]; d.shu[k] = ring.v[sc][1][lane]; d.shv[k] = ring.v[sc][2][lane];
+            }
+            s.oh[k] = h; s.ohu[k] = hu; s.ohv[k] = hv;
+        }
+        put(sc, nxt);   // row j+3 takes the place of row j
+        const int free_slot = sc;
+        sc = sn; sn = snn; snn = free_slot;
     }
     fsum = facc;
     ssum = sacc;
-    return smax;
+    return cfl_max(smax, same, d.dx, d.dy);
 }
 
 }  // namespace rk

@@ -306,6 +306,6 @@ class Grid:
         check("rkg_set_tile_rows", self._lib.rkg_set_tile_rows(self.handle, int(rows)))
 
     def set_fast_path(self, mode: int) -> None:
-        """Stage kernels' fast path: 0 by the launch's tile count (default),
-        1 always, -1 never; the results are the same bits."""
+        """Stage kernels' row path: 0 (default) and 1 on, -1 plain divisions
+        for every row; the results are the same bits."""
         check("rkg_set_fast_path", self._lib.rkg_set_fast_path(self.handle, int(mode)))
