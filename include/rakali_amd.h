@@ -194,9 +194,8 @@ int rkg_total_mass(rkg_grid *g, double *mass);
 /* Waits for all queued work of this grid. */
 int rkg_sync(rkg_grid *g);
 
-/* Rows per tile of the stage kernels (1..64; 0, the default, chooses 16 for
- * grids of at least 8192 such tiles and 8 below).  The get call returns the
- * rows in use. */
+/* Rows per tile of the stage kernels (1..64; 0, the default, chooses 1 to
+ * 20 by the grid's size).  The get call returns the rows in use. */
 int rkg_set_tile_rows(rkg_grid *g, int rows);
 int rkg_get_tile_rows(rkg_grid *g, int *rows);
 /* How the stage kernels evaluate their rows: 0 (default) and 1 take the row
