@@ -1778,9 +1778,12 @@ int rkg_adjoint_gradient(rkg_adjoint* a, int field, double* dst, int ld, int on_
     default: set_error("no gradient for field %d", field); return RKG_ERR_RANGE;
     }
     if (!dst || ld < g->cfg.nx) { set_error("bad buffer or leading dimension"); return RKG_ERR_RANGE; }
-    HIP_TRY(hipMemcpy2DAsync(dst, (size_t)ld * sizeof(double), src, (size_t)g->pitch * sizeof(double),
-                             (size_t)g->cfg.nx * sizeof(double), (size_t)g->cfg.ny,
-                             on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, g->stream));
+    const size_t W = sizeof(double), nx = (size_t)g->cfg.nx, ny = (size_t)g->cfg.ny, pitch = (size_t)g->pitch;
+    if (!on_device) {
+        HIP_TRY(plane_to_host(*g->stage, dst, (size_t)ld, src, pitch, nx, ny, g->stream));
+        return RKG_OK;
+    }
+    HIP_TRY(hipMemcpy2DAsync(dst, (size_t)ld * W, src, pitch * W, nx * W, ny, hipMemcpyDeviceToDevice, g->stream));
     HIP_TRY(hipStreamSynchronize(g->stream));
     return RKG_OK;
 }

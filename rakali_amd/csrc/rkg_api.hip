@@ -325,6 +325,90 @@ int check_config(const rkg_config* c) {
 
 }  // namespace
 
+rk::HostStage::~HostStage() {
+    if (mem) (void)hipHostFree(mem);
+}
+
+namespace {
+
+// Whether this host memory goes through the stage: pageable memory, more than
+// one row (a single row is one transfer anyway), rows that fit a piece; and
+// the stage has room for two pieces, or for the plane.
+bool staged(HostStage& st, const void* host, size_t row, size_t ny) {
+    if (ny < 2 || row > HostStage::PIECE) return false;
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, host) != hipSuccess) { (void)hipGetLastError(); return false; }
+    if (a.type != hipMemoryTypeUnregistered) return false;
+    const size_t whole = row * ny, need = whole <= HostStage::PIECE ? whole : 2 * HostStage::PIECE;
+    if (st.bytes < need) {
+        // an allocation does not disturb a capture on another thread
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (st.mem) (void)hipHostFree(st.mem);
+        st.bytes = 0;
+        const bool ok = hipHostMalloc((void**)&st.mem, need, hipHostMallocDefault) == hipSuccess;
+        if (!ok) { st.mem = nullptr; (void)hipGetLastError(); }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (!ok) return false;
+        st.bytes = need;
+    }
+    return true;
+}
+
+void copy_rows(double* dst, size_t ldd, const double* src, size_t lds, size_t nx, size_t rows) {
+    if (ldd == nx && lds == nx) { memcpy(dst, src, nx * rows * sizeof(double)); return; }
+    for (size_t j = 0; j < rows; ++j) memcpy(dst + j * ldd, src + j * lds, nx * sizeof(double));
+}
+
+}  // namespace
+
+hipError_t rk::plane_to_host(HostStage& st, double* dst, size_t ld, const double* plane, size_t pitch, size_t nx, size_t ny,
+                             hipStream_t stream) {
+    const size_t W = sizeof(double);
+    std::lock_guard<std::mutex> hold(st.lock);
+    hipError_t e = hipSuccess;
+    if (!staged(st, dst, nx * W, ny)) {
+        e = hipMemcpy2DAsync(dst, ld * W, plane, pitch * W, nx * W, ny, hipMemcpyDeviceToHost, stream);
+        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    }
+    const size_t rows = HostStage::PIECE / (nx * W);   // per piece
+    auto rows_of = [&](size_t j) { return std::min(rows, ny - j); };
+    auto half = [&](size_t k) { return st.mem + (k & 1) * (HostStage::PIECE / W); };
+    auto fetch = [&](size_t k) {
+        const size_t j = k * rows;
+        return hipMemcpy2DAsync(half(k), nx * W, plane + j * pitch, pitch * W, nx * W, rows_of(j), hipMemcpyDeviceToHost, stream);
+    };
+    e = fetch(0);
+    for (size_t k = 0, j = 0; j < ny && e == hipSuccess; ++k, j += rows) {
+        e = hipStreamSynchronize(stream);
+        if (e == hipSuccess && j + rows < ny) e = fetch(k + 1);
+        if (e == hipSuccess) copy_rows(dst + j * ld, ld, half(k), nx, nx, rows_of(j));
+    }
+    return e;
+}
+
+hipError_t rk::plane_from_host(HostStage& st, double* plane, size_t pitch, const double* src, size_t ld, size_t nx, size_t ny,
+                               hipStream_t stream) {
+    const size_t W = sizeof(double);
+    std::lock_guard<std::mutex> hold(st.lock);
+    hipError_t e = hipSuccess;
+    if (!staged(st, src, nx * W, ny)) {
+        e = hipMemcpy2DAsync(plane, pitch * W, src, ld * W, nx * W, ny, hipMemcpyHostToDevice, stream);
+        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    }
+    const size_t rows = HostStage::PIECE / (nx * W);
+    for (size_t k = 0, j = 0; j < ny && e == hipSuccess; ++k, j += rows) {
+        // the half's previous piece, two before, has left: the last wait was for it
+        double* half = st.mem + (k & 1) * (HostStage::PIECE / W);
+        const size_t n = std::min(rows, ny - j);
+        copy_rows(half, nx, src + j * ld, ld, nx, n);
+        if (k > 0) e = hipStreamSynchronize(stream);
+        if (e == hipSuccess)
+            e = hipMemcpy2DAsync(plane + j * pitch, pitch * W, half, nx * W, nx * W, n, hipMemcpyHostToDevice, stream);
+    }
+    return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+}
+
 int rk::validate_config(const rkg_config* c) { return check_config(c); }
 
 void rk::grid_retain(rkg_grid* g) { ++g->refs; }
@@ -347,6 +431,7 @@ void rk::grid_release(rkg_grid* g) {
         if (g->ev[k]) (void)hipEventDestroy(g->ev[k]);
     if (g->own_stream && g->stream && stream_release(g->stream)) (void)hipStreamDestroy(g->stream);
     g->magic = GRID_DEAD;
+    delete g->stage;
     delete g;
 }
 
@@ -388,6 +473,7 @@ int rkg_create(const rkg_config* cfg, void* stream, rkg_grid** out) {
         stream_register(g->stream);
         g->own_stream = true;
     }
+    g->stage = new HostStage();
     long long pitch = ((long long)cfg->nx + 15) / 16 * 16;
     if (pitch % 1024 == 0) pitch += 32;  // break power-of-two row strides
     g->pitch = pitch;
@@ -436,17 +522,22 @@ static int copy_field(rkg_grid* g, int field, double* host_or_dev, int ld, bool 
         return RKG_ERR_RANGE;
     }
     if (!host_or_dev || ld < g->cfg.nx) { set_error("bad buffer or leading dimension"); return RKG_ERR_RANGE; }
-    const size_t w = (size_t)g->cfg.nx * sizeof(double);
+    const size_t W = sizeof(double), nx = (size_t)g->cfg.nx, ny = (size_t)g->cfg.ny, pitch = (size_t)g->pitch;
+    if (kind == hipMemcpyHostToDevice) {
+        HIP_TRY(plane_from_host(*g->stage, f, pitch, host_or_dev, (size_t)ld, nx, ny, g->stream));
+    } else if (kind == hipMemcpyDeviceToHost) {
+        HIP_TRY(plane_to_host(*g->stage, host_or_dev, (size_t)ld, f, pitch, nx, ny, g->stream));
+    } else {
+        if (upload)
+            HIP_TRY(hipMemcpy2DAsync(f, pitch * W, host_or_dev, (size_t)ld * W, nx * W, ny, kind, g->stream));
+        else
+            HIP_TRY(hipMemcpy2DAsync(host_or_dev, (size_t)ld * W, f, pitch * W, nx * W, ny, kind, g->stream));
+        HIP_TRY(hipStreamSynchronize(g->stream));
+    }
     if (upload) {
-        HIP_TRY(hipMemcpy2DAsync(f, (size_t)g->pitch * sizeof(double), host_or_dev, (size_t)ld * sizeof(double), w,
-                                 (size_t)g->cfg.ny, kind, g->stream));
         g->speed_stale = true;
         if (field == RKG_FIELD_PRESSURE) g->frc_grad_stale = true;
-    } else {
-        HIP_TRY(hipMemcpy2DAsync(host_or_dev, (size_t)ld * sizeof(double), f, (size_t)g->pitch * sizeof(double), w,
-                                 (size_t)g->cfg.ny, kind, g->stream));
     }
-    HIP_TRY(hipStreamSynchronize(g->stream));
     return RKG_OK;
 }
 

@@ -102,6 +102,7 @@ struct rkg_ensemble {
     hipGraphExec_t graph;  // two steps, starting at parity 0
     bool graph_valid;
     long long steps_since_graph;
+    HostStage stage;       // uploads and downloads from and to pageable memory
 };
 
 namespace {
@@ -402,10 +403,8 @@ int rkg_ensemble_upload(rkg_ensemble* e, int m, int field, const double* src, in
     if (field < RKG_FIELD_H || field > RKG_FIELD_B) { set_error("field %d is not writable", field); return RKG_ERR_RANGE; }
     const rkg_config& c = e->cfg[m];
     if (!src || ld < c.nx) { set_error("bad buffer or leading dimension"); return RKG_ERR_RANGE; }
-    HIP_TRY(hipMemcpy2DAsync(ens_field(e, m, field), (size_t)e->pitch[m] * sizeof(double), src,
-                             (size_t)ld * sizeof(double), (size_t)c.nx * sizeof(double), (size_t)c.ny,
-                             hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
+    HIP_TRY(plane_from_host(e->stage, ens_field(e, m, field), (size_t)e->pitch[m], src, (size_t)ld, (size_t)c.nx, (size_t)c.ny,
+                            e->stream));
     e->speed_stale[m] = 1;
     return RKG_OK;
 }
@@ -417,9 +416,7 @@ int rkg_ensemble_download(rkg_ensemble* e, int m, int field, double* dst, int ld
     const rkg_config& c = e->cfg[m];
     if (!f) { set_error("unknown field %d", field); return RKG_ERR_RANGE; }
     if (!dst || ld < c.nx) { set_error("bad buffer or leading dimension"); return RKG_ERR_RANGE; }
-    HIP_TRY(hipMemcpy2DAsync(dst, (size_t)ld * sizeof(double), f, (size_t)e->pitch[m] * sizeof(double),
-                             (size_t)c.nx * sizeof(double), (size_t)c.ny, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
+    HIP_TRY(plane_to_host(e->stage, dst, (size_t)ld, f, (size_t)e->pitch[m], (size_t)c.nx, (size_t)c.ny, e->stream));
     return RKG_OK;
 }
 

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <mutex>
 
 #include "../../include/rakali_amd.h"
 #include "swe_kernels.hpp"
@@ -18,6 +19,28 @@ __attribute__((visibility("hidden"), format(printf, 1, 2))) void set_error(const
 
 namespace rk {
 struct GaugeState;   // gauge stations and their time series (rkg_gauges.hip)
+
+// Pinned memory between the planes of one grid or ensemble and its caller's
+// pageable arrays.  A pitched copy to pageable memory goes row by row, 7 us
+// each (768 x 700: 4.9 ms down, 6.5 ms up); to pinned memory it is one
+// transfer at the link's rate (83 us) plus a copy in host memory (55 us).  A
+// plane goes through in pieces, one in transfer while the host copies the
+// other.  Made on first use, at most 2 * PIECE bytes, freed with its owner;
+// calls from several threads take turns.
+struct HostStage {
+    static constexpr size_t PIECE = (size_t)2 << 20;
+    std::mutex lock;
+    double* mem = nullptr;
+    size_t bytes = 0;     // of mem
+    ~HostStage();
+};
+
+// ny rows of nx values between a plane (rows `pitch` apart) and host memory
+// (rows ld apart), complete on return.
+__attribute__((visibility("hidden"))) hipError_t plane_to_host(HostStage& st, double* dst, size_t ld, const double* plane,
+                                                               size_t pitch, size_t nx, size_t ny, hipStream_t stream);
+__attribute__((visibility("hidden"))) hipError_t plane_from_host(HostStage& st, double* plane, size_t pitch, const double* src,
+                                                                 size_t ld, size_t nx, size_t ny, hipStream_t stream);
 }
 
 // One grid: device buffers, stream and control slots (rkg_grid of the ABI).
@@ -58,6 +81,7 @@ struct rkg_grid {
     double prof_ms[2];     // accumulated stage-1 / stage-2 kernel time
     long long prof_n;
     rk::GaugeState* gauges;  // stations, or null
+    rk::HostStage* stage;    // uploads and downloads from and to pageable memory
 };
 
 namespace rk {
