@@ -309,7 +309,11 @@ int rkg_ensemble_create(const rkg_config* cfgs, int n, void* stream, rkg_ensembl
     e->magic = 0;
     e->n = n;
     e->cfg.assign(cfgs, cfgs + n);
-    e->ty = 32;
+    e->ty = rows_for([=](int rows) {
+        long long t = 0;
+        for (int m = 0; m < n; ++m) t += grid_tiles(cfgs[m].nx, cfgs[m].ny, rows);
+        return t;
+    }, 4);
     e->schedule = 0;
     e->use_hllc = cfgs[0].use_hllc != 0;
     e->speed_stale.assign(n, 1);

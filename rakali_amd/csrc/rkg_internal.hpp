@@ -157,13 +157,13 @@ inline double* field_ptr(rkg_grid* g, int field) {
     }
 }
 
-// Rows per stage tile by grid size.  A tile costs half a row more than its
-// rows (the march starts a row early), and a launch of few tiles lasts as long
-// as one tile, so a grid takes the shortest tiles that leave one wavefront on
-// each of the 1024 SIMDs while they have at most 8 rows, then two while at
-// most 10.  Larger grids run several tiles per wavefront slot: 10 rows, and
-// 20 once they have 8192 tiles of 16, where the uneven end of a launch no
-// longer matters.  Measured (us per step, one grid / each of three grids on
+// Rows per stage tile; tiles(rows) counts a launch's tiles.  A tile costs half
+// a row more than its rows (the march starts a row early), and a launch of few
+// tiles lasts as long as one tile, so it takes the shortest tiles that leave
+// one wavefront on each of the 1024 SIMDs while they have at most 8 rows, then
+// two while at most 10.  Larger launches run several tiles per wavefront slot:
+// 10 rows, and 20 once there are 8192 tiles of 16, where the uneven end of a
+// launch no longer matters.  Measured (us per step, one grid / each of three grids on
 // their own streams):
 //   200x100    1 row  30 / 11,   8 rows  62 / 24
 //   512x512    5 rows 56 / 25,   8 rows  66 / 29
@@ -171,14 +171,25 @@ inline double* field_ptr(rkg_grid* g, int field) {
 //   1024x1024  10 rows 114 / 57, 6 rows 110 / 68,  19 rows 145 / 66
 //   3000x2000  10 rows 386 / 331, 16 rows 416 / 326
 //   4096x4096  20 rows 950 / 880, 10 rows 967 / 916, 32 rows 978 / 870
+// and for ensembles (their tiles have 4 rows at least):
+//   4 of 64..200      4 rows 45, 8 rows 65, 32 rows 192
+//   12 of 200..400    10 rows 108, 4 rows 117, 32 rows 204
+//   16 of 128..768    10 rows 250, 20 rows 286, 32 rows 278
+//   32 of 512..1024   20 rows 1207, 10 rows 1301, 32 rows 1208
+template <class TILES>
+int rows_for(TILES tiles, int least) {
+    for (int waves = 1; waves <= 2; ++waves)
+        for (int rows = least; rows <= (waves == 1 ? 8 : 10); ++rows)
+            if (tiles(rows) <= 1024 * waves) return rows;
+    return tiles(16) >= 8192 ? 20 : 10;
+}
+
+inline long long grid_tiles(int nx, int ny, int rows) {
+    return (long long)((nx + OWN - 1) / OWN) * ((ny + rows - 1) / rows);
+}
+
 inline int default_tile_rows(int nx, int ny) {
-    const long long strips = (nx + OWN - 1) / OWN;
-    for (int waves = 1; waves <= 2; ++waves) {
-        const long long segs = 1024 * waves / strips;
-        const long long rows = segs > 0 ? (ny + segs - 1) / segs : ny;
-        if (rows <= (waves == 1 ? 8 : 10)) return (int)rows;
-    }
-    return strips * ((ny + 15) / 16) >= 8192 ? 20 : 10;
+    return rows_for([=](int rows) { return grid_tiles(nx, ny, rows); }, 1);
 }
 
 // A tile next to a one-row tile at a south Chapman edge would read a ghost
