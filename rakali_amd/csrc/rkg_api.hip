@@ -109,9 +109,7 @@ int refresh_speed(rkg_grid* g) {
     const CtrlSlot c = g->ctrl_host[g->parity];
     hipLaunchKernelGGL(k_ctrl_reset, dim3(1), dim3(64), 0, g->stream, g->ctrl, g->parity, c.t, c.dt,
                        c.step_count, c.mass_out, c.mass_src);
-    const long long n = (long long)g->cfg.nx * g->cfg.ny;
-    int blocks = (int)std::min<long long>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_init_speed, dim3(blocks), dim3(256), 0, g->stream, d, g->parity);
+    hipLaunchKernelGGL(k_init_speed, dim3(sweep_blocks((long long)g->cfg.nx * g->cfg.ny)), dim3(256), 0, g->stream, d, g->parity);
     HIP_TRY(hipGetLastError());
     g->speed_stale = false;
     return RKG_OK;
@@ -198,9 +196,7 @@ int launch_generic(rkg_grid* g, int n, int mode, double tlim) {
             in = out;
         }
         if (T.n == 1) {
-            const long long cells = (long long)d.nx * d.ny;
-            const int blocks = (int)std::min<long long>((cells + 255) / 256, 4096);
-            hipLaunchKernelGGL(k_euler_finish, dim3(blocks), dim3(256), 0, g->stream, d, g->parity);
+            hipLaunchKernelGGL(k_euler_finish, dim3(sweep_blocks((long long)d.nx * d.ny)), dim3(256), 0, g->stream, d, g->parity);
         }
         g->parity ^= 1;
         if (g->gauges) {

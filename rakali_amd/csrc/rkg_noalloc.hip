@@ -28,10 +28,9 @@ using namespace rk;
 
 namespace {
 
-constexpr long long CTRL_DOUBLES = 32;   // 256 B: two 64-byte control slots, padded
+constexpr long long CTRL_DOUBLES = 2 * sizeof(CtrlSlot) / sizeof(double);   // two control slots
+static_assert(CTRL_DOUBLES % 16 == 0, "the planes behind the control slots stay aligned to cache lines");
 constexpr long long SCRATCH_DOUBLES = CTRL_DOUBLES + 3LL * RKG_NOALLOC_MAX_CELLS;
-
-static_assert(2 * sizeof(CtrlSlot) <= CTRL_DOUBLES * sizeof(double), "control slots exceed their region");
 
 __device__ __align__(256) double scratch[SCRATCH_DOUBLES];
 
@@ -109,8 +108,7 @@ extern "C" int rkg_step_noalloc(const rkg_config* cfg, double* h, double* hu, do
     // node if the caller captures the call); the speed maximum of the state
     // is taken afresh, as rkg_step does after an upload.
     hipLaunchKernelGGL(k_ctrl_reset, dim3(1), dim3(64), 0, st, d.ctrl, 0, *t, *dt, *step_count, 0.0, 0.0);
-    const int blocks = (int)std::min<long long>(((long long)cfg->nx * cfg->ny + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_init_speed, dim3(blocks), dim3(256), 0, st, d, 0);
+    hipLaunchKernelGGL(k_init_speed, dim3(sweep_blocks((long long)cfg->nx * cfg->ny)), dim3(256), 0, st, d, 0);
     int parity = 0;
     for (int k = 0; k < n; ++k) {
         for (int stage = 1; stage <= 2; ++stage) {

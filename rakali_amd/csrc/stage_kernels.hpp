@@ -17,12 +17,45 @@ constexpr int MODE_STEP = 0;
 constexpr int MODE_ADVANCE = 1;
 constexpr int MASS_BLOCKS = 512;
 
+// Way `lane % SPEED_WAYS` of a slot's max CFL speed.
+__device__ __forceinline__ unsigned long long speed_way(const CtrlSlot& c) {
+    return c.speed[(threadIdx.x & (SPEED_WAYS - 1)) * SPEED_STRIDE];
+}
+
+template <int ROR>
+__device__ __forceinline__ double row_ror(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + ROR, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + ROR, 0xf, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+__device__ __forceinline__ double wave_first(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// The maximum of the ways that the lanes of a row of 16 hold.
+__device__ __forceinline__ double speed_max(unsigned long long way) {
+    static_assert(SPEED_WAYS == 16, "one way per lane of a row");
+    double v = __longlong_as_double((long long)way);
+    v = dmax(v, row_ror<8>(v));
+    v = dmax(v, row_ror<4>(v));
+    v = dmax(v, row_ror<2>(v));
+    v = dmax(v, row_ror<1>(v));
+    return v;
+}
+
+__device__ __forceinline__ void speed_add(CtrlSlot& c, unsigned who, double speed) {
+    atomicMax(&c.speed[(who & (SPEED_WAYS - 1)) * SPEED_STRIDE], (unsigned long long)__double_as_longlong(speed));
+}
+
 // dt of a step from the control slot of the state it starts from:
 // rki_solver.F90:728-745 with rki_api.F90:377 (step) / :402 (advance).
-__device__ __forceinline__ double step_dt(const GridDesc& d, const CtrlSlot& cp, double dt_max) {
+__device__ __forceinline__ double step_dt(const GridDesc& d, const CtrlClock& cp, double max_speed, double dt_max) {
     if (d.dt_fixed > 0.0) return dmin(d.dt_fixed, dt_max);
     if (cp.step_count % d.cfl_interval == 0 || cp.dt <= 0.0) {
-        const double max_speed = __longlong_as_double((long long)cp.speed_bits);
         double dt;
         if (max_speed > 0.0)
             dt = d.cfl / max_speed;
@@ -79,16 +112,17 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, in
     s.eta_tidal = 0.0;
     double t_tide;   // bc%time of the stage; the tide is evaluated by edge tiles only
     if (STAGE == 1 || (STAGE == 3 && gs.first)) {
-        const CtrlSlot cp = d.ctrl[p];
+        const CtrlClock cp = d.ctrl[p];
+        const unsigned long long way = speed_way(d.ctrl[p]);
         const bool active = (mode == MODE_STEP) || (cp.t < tlim - 1.0e-10);
         const double dt_max = tlim - cp.t;
-        const double dt = active ? step_dt(d, cp, dt_max) : cp.dt;
+        const double dt = active ? wave_first(step_dt(d, cp, speed_max(way), dt_max)) : cp.dt;
+        if (leader && threadIdx.x < SPEED_WAYS) d.ctrl[1 - p].speed[threadIdx.x * SPEED_STRIDE] = active ? 0ull : way;
         if (leader && threadIdx.x == 0) {
-            CtrlSlot* q = &d.ctrl[1 - p];
+            CtrlClock* q = &d.ctrl[1 - p];
             q->t = active ? cp.t + dt : cp.t;
             q->dt = dt;
             q->step_count = active ? cp.step_count + 1 : cp.step_count;
-            q->speed_bits = active ? 0ull : cp.speed_bits;
             q->mass_out = cp.mass_out;
             q->mass_src = cp.mass_src;
             q->active = active ? 1 : 0;
@@ -114,8 +148,8 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, in
         }
         t_tide = cp.t;  // stage abscissa c_1 = 0
     } else if (STAGE == 3) {
-        const CtrlSlot cp = d.ctrl[p];
-        const CtrlSlot cq = d.ctrl[1 - p];
+        const CtrlClock cp = d.ctrl[p];
+        const CtrlClock cq = d.ctrl[1 - p];
         if (!cq.active) return;
         s.oh = gs.oh; s.ohu = gs.ohu; s.ohv = gs.ohv;
         s.dt = gs.beta * cq.dt;
@@ -124,7 +158,7 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, in
         s.radiate = true;       // against the previous stage's input
         s.prev_h = gs.ph;
     } else {
-        const CtrlSlot cq = d.ctrl[1 - p];
+        const CtrlClock cq = d.ctrl[1 - p];
         if (!cq.active) return;
         s.oh = d.o2h; s.ohu = d.o2hu; s.ohv = d.o2hv;
         s.dt = cq.dt;
@@ -154,8 +188,7 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, in
     }
     if (STAGE == 2 || STAGE == 3) {
         smax = wave_max(smax);
-        if (threadIdx.x == 0 && smax > 0.0)
-            atomicMax(&d.ctrl[1 - p].speed_bits, (unsigned long long)__double_as_longlong(smax));
+        if (threadIdx.x == 0 && smax > 0.0) speed_add(d.ctrl[1 - p], (unsigned)(strip + seg * d.nstrips), smax);
     }
     if (STAGE != 3 && d.mpart != nullptr) {  // accumulate_boundary_mass_out's sum, per tile
         fsum = wave_sum(fsum);
@@ -192,14 +225,14 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_
 }
 
 // Resets control slot p to time t / step count n with an empty speed max;
-// the mass budget is set to mass_out.
+// the mass budget is set to mass_out.  One workgroup of 64 threads.
 __global__ void k_ctrl_reset(CtrlSlot* ctrl, int p, double t, double dt, long long n, double mass_out,
                              double mass_src) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+    if (threadIdx.x < SPEED_WAYS) ctrl[p].speed[threadIdx.x * SPEED_STRIDE] = 0ull;
+    if (threadIdx.x == 0) {
         ctrl[p].t = t;
         ctrl[p].dt = dt;
         ctrl[p].step_count = n;
-        ctrl[p].speed_bits = 0ull;
         ctrl[p].mass_out = mass_out;
         ctrl[p].mass_src = mass_src;
         ctrl[p].active = 1;
@@ -253,40 +286,55 @@ __global__ __launch_bounds__(256) void k_budget(CtrlSlot* ctrl, int p, const dou
     }
 }
 
+// Max CFL speed over all cells, whose states load(offset, h, hu, hv) gives;
+// the result is valid in thread 0.  Workgroups of 256 threads, cell after cell
+// with the grid as stride, row and column kept without divisions.
+template <class LOAD>
+__device__ __forceinline__ double plane_speed(const GridDesc& d, LOAD load) {
+    __shared__ double red[4];
+    const long long stride = (long long)gridDim.x * 256, k = blockIdx.x * 256ll + threadIdx.x;
+    const int dj = (int)(stride / d.nx), di = (int)(stride % d.nx);
+    int j = (int)(k / d.nx), i = (int)(k % d.nx);
+    double m = 0.0;
+    while (j < d.ny) {
+        double h, hu, hv;
+        load((long long)j * d.pitch + i, h, hu, hv);
+        m = dmax(m, cfl_speed(d.g, d.dx, d.dy, h, hu, hv));
+        i += di; j += dj;
+        if (i >= d.nx) { i -= d.nx; ++j; }
+    }
+    m = wave_max(m);
+    if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = m;
+    __syncthreads();
+    return dmax(dmax(red[0], red[1]), dmax(red[2], red[3]));
+}
+
 // End of a one-stage (Euler) step: the stage wrote B, so B is copied to A
 // and the CFL max of the new state goes to slot 1-p.  (The stage kernel
 // cannot take that max itself: its leader clears the slot's max while the
 // other tiles of the same launch run.)
 __global__ __launch_bounds__(256) void k_euler_finish(GridDesc d, int p) {
     if (!d.ctrl[1 - p].active) return;
-    double m = 0.0;
-    const long long n = (long long)d.nx * d.ny;
-    for (long long k = blockIdx.x * 256ll + threadIdx.x; k < n; k += (long long)gridDim.x * 256) {
-        const int j = (int)(k / d.nx), i = (int)(k % d.nx);
-        const long long o = (long long)j * d.pitch + i;
-        const double h = d.bh[o], hu = d.bhu[o], hv = d.bhv[o];
+    const double m = plane_speed(d, [&](long long o, double& h, double& hu, double& hv) {
+        h = d.bh[o]; hu = d.bhu[o]; hv = d.bhv[o];
         d.ah[o] = h; d.ahu[o] = hu; d.ahv[o] = hv;
-        m = dmax(m, cfl_speed(d.g, d.dx, d.dy, h, hu, hv));
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & (WAVE - 1)) == 0 && m > 0.0)
-        atomicMax(&d.ctrl[1 - p].speed_bits, (unsigned long long)__double_as_longlong(m));
+    });
+    if (threadIdx.x == 0 && m > 0.0) speed_add(d.ctrl[1 - p], blockIdx.x, m);
 }
 
 // Max CFL speed of the state A into slot p (compute_timestep's reduction,
-// rki_kernel_timestep.F90:53-70).
+// rki_kernel_timestep.F90:53-70).  One atomic per workgroup, spread over the
+// slot's ways: the 16384 atomics of one per wavefront on one address took
+// 190 us at 1024x1024 and more; the sweep now takes 12.
 __global__ __launch_bounds__(256) void k_init_speed(GridDesc d, int p) {
-    double m = 0.0;
-    const long long n = (long long)d.nx * d.ny;
-    for (long long k = blockIdx.x * 256ll + threadIdx.x; k < n; k += (long long)gridDim.x * 256) {
-        const int j = (int)(k / d.nx), i = (int)(k % d.nx);
-        const long long o = (long long)j * d.pitch + i;
-        m = dmax(m, cfl_speed(d.g, d.dx, d.dy, d.ah[o], d.ahu[o], d.ahv[o]));
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & (WAVE - 1)) == 0 && m > 0.0)
-        atomicMax(&d.ctrl[p].speed_bits, (unsigned long long)__double_as_longlong(m));
+    const double m = plane_speed(d, [&](long long o, double& h, double& hu, double& hv) {
+        h = d.ah[o]; hu = d.ahu[o]; hv = d.ahv[o];
+    });
+    if (threadIdx.x == 0 && m > 0.0) speed_add(d.ctrl[p], blockIdx.x, m);
 }
+
+// Workgroups of a sweep over all cells: 1024 (four per CU) cover the chip.
+inline int sweep_blocks(long long cells) { return (int)((cells + 255) / 256 < 1024 ? (cells + 255) / 256 : 1024); }
 
 // Mass partials: block b sums rows b, b + gridDim.x, ... in a fixed order
 // (compute_total_mass, rki_init.F90:287-317).

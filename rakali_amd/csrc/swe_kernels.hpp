@@ -19,16 +19,26 @@ constexpr int WAVE = 64;        // wavefront width on CDNA
 constexpr int MAX_TC = 10;      // MAX_TIDAL_CONSTITUENTS
 // Time-control slot.  Two slots ping-pong: a step reads slot p (state at
 // the start of the step) and its stage-1 kernel writes slot 1-p.
-struct alignas(64) CtrlSlot {
+struct CtrlClock {
     double t;                     // time at the start of the step
     double dt;                    // dt of the step that produced this slot
-    unsigned long long speed_bits;// max CFL speed of the state (as bits)
     long long step_count;         // state%step_count
     double mass_out;              // boundary mass budget (rki_solver.F90:507-537)
     int active;                   // 1 if the step that wrote this slot ran
     int pad;
     double mass_src;              // surface mass source (accumulate_mass_src, rki_solver.F90:539-606)
     double t_bc;                  // bc%time of the step's last boundary call
+};
+
+// The clock and the max CFL speed of its state, as the bits of positive
+// doubles.  Atomics on one address complete one after the other, 12 ns apart
+// (16384 of them take 190 us): the tiles of a launch spread theirs over
+// SPEED_WAYS cache lines, and a reader takes the maximum of the ways.
+constexpr int SPEED_WAYS = 16;
+constexpr int SPEED_STRIDE = 16;  // 128 bytes
+
+struct alignas(128) CtrlSlot : CtrlClock {
+    alignas(128) unsigned long long speed[SPEED_WAYS * SPEED_STRIDE];
 };
 
 // Optional source terms of the stage kernels (template bit mask).
