@@ -158,19 +158,23 @@ inline double* field_ptr(rkg_grid* g, int field) {
 }
 
 // Rows per stage tile; tiles(rows) counts a launch's tiles.  A tile costs half
-// a row more than its rows (the march starts a row early), and a launch of few
-// tiles lasts as long as one tile, so it takes the shortest tiles that leave
-// one wavefront on each of the 1024 SIMDs while they have at most 8 rows, then
-// two while at most 10.  Larger launches run several tiles per wavefront slot:
-// 10 rows, and 20 once there are 8192 tiles of 16, where the uneven end of a
-// launch no longer matters.  Measured (us per step, one grid / each of three grids on
+// a row more than its rows (the march starts a row early), and a launch whose
+// tiles are all resident lasts as long as one tile.  So a launch takes the
+// shortest tiles, up to 3 rows, that still fit the chip's 3072 wavefront slots
+// at once; else the shortest, up to 10, that leave two wavefronts on each of
+// the 1024 SIMDs, which is enough to keep them busy and costs grids that run
+// beside others less.  Larger launches run several tiles per slot: 10 rows,
+// and 20 once there are 8192 tiles of 16, where the uneven end of a launch no
+// longer matters.  Measured (us per step, one grid / each of three grids on
 // their own streams):
-//   200x100    1 row  30 / 11,   8 rows  62 / 24
-//   512x512    5 rows 56 / 25,   8 rows  66 / 29
-//   701x515    7 rows 67 / 29,   3 rows  63 / 33,  16 rows 108 / 46
-//   1024x1024  10 rows 114 / 57, 6 rows 110 / 68,  19 rows 145 / 66
-//   3000x2000  10 rows 386 / 331, 16 rows 416 / 326
-//   4096x4096  20 rows 950 / 880, 10 rows 967 / 916, 32 rows 978 / 870
+//   200x100    1 row  29 / 11,   3 rows  35 / 14,   6 rows 51 / 19
+//   400x300    1 row  33 / 15,   3 rows  37 / 16,   6 rows 52 / 22
+//   512x512    2 rows 42 / 22,   1 row   50 / 30,   5 rows 48 / 24
+//   701x515    3 rows 47 / 29,   7 rows  60 / 29,  10 rows 76 / 34
+//   800x800    6 rows 72 / 41,   3 rows  73 / 46,  10 rows 90 / 43
+//   1024x1024  10 rows 103 / 60, 5 rows 101 / 65,  19 rows 129 / 69
+//   3000x2000  10 rows 380 / 345, 16 rows 403 / 339
+//   4096x4096  20 rows 976 / 924, 10 rows 1004 / 960, 32 rows 998 / 912
 // and for ensembles (their tiles have 4 rows at least):
 //   4 of 64..200      4 rows 45, 8 rows 65, 32 rows 192
 //   12 of 200..400    10 rows 108, 4 rows 117, 32 rows 204
@@ -178,9 +182,10 @@ inline double* field_ptr(rkg_grid* g, int field) {
 //   32 of 512..1024   20 rows 1207, 10 rows 1301, 32 rows 1208
 template <class TILES>
 int rows_for(TILES tiles, int least) {
-    for (int waves = 1; waves <= 2; ++waves)
-        for (int rows = least; rows <= (waves == 1 ? 8 : 10); ++rows)
-            if (tiles(rows) <= 1024 * waves) return rows;
+    for (int rows = least; rows <= 3; ++rows)
+        if (tiles(rows) <= 3 * 1024) return rows;
+    for (int rows = least; rows <= 10; ++rows)
+        if (tiles(rows) <= 2 * 1024) return rows;
     return tiles(16) >= 8192 ? 20 : 10;
 }
 
