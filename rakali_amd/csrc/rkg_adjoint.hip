@@ -60,7 +60,6 @@ struct AdjStage {
     double* edge_lg;            // adjoint (h, normal momentum) of every tidal ghost cell, see edge_slot
     int edge_len;               // max(nx, ny)
     int ty;                     // rows per tile of k_adj_y
-    int xrows;                  // rows per workgroup of k_adj_x
 };
 
 // Slot of ghost layer kk (0 = next to the edge) at position p along edge e
@@ -190,32 +189,54 @@ __device__ __forceinline__ adj::C4 sh_from(const adj::C4& c, int src) {
     return adj::C4{__shfl(c.h, src, WAVE), __shfl(c.hu, src, WAVE), __shfl(c.hv, src, WAVE), __shfl(c.b, src, WAVE)};
 }
 
-__device__ __forceinline__ adj::S3 load_ldiv(const AdjStage& a, int x, int y) {
+// The planes a row of a face reverse needs, in the order of the LDS rows: the
+// stage input (h, hu, hv, b), the adjoint of the flux divergence, and what the
+// row adds to, the adjoint of the input and the bed gradient.
+constexpr int ADJ_PLANES = 11;
+
+__device__ __forceinline__ const double* adj_plane(const AdjStage& a, int p) {
     const GridDesc& d = a.d;
-    if ((unsigned)x >= (unsigned)d.nx || (unsigned)y >= (unsigned)d.ny) return adj::S3{0.0, 0.0, 0.0};
-    const long long k = (long long)y * d.pitch + x;
-    return adj::S3{a.lam_div[k], a.lam_div[d.plane + k], a.lam_div[2 * d.plane + k]};
+    if (p < 3) return d.ah + p * d.plane;   // ah, ahu, ahv follow each other
+    if (p == 3) return d.bed;
+    if (p < 7) return a.lam_div + (p - 4) * d.plane;
+    if (p < 10) return a.lam_in + (p - 7) * d.plane;
+    return a.grad_b;
 }
 
-__device__ __forceinline__ Cell vload(const GridDesc& d, int x, int y, double eta) {
-    return load_cell(d, d.ah, d.ahu, d.ahv, x, y, eta);
+// 16 bytes per lane from memory into 64 x 16 bytes of LDS, without registers.
+__device__ __forceinline__ void to_lds(const double* src, double* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// Waits for every load of the wavefront before what follows (the stores of a
+// row, which share the loads' in-order counter: a row's loads must not be
+// waited for behind the stores of the row before).
+__device__ __forceinline__ void wait_loads() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// A ghost cell of side `side` from its source cell (see lane_source).
+__device__ __forceinline__ Cell side_ghost(const GridDesc& d, int side, double eta, const Cell& src) {
+    return ghost_from(d, d.bc[side], eta, src, src, (side & 1) ? 1.0 : -1.0, side < 2);
 }
 
 // Adjoint of the row-y ghost at column x onto interior cells (x-direction
-// ghosts: normal momentum hu).  Returns the contributions for the mirror
-// and first-interior columns.
-__device__ __forceinline__ void ghost_x_rev(const GridDesc& d, double eta, int x, int y, const adj::C4& lg, int& mcol,
+// ghosts: normal momentum hu); cell(col) gives the row's interior cells.
+// Returns the contributions for the mirror and first-interior columns.
+template <class CELL>
+__device__ __forceinline__ void ghost_x_rev(const GridDesc& d, double eta, int x, CELL cell, const adj::C4& lg, int& mcol,
                                             int& icol, adj::C4& lm, adj::C4& li) {
     const bool west = x < 0;
     const int kk = west ? (-x - 1) : (x - d.nx);
     mcol = west ? kk : (d.nx - 1 - kk);
     icol = west ? 0 : (d.nx - 1);
-    const Cell mir = load_direct(d.ah, d.ahu, d.ahv, d.bed, d.pitch, mcol, y);
-    const Cell in0 = load_direct(d.ah, d.ahu, d.ahv, d.bed, d.pitch, icol, y);
     lm = adj::C4{0, 0, 0, 0};
     li = adj::C4{0, 0, 0, 0};
-    adj::ghost_rev(d.bc[west ? 0 : 1], d.g, eta, d.inflow_velocity, d.clamped_elevation, mir, in0, west ? -1.0 : 1.0,
-                   true, lg, lm, li);
+    adj::ghost_rev(d.bc[west ? 0 : 1], d.g, eta, d.inflow_velocity, d.clamped_elevation, cell(mcol), cell(icol),
+                   west ? -1.0 : 1.0, true, lg, lm, li);
 }
 
 __device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, int x, int y, const adj::C4& lg, int& mrow,
@@ -232,173 +253,296 @@ __device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, int x
                    south ? -1.0 : 1.0, false, lg, lm, li);
 }
 
-constexpr int NWIN = 6;   // accumulator rows r-3 .. r+2
+// Two LDS rows of the 11 planes over 64 columns (the twelfth is a spare: two
+// planes make one load), and two accumulators that wait for their ghost rows:
+// the south ghost rows', then row ny-2's with its old values.
+struct YRows {
+    double v[2][ADJ_PLANES + 1][WAVE];
+    double kept[8][WAVE];
+};
 
 // Reverse of the y faces and y slopes of one stage (and the south / north
 // ghost rows) onto the stage input and the bed.  One wavefront per tile of
 // 64 whole columns (lane l holds column c0 + l; this direction is
 // column-local, so no halo columns) and rows [j0, j1).  The rows are
 // marched from j0 - 2 to j1: iteration r reverses the y face between rows
-// r and r+1 and the y slope of row r.  Row r-1 is complete after iteration
-// r; rows are written two iterations later so that ghost rows can still be
-// folded into their source rows.  TY: a south or north edge is tidal, and
-// the adjoints of its ghost cells are kept in edge_lg for k_dt_rev.
+// r and r+1 and the y slope of row r, which completes row r-1.  A ghost row's
+// adjoint is added to its source rows when row 0 is complete (south), or with
+// the last row (north, row ny-2 waiting for it).  TY: a south or north edge is
+// tidal, and the adjoints of its ghost cells are kept in edge_lg for k_dt_rev.
+//
+// Bound by latency with two wavefronts on a SIMD (face_rev's live values leave
+// no room for a third): what iteration r + 1 needs is loaded into LDS during
+// iteration r, so that a row waits for no memory.  1024^2:
+// 57 us when each row loaded its own, 48 now, of which its 126 MB take 27.
 template <bool HLLC, int STAGE, bool TY>
-__device__ __forceinline__ void adj_y(const AdjStage& a, int blk) {
+__device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
     const GridDesc& d = a.d;
-    const double tau = STAGE == 1 ? a.hist[0] : a.hist[0] + a.hist[1];   // bc%time of the stage
     const int lane = threadIdx.x;
     const int nstr = (d.nx + WAVE - 1) / WAVE;
     const int sx = blk % nstr, sy = blk / nstr;
     const int c0 = sx * WAVE;
     int j0, j1;
     tile_range(d.ny, a.ty, sy, j0, j1);
-    const bool xin = c0 + lane < d.nx;
-    const int x = xin ? c0 + lane : d.nx - 1;   // lanes past the edge repeat the last column, unwritten
-    // rows j0 - 3 .. j1 + 2 are read; only ghost rows need the tide (whose
-    // correctly rounded sine is a long dependent chain)
-    const double eta = (j0 < 3 || j1 + 2 >= d.ny) ? tidal_eta(d, tau) : 0.0;
+    const int x = c0 + lane;
+    const bool xin = x < d.nx;   // lanes past the edge compute on the rows' padding, unwritten
+    const int xs = xin ? x : d.nx - 1;
+    const bool south = j0 < 3, north = j1 + 2 >= d.ny;
+    const int ny = d.ny;
+    const long long P = d.plane;
+
+    // lane l loads columns 2 (l % 32) and the next of planes 2 i and 2 i + 1
+    const int col = min(c0 + 2 * (lane & 31), (int)d.pitch - 2);
+    const double* src[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) src[i] = adj_plane(a, min(2 * i + (lane >> 5), ADJ_PLANES - 1)) + col;
+    // the source row of row j (lane_source's rule for rows)
+    auto source_row = [&](int j) {
+        if (j < 0) return min(mirrors(d.bc[2]) ? -j - 1 : 0, ny - 1);
+        if (j >= ny) return max(mirrors(d.bc[3]) ? 2 * ny - 1 - j : ny - 1, 0);
+        return j;
+    };
+    auto fetch = [&](int r, int buf) {   // what iteration r needs
+        const long long ov = source_row(r + 2) * d.pitch, od = min(max(r + 1, 0), ny - 1) * d.pitch,
+                        ol = min(max(r - 1, 0), ny - 1) * d.pitch;
+        const long long o67 = lane < WAVE / 2 ? od : ol;
+        to_lds(src[0] + ov, rows.v[buf][0]);
+        to_lds(src[1] + ov, rows.v[buf][2]);
+        to_lds(src[2] + od, rows.v[buf][4]);
+        to_lds(src[3] + o67, rows.v[buf][6]);
+        to_lds(src[4] + ol, rows.v[buf][8]);
+        to_lds(src[5] + ol, rows.v[buf][10]);
+    };
+    const int rs = j0 - 2, re = j1;
+    const long long q0 = source_row(rs - 1) * d.pitch + xs, q1 = source_row(rs) * d.pitch + xs,
+                    q2 = source_row(rs + 1) * d.pitch + xs;
+    Cell v0{d.ah[q0], d.ahu[q0], d.ahv[q0], d.bed[q0]}, v1{d.ah[q1], d.ahu[q1], d.ahv[q1], d.bed[q1]},
+        v2{d.ah[q2], d.ahu[q2], d.ahv[q2], d.bed[q2]}, v3;
+    adj::S3 ld_r{0.0, 0.0, 0.0};
+    if (rs >= 0) {
+        const long long o = rs * d.pitch + xs;
+        ld_r = adj::S3{a.lam_div[o], a.lam_div[P + o], a.lam_div[2 * P + o]};
+    }
+    fetch(rs, 0);
+    const double tau = STAGE == 1 ? a.hist[0] : a.hist[0] + a.hist[1];   // bc%time of the stage
+    // the tide (a long dependent chain) only where a tidal edge's ghosts are read
+    const bool tidal = (south && d.bc[2] == BC_TIDAL) || (north && d.bc[3] == BC_TIDAL);
+    const double eta = tidal ? tidal_eta(d, tau) : 0.0;
+    auto row_ghost = [&](int j, const Cell& c) {
+        if (j >= 0 && j < ny) return c;
+        if (j < -2 || j > ny + 1) return Cell{0.0, 0.0, 0.0, 0.0};
+        return side_ghost(d, j < 0 ? 2 : 3, eta, c);
+    };
+    if (south || north) {
+        v0 = row_ghost(rs - 1, v0);
+        v1 = row_ghost(rs, v1);
+        v2 = row_ghost(rs + 1, v2);
+    }
     const double g = d.g;
     const bool fast = g >= 1.0e-3 && g <= 1.0e6;   // face_rev_fast's ranges assume an ordinary gravity
     const double rdy = 1.0 / d.dy;
-    const long long P = d.plane;
 
-    Acc acc[NWIN];
+    Acc acc[3];   // rows r-1, r, r+1
 #pragma unroll
-    for (int q = 0; q < NWIN; ++q) acc[q] = Acc{0.0, 0.0, 0.0, 0.0};
-    const int rs = j0 - 2, re = j1;
-    Cell v0 = vload(d, x, rs - 1, eta), v1 = vload(d, x, rs, eta), v2 = vload(d, x, rs + 1, eta), v3;
+    for (int q = 0; q < 3; ++q) acc[q] = Acc{0.0, 0.0, 0.0, 0.0};
     FState hi_r, lo_tmp;
     adj::states_fwd(v0, v1, v2, lo_tmp, hi_r);
     adj::S3 llo_r{0.0, 0.0, 0.0};        // adjoint of the y lo-state of row r (from face r - 1/2)
-    adj::S3 ld_r = load_ldiv(a, x, rs);
 
-    // Folds the completed row `rho` (window slot `q`): a ghost row onto its
-    // source rows, an owned row into the adjoint arrays.
-    auto flush = [&](int rho, int q, int r) {
-        if (rho < -2 || rho > d.ny + 1) return;
-        const adj::C4 lg = c4(acc[q]);
-        if (rho < 0 || rho >= d.ny) {
-            int mrow, irow;
-            adj::C4 lm, li;
-            ghost_y_rev(d, eta, x, rho, lg, mrow, irow, lm, li);
-            // source rows are in the window: slot of row t is t - (r - 3)
-            const int qm = mrow - (r - 3), qi = irow - (r - 3);
-#pragma unroll
-            for (int s = 0; s < NWIN; ++s) {
-                if (s == qm) add(acc[s], lm);
-                if (s == qi) add(acc[s], li);
-            }
-            // a tidal ghost row cell is kept once, by the tile holding the edge
-            // row (a tile next to a short last tile also reaches the ghost
-            // rows, with partial sums)
-            const int e = rho < 0 ? 2 : 3;
-            if (TY && xin && (rho < 0 ? j0 == 0 : j1 == d.ny) && d.bc[e] == BC_TIDAL) {
-                const long long o = edge_slot(e, rho < 0 ? -rho - 1 : rho - d.ny, x, a.edge_len);
-                a.edge_lg[o] = lg.h;
-                a.edge_lg[o + 1] = lg.hv;
-            }
-            return;
-        }
-        if (xin && rho >= j0 && rho < j1) {
-            const long long k = (long long)rho * d.pitch + x;
-            a.lam_in[k] += lg.h;
-            a.lam_in[P + k] += lg.hu;
-            a.lam_in[2 * P + k] += lg.hv;
-            a.grad_b[k] += lg.b;
+    // Adjoint lg of ghost row rho onto rows mrow and irow.
+    auto fold = [&](int rho, const Acc& ghost, int& mrow, int& irow, adj::C4& lm, adj::C4& li) {
+        const adj::C4 lg = c4(ghost);
+        ghost_y_rev(d, eta, xs, rho, lg, mrow, irow, lm, li);
+        const int e = rho < 0 ? 2 : 3;
+        if (TY && xin && d.bc[e] == BC_TIDAL) {
+            const long long o = edge_slot(e, rho < 0 ? -rho - 1 : rho - ny, x, a.edge_len);
+            a.edge_lg[o] = lg.h;
+            a.edge_lg[o + 1] = lg.hv;
         }
     };
 
     for (int r = rs; r <= re; ++r) {
-        // window: acc[q] is row r - 3 + q; v0..v3 rows r-1 .. r+2
-        v3 = vload(d, x, r + 2, eta);
-        const adj::S3 ld_r1 = load_ldiv(a, x, r + 1);
+        // v0..v2 are rows r-1 .. r+1
+        const double(*in)[WAVE] = rows.v[(r - rs) & 1];
+        v3 = Cell{in[0][lane], in[1][lane], in[2][lane], in[3][lane]};
+        adj::S3 ld_r1{in[4][lane], in[5][lane], in[6][lane]};
+        const adj::C4 old{in[7][lane], in[8][lane], in[9][lane], in[10][lane]};   // row r-1
+        if (r < re) fetch(r + 1, (r + 1 - rs) & 1);
+        if (south || north) {
+            v3 = row_ghost(r + 2, v3);
+            if (r + 1 < 0 || r + 1 >= ny) ld_r1 = adj::S3{0.0, 0.0, 0.0};
+        }
         FState lo_r1, hi_r1;
         adj::states_fwd(v1, v2, v3, lo_r1, hi_r1);
         // y face r + 1/2 (faces -1/2 .. ny - 1/2)
         adj::S3 lhi_r{0.0, 0.0, 0.0}, llo_r1{0.0, 0.0, 0.0};
-        if (r >= -1 && r <= d.ny - 1) {
+        if (r >= -1 && r <= ny - 1) {
             const Face lf = adj::face_seed<true>(g, rdy, ld_r, ld_r1);
             double lbL = 0.0, lbR = 0.0;
             if (!(fast && adj::face_rev_fast<HLLC, true>(g, hi_r, v1.b, lo_r1, v2.b, lf, lhi_r, lbL, llo_r1, lbR,
                                                           xin)))
                 adj::face_rev<HLLC, true>(g, hi_r, v1.b, lo_r1, v2.b, lf, lhi_r, lbL, llo_r1, lbR);
-            acc[3].b += lbL;
-            acc[4].b += lbR;
+            acc[1].b += lbL;
+            acc[2].b += lbR;
         }
         // y slope of row r
         {
             adj::C4 lm{0, 0, 0, 0}, lc{0, 0, 0, 0}, lp{0, 0, 0, 0};
             adj::states_rev(v0, v1, v2, llo_r, lhi_r, lm, lc, lp);
-            add(acc[2], lm);
-            add(acc[3], lc);
-            add(acc[4], lp);
+            add(acc[0], lm);
+            add(acc[1], lc);
+            add(acc[2], lp);
         }
-        // row r - 3 is complete and past the ghost folding window
-        flush(r - 3, 0, r);
-#pragma unroll
-        for (int q = 0; q < NWIN - 1; ++q) acc[q] = acc[q + 1];
-        acc[NWIN - 1] = Acc{0.0, 0.0, 0.0, 0.0};
+        auto keep = [&](int q, double h, double hu, double hv, double lb) {
+            rows.kept[q][lane] = h; rows.kept[q + 1][lane] = hu; rows.kept[q + 2][lane] = hv; rows.kept[q + 3][lane] = lb;
+        };
+        auto kept = [&](int q) {
+            return Acc{rows.kept[q][lane], rows.kept[q + 1][lane], rows.kept[q + 2][lane], rows.kept[q + 3][lane]};
+        };
+        adj::C4 lm, li;
+        int mrow, irow;
+        if (j0 == 0 && r <= 1) {
+            if (r == -1 || r == 0) {   // row -2, -1 complete
+                keep(4 * (r + 1), acc[0].h, acc[0].hu, acc[0].hv, acc[0].b);
+            } else if (r == 1) {       // acc[0], acc[1] are rows 0 and 1
+                fold(-2, kept(0), mrow, irow, lm, li);
+                add(acc[1], lm);       // the mirror row is 1, the first row 0
+                add(acc[0], li);
+                fold(-1, kept(4), mrow, irow, lm, li);
+                add(acc[0], lm);
+                add(acc[0], li);
+            }
+        }
+        const int rho = r - 1;
+        auto put = [&](int row, const adj::C4& from, const Acc& more) {
+            const long long k = row * d.pitch + x;
+            a.lam_in[k] = from.h + more.h;
+            a.lam_in[P + k] = from.hu + more.hu;
+            a.lam_in[2 * P + k] = from.hv + more.hv;
+            a.grad_b[k] = from.b + more.b;
+        };
+        const bool waits = j1 == ny && rho == ny - 2 && rho >= j0;
+        if (waits) {
+            keep(0, old.h, old.hu, old.hv, old.b);
+            keep(4, acc[0].h, acc[0].hu, acc[0].hv, acc[0].b);
+        }
+        if (j1 == ny && r == ny) {   // acc[0..2] are rows ny-1, ny, ny+1
+            Acc last = kept(4);      // row ny-2
+            fold(ny, acc[1], mrow, irow, lm, li);
+            add(acc[0], lm);
+            add(acc[0], li);
+            fold(ny + 1, acc[2], mrow, irow, lm, li);
+            add(last, lm);
+            add(acc[0], li);
+            if (xin) put(ny - 2, c4(kept(0)), last);
+        }
+        wait_loads();
+        if (xin && rho >= j0 && rho < j1 && !waits) put(rho, old, acc[0]);
+        acc[0] = acc[1];
+        acc[1] = acc[2];
+        acc[2] = Acc{0.0, 0.0, 0.0, 0.0};
         v0 = v1; v1 = v2; v2 = v3;
         hi_r = hi_r1;
         llo_r = llo_r1;
         ld_r = ld_r1;
     }
-    // remaining rows re-2 .. re+2 in slots 0..4 (window base re + 1 - 3):
-    // ghost rows first (their sources are among the owned rows), then the rest
-    const int base = re + 1 - 3;
-    for (int q = 0; q < NWIN; ++q) {
-        const int rho = base + q;
-        if (rho >= d.ny) flush(rho, q, re + 1);
-    }
-    for (int q = 0; q < NWIN; ++q) {
-        const int rho = base + q;
-        if (rho < d.ny) flush(rho, q, re + 1);
-    }
 }
 
 template <bool HLLC, int STAGE, bool TY>
 __global__ __launch_bounds__(WAVE) void k_adj_y(AdjStage a) {
-    adj_y<HLLC, STAGE, TY>(a, blockIdx.x);
+    __shared__ alignas(16) YRows rows;
+    adj_y<HLLC, STAGE, TY>(a, rows, blockIdx.x);
 }
+
+// Two LDS rows of the 11 planes over 68 columns, 34 pairs each: the 374 pairs
+// of a row are loaded 64 at a time.
+// Rows per workgroup of k_adj_x: with the loads a row ahead a workgroup costs
+// little to start, and many short ones even out the edge strips (us: 1024^2
+// 4 rows 54, 2 rows 53, 9 rows 58; 4096 x 1024 4 rows 144, 32 rows 206).
+constexpr int XROWS = 4;
+constexpr int XCOLS = 68;
+constexpr int XLOADS = (ADJ_PLANES * XCOLS / 2 + WAVE - 1) / WAVE;
+struct XRows {
+    double v[2][XLOADS * WAVE * 2];
+};
 
 // Reverse of the x faces and x slopes of one stage (and the west / east
 // ghost columns) onto the stage input and the bed.  This direction is
 // row-local: every row is independent.  One wavefront per strip of at
-// most 60 owned columns [c0, c1) and `xrows` rows; lane l holds column
+// most 60 owned columns [c0, c1) and XROWS rows; lane l holds column
 // c0 - 2 + l, so the faces and slopes that touch an owned cell are all in
-// the wavefront.  The face right of a cell is reversed by the cell's lane;
-// neighbours' parts move by lane shuffles; ghost columns fold onto their
-// source columns by lane permutes.  TX: a west or east edge is tidal (see
-// k_adj_y's TY).
+// the wavefront (lanes 0 and 63 need one column more).  The face right of a
+// cell is reversed by the cell's lane; neighbours' parts move by lane
+// shuffles; ghost columns fold onto their source columns by lane permutes.
+// TX: a west or east edge is tidal (see k_adj_y's TY).
+//
+// Bound by latency, as adj_y: the next row is loaded into LDS while a row is
+// computed.  1024^2: 78 us when each row loaded its own, 54 now,
+// of which its 138 MB take 30; 4096 x 1024: 144 us, at 3.8 TB/s.
 template <bool HLLC, int STAGE, bool TX>
-__device__ __forceinline__ void adj_x(const AdjStage& a, int blk) {
+__device__ __forceinline__ void adj_x(const AdjStage& a, XRows& rows, int blk) {
     const GridDesc& d = a.d;
-    const double tau = STAGE == 1 ? a.hist[0] : a.hist[0] + a.hist[1];
     const int lane = threadIdx.x;
     const int nstr = (d.nx + AW - 1) / AW;
     const int sx = blk % nstr, sy = blk / nstr;
     int c0, c1;
     tile_range(d.nx, AW, sx, c0, c1);
-    const int r0 = sy * a.xrows, r1 = min(r0 + a.xrows, d.ny);
+    const int r0 = sy * XROWS, r1 = min(r0 + XROWS, d.ny);
     const int x = c0 - 2 + lane;
     const bool own_col = x >= c0 && x < c1;
-    const bool edge_tile = c0 - 2 < 0 || c0 + WAVE - 3 >= d.nx;
-    // columns c0 - 3 .. c0 + 62 are read (lanes 0 and 63 load one more);
-    // only ghost columns need the tide
-    const double eta = (c0 < 3 || c0 + 62 >= d.nx) ? tidal_eta(d, tau) : 0.0;
+    // columns c0 - 3 .. c0 + 62 are read
+    const bool edge_tile = c0 < 3 || c0 + 62 >= d.nx;
+    const long long P = d.plane;
+    // The LDS rows start at the even column cb; pairs outside the rows are
+    // read from their ends and not used.
+    const int cb = (c0 - 3) & ~1;
+    const double* src[XLOADS];
+#pragma unroll
+    for (int i = 0; i < XLOADS; ++i) {
+        const int q = i * WAVE + lane;
+        const int p = min(q / (XCOLS / 2), ADJ_PLANES - 1);
+        const int col = cb + 2 * (q % (XCOLS / 2));
+        src[i] = adj_plane(a, p) + min(max(col, 0), (int)d.pitch - 2);
+    }
+    auto fetch = [&](int r, int buf) {
+        const long long o = r * d.pitch;
+#pragma unroll
+        for (int i = 0; i < XLOADS; ++i) to_lds(src[i] + o, rows.v[buf] + i * WAVE * 2);
+    };
+    if (r0 < r1) fetch(r0, 0);
+    const double tau = STAGE == 1 ? a.hist[0] : a.hist[0] + a.hist[1];
+    // the tide only where a tidal edge's ghosts are read
+    const bool tidal = (c0 < 3 && d.bc[0] == BC_TIDAL) || (c0 + 62 >= d.nx && d.bc[1] == BC_TIDAL);
+    const double eta = tidal ? tidal_eta(d, tau) : 0.0;
     const double g = d.g;
     const bool fast = g >= 1.0e-3 && g <= 1.0e6;
     const double rdx = 1.0 / d.dx;
-    const long long P = d.plane;
+    const LaneSource l1 = edge_tile ? lane_source<true>(d, x) : lane_source<false>(d, x);
+    const LaneSource l2 = edge_tile ? lane_source<true>(d, lane == 0 ? x - 1 : x + 1) : l1;
+    const int i1 = min(max(l1.c - cb, 0), XCOLS - 1), i2 = min(max(l2.c - cb, 0), XCOLS - 1);
     for (int r = r0; r < r1; ++r) {
-        const Cell v1 = vload(d, x, r, eta);
-        const adj::S3 ld_r = load_ldiv(a, x, r);
-        Cell xm, xp;
-        xm.h = sh_up(v1.h); xm.hu = sh_up(v1.hu); xm.hv = sh_up(v1.hv); xm.b = sh_up(v1.b);
-        xp.h = sh_dn(v1.h); xp.hu = sh_dn(v1.hu); xp.hv = sh_dn(v1.hv); xp.b = sh_dn(v1.b);
-        if (lane == 0) xm = vload(d, x - 1, r, eta);
-        if (lane == WAVE - 1) xp = vload(d, x + 1, r, eta);
+        const double* row = rows.v[(r - r0) & 1];
+        auto cell_at = [&](int i) { return Cell{row[i], row[XCOLS + i], row[2 * XCOLS + i], row[3 * XCOLS + i]}; };
+        Cell v1 = cell_at(i1), xm, xp;
+        adj::S3 ld_r{row[4 * XCOLS + i1], row[5 * XCOLS + i1], row[6 * XCOLS + i1]};
+        const adj::C4 old{row[7 * XCOLS + i1], row[8 * XCOLS + i1], row[9 * XCOLS + i1], row[10 * XCOLS + i1]};
+        if (!edge_tile) {
+            xm = cell_at(i1 - 1);
+            xp = cell_at(i1 + 1);
+        } else {
+            Cell out = cell_at(i2);
+            const Cell zero{0.0, 0.0, 0.0, 0.0};
+            if (l1.side != -1) {
+                v1 = l1.side < 0 ? zero : side_ghost(d, l1.side, eta, v1);
+                ld_r = adj::S3{0.0, 0.0, 0.0};
+            }
+            if (l2.side != -1) out = l2.side < 0 ? zero : side_ghost(d, l2.side, eta, out);
+            xm.h = sh_up(v1.h); xm.hu = sh_up(v1.hu); xm.hv = sh_up(v1.hv); xm.b = sh_up(v1.b);
+            xp.h = sh_dn(v1.h); xp.hu = sh_dn(v1.hu); xp.hv = sh_dn(v1.hv); xp.b = sh_dn(v1.b);
+            if (lane == 0) xm = out;
+            if (lane == WAVE - 1) xp = out;
+        }
+        if (r + 1 < r1) fetch(r + 1, (r + 1 - r0) & 1);
         FState lo_x, hi_x;
         adj::states_fwd(xm, v1, xp, lo_x, hi_x);
         FState R;
@@ -427,7 +571,7 @@ __device__ __forceinline__ void adj_x(const AdjStage& a, int blk) {
             adj::C4 gm{0, 0, 0, 0}, gi{0, 0, 0, 0};
             int mcol = -100, icol = -100;
             if (x == -1 || x == -2 || x == d.nx || x == d.nx + 1) {
-                ghost_x_rev(d, eta, x, r, mine, mcol, icol, gm, gi);
+                ghost_x_rev(d, eta, x, [&](int c) { return cell_at(c - cb); }, mine, mcol, icol, gm, gi);
                 const int e = x < 0 ? 0 : 1;
                 // kept once, by the tile holding the edge column
                 if (TX && (x < 0 ? c0 == 0 : c1 == d.nx) && d.bc[e] == BC_TIDAL) {
@@ -448,19 +592,21 @@ __device__ __forceinline__ void adj_x(const AdjStage& a, int blk) {
                 if (x == ricol) { mine.h += ri.h; mine.hu += ri.hu; mine.hv += ri.hv; mine.b += ri.b; }
             }
         }
+        wait_loads();
         if (own_col) {
-            const long long k = (long long)r * d.pitch + x;
-            a.lam_in[k] += mine.h;
-            a.lam_in[P + k] += mine.hu;
-            a.lam_in[2 * P + k] += mine.hv;
-            a.grad_b[k] += mine.b;
+            const long long k = r * d.pitch + x;
+            a.lam_in[k] = old.h + mine.h;
+            a.lam_in[P + k] = old.hu + mine.hu;
+            a.lam_in[2 * P + k] = old.hv + mine.hv;
+            a.grad_b[k] = old.b + mine.b;
         }
     }
 }
 
 template <bool HLLC, int STAGE, bool TX>
 __global__ __launch_bounds__(WAVE) void k_adj_x(AdjStage a) {
-    adj_x<HLLC, STAGE, TX>(a, blockIdx.x);
+    __shared__ alignas(16) XRows rows;
+    adj_x<HLLC, STAGE, TX>(a, rows, blockIdx.x);
 }
 
 // d L / d eta_tidal from one tidal ghost cell (adjoints lg0 of h and lg1
@@ -793,15 +939,17 @@ __global__ __launch_bounds__(256) void k_adj_body_batch(const AdjStage* __restri
 template <bool HLLC, int STAGE>
 __global__ __launch_bounds__(WAVE) void k_adj_y_batch(const AdjStage* __restrict__ as,
                                                      const BlockRef* __restrict__ tab) {
+    __shared__ alignas(16) YRows rows;
     const BlockRef r = tab[blockIdx.x];
-    adj_y<HLLC, STAGE, true>(as[r.member], r.blk);
+    adj_y<HLLC, STAGE, true>(as[r.member], rows, r.blk);
 }
 
 template <bool HLLC, int STAGE>
 __global__ __launch_bounds__(WAVE) void k_adj_x_batch(const AdjStage* __restrict__ as,
                                                      const BlockRef* __restrict__ tab) {
+    __shared__ alignas(16) XRows rows;
     const BlockRef r = tab[blockIdx.x];
-    adj_x<HLLC, STAGE, true>(as[r.member], r.blk);
+    adj_x<HLLC, STAGE, true>(as[r.member], rows, r.blk);
 }
 
 __global__ __launch_bounds__(1024) void k_dt_rev_batch(const DtArgs* __restrict__ da) { dt_rev(da[blockIdx.x]); }
@@ -916,7 +1064,7 @@ void launch_faces(rkg_grid* g, const AdjStage& st) {
     const bool tx = bc[0] == BC_TIDAL || bc[1] == BC_TIDAL, ty = bc[2] == BC_TIDAL || bc[3] == BC_TIDAL;
     const int nx = g->cfg.nx, ny = g->cfg.ny;
     const int yblocks = ((nx + WAVE - 1) / WAVE) * ((ny + st.ty - 1) / st.ty);
-    const int xblocks = ((nx + AW - 1) / AW) * ((ny + st.xrows - 1) / st.xrows);
+    const int xblocks = ((nx + AW - 1) / AW) * ((ny + XROWS - 1) / XROWS);
     if (ty)
         hipLaunchKernelGGL((k_adj_y<HLLC, STAGE, true>), dim3(yblocks), dim3(WAVE), 0, g->stream, st);
     else
@@ -1218,7 +1366,7 @@ int fwd_finish(rkg_adjoint* a, double* loss) {
 
 // Per-sweep settings of one session.
 struct BwdPlan {
-    int tile_rows, xrows, nb, nargmax;
+    int tile_rows, nb, nargmax;
     bool cfl_dt;
     long long edge_size;
     double scale;
@@ -1228,16 +1376,13 @@ struct BwdPlan {
 int bwd_begin(rkg_adjoint* a, double loss_scale, int tile_rows, BwdPlan& pl) {
     if (!a->have_forward) { set_error("rkg_adjoint_backward before rkg_adjoint_forward"); return RKG_ERR_NOT_READY; }
     rkg_grid* g = a->g;
-    // rows per workgroup: about 2048 workgroups of k_adj_y and of k_adj_x
-    // (two waves on each of the 1024 SIMDs); on the 1024^2 basin 8 rows of
-    // k_adj_y (2048 workgroups) beat 9 (1821) by 1 %, and 9 rows of k_adj_x
-    // (2048) beat 10 (1844) by about 1 %
+    // rows per workgroup of k_adj_y: about 2048 workgroups, two waves on each
+    // of the 1024 SIMDs (1024^2 basin, us: 8 rows 48, 7 rows 57, 10 rows 56)
     const long long ny = g->cfg.ny;
-    const long long ystrips = (g->cfg.nx + WAVE - 1) / WAVE, xstrips = (g->cfg.nx + AW - 1) / AW;
+    const long long ystrips = (g->cfg.nx + WAVE - 1) / WAVE;
     if (tile_rows <= 0) tile_rows = (int)std::min<long long>(32, std::max<long long>(4, (ny * ystrips + 2047) / 2048));
     if (tile_rows < 4 || tile_rows > 256) { set_error("tile_rows must lie in [4, 256]"); return RKG_ERR_RANGE; }
     pl.tile_rows = tile_rows;
-    pl.xrows = (int)std::min<long long>(32, std::max<long long>(1, (ny * xstrips + 2047) / 2048));
     pl.nb = body_blocks(g);
     pl.cfl_dt = g->cfg.dt_fixed <= 0.0;
     pl.nargmax = pl.cfl_dt ? pl.nb : 0;   // argmax partials, one per body workgroup of stage 1
@@ -1352,7 +1497,6 @@ AdjStage stage_args(rkg_adjoint* a, int k, int stage, const BwdPlan& pl) {
     st.hist = a->hist + HIST * k;
     st.edge_len = a->edge_len;
     st.ty = pl.tile_rows;
-    st.xrows = pl.xrows;
     if (stage == 2) {   // input U* (B_k), U^n = A_k
         st.d = stage_desc(a, wsB(a, k), wsB(a, k), wsA(a, k + 1));
         st.un = wsA(a, k);
@@ -1493,7 +1637,7 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
         for (int b = 0; b < nb; ++b) tb.push_back(BlockRef{m, b, nb, 0});
         const int yb = ((nx + WAVE - 1) / WAVE) * ((ny + pl[m].tile_rows - 1) / pl[m].tile_rows);
         for (int b = 0; b < yb; ++b) ty.push_back(BlockRef{m, b, yb, 0});
-        const int xb = ((nx + AW - 1) / AW) * ((ny + pl[m].xrows - 1) / pl[m].xrows);
+        const int xb = ((nx + AW - 1) / AW) * ((ny + XROWS - 1) / XROWS);
         for (int b = 0; b < xb; ++b) tx.push_back(BlockRef{m, b, xb, 0});
         if (as[m]->ng > 0) {
             const int sb = (as[m]->ncells + 255) / 256;

@@ -164,38 +164,6 @@ __host__ __device__ __forceinline__ Cell ghost_from(const GridDesc& d, int tag, 
     }
 }
 
-// Cell (c, j) of the state (h, hu, hv) with bed d.bed, synthesizing the
-// two ghost layers around the domain.  Corner cells and cells beyond the
-// second ghost layer are never read by the stencil; they return zeros.
-__device__ __forceinline__ Cell load_cell(const GridDesc& d, const double* __restrict__ h,
-                                          const double* __restrict__ hu, const double* __restrict__ hv,
-                                          int c, int j, double eta_tidal) {
-    const bool xin = (unsigned)c < (unsigned)d.nx;
-    const bool yin = (unsigned)j < (unsigned)d.ny;
-    if (xin && yin) return load_direct(h, hu, hv, d.bed, d.pitch, c, j);
-    Cell z; z.h = 0.0; z.hu = 0.0; z.hv = 0.0; z.b = 0.0;
-    if (!xin && !yin) return z;
-    if (!xin) {
-        const bool west = c < 0;
-        const int kk = west ? (-c - 1) : (c - d.nx);
-        if (kk > 1) return z;
-        const int mc = west ? kk : (d.nx - 1 - kk);
-        const int ic = west ? 0 : (d.nx - 1);
-        const Cell mir = load_direct(h, hu, hv, d.bed, d.pitch, mc, j);
-        const Cell in0 = load_direct(h, hu, hv, d.bed, d.pitch, ic, j);
-        return ghost_from(d, d.bc[west ? 0 : 1], eta_tidal, mir, in0, west ? -1.0 : 1.0, true);
-    } else {
-        const bool south = j < 0;
-        const int kk = south ? (-j - 1) : (j - d.ny);
-        if (kk > 1) return z;
-        const int mj = south ? kk : (d.ny - 1 - kk);
-        const int ij = south ? 0 : (d.ny - 1);
-        const Cell mir = load_direct(h, hu, hv, d.bed, d.pitch, c, mj);
-        const Cell in0 = load_direct(h, hu, hv, d.bed, d.pitch, c, ij);
-        return ghost_from(d, d.bc[south ? 2 : 3], eta_tidal, mir, in0, south ? -1.0 : 1.0, false);
-    }
-}
-
 // Workgroup id -> tile id so that each XCD (workgroups are dispatched to
 // the 8 XCDs round-robin) owns one contiguous band of tiles and the halo
 // rows and columns it shares stay in that XCD's L2.
