@@ -20,7 +20,7 @@
 // 1/3 - 2^-54/3 (ln x from a float polynomial; its error moves the result
 // by < 4e-24 relative).
 // sin/cos: Cody-Waite reduction by pi/2 held in three doubles, Taylor
-// series to x^25 / x^26 in double-double.
+// series to x^25 / x^26, the leading terms in double-double.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -169,29 +169,51 @@ __host__ __device__ __forceinline__ dd reduce(double x, double k) {
     return add(r, dd{-(k * P3), 0.0});
 }
 
-// Taylor series of sin (odd = 1) or cos (odd = 0); term n has sign
-// (-1)^((n - odd) / 2).
-__host__ __device__ __forceinline__ dd series(dd r, int odd) {
+// Term n of the Taylor series of sin (odd n) or cos (even n): 1/n! with sign
+// (-1)^(n / 2).
+__host__ __device__ __forceinline__ dd term(int n) {
+    dd c = inv_fact(n);
+    if ((n / 2) % 2 == 1) { c.hi = -c.hi; c.lo = -c.lo; }
+    return c;
+}
+
+// Series of sin (ODD) or cos from term TOP down: the terms above DD, which are
+// below 2^-53 of the result, in double (their rounding is below 2^-106 of
+// it), the others in double-double.
+template <bool ODD, int TOP, int DD>
+__host__ __device__ __forceinline__ dd series_from(dd r) {
+    static_assert(TOP % 2 == (ODD ? 1 : 0) && DD % 2 == TOP % 2 && DD < TOP, "");
     const dd r2 = mul(r, r);
-    int n = odd ? 25 : 26;
-    dd poly = inv_fact(n);
-    if (((n - odd) / 2) % 2 == 1) { poly.hi = -poly.hi; poly.lo = -poly.lo; }
-    for (n = n - 2; n >= 0; n -= 2) {
-        dd c = inv_fact(n);
-        if (((n - odd) / 2) % 2 == 1) { c.hi = -c.hi; c.lo = -c.lo; }
-        poly = add(c, mul(r2, poly));
-    }
-    return odd ? mul(r, poly) : poly;
+    double q = term(TOP).hi;
+#pragma unroll
+    for (int n = TOP - 2; n > DD; n -= 2) q = term(n).hi + r2.hi * q;
+    dd poly{q, 0.0};
+#pragma unroll
+    for (int n = DD; n >= 0; n -= 2) poly = add(term(n), mul(r2, poly));
+    return ODD ? mul(r, poly) : poly;
+}
+
+// |r| <= pi/4: to x^25 / x^26 (below 2^-90 of the result), in double from
+// x^17 (2^-54) / x^18 (2^-58).  |r| < 2^-8, where the rotation of one step
+// always is: to x^11 / x^10 (the next terms are below 2^-124), in double from
+// x^7 (2^-60) / x^6 (2^-57).
+template <bool ODD>
+__host__ __device__ __forceinline__ double series(dd r) {
+    if (fabs(r.hi) < 0x1p-8) return series_from<ODD, ODD ? 11 : 10, ODD ? 5 : 4>(r).hi;
+    return series_from<ODD, ODD ? 25 : 26, ODD ? 15 : 16>(r).hi;
+}
+
+// sin and cos of k pi/2 + r.
+__host__ __device__ __forceinline__ double quadrant(dd r, double k, int want_cos) {
+    const long long ki = (long long)k;
+    const int quad = (int)((ki + want_cos) & 3);
+    const double v = quad % 2 == 0 ? series<true>(r) : series<false>(r);
+    return (quad >= 2) ? -v : v;
 }
 
 __host__ __device__ __forceinline__ double sincos_one(double x, int want_cos) {
     const double k = rint(x * 0x1.45f306dc9c883p-1);  // x * 2/pi
-    const dd r = reduce(x, k);
-    const long long ki = (long long)k;
-    int quad = (int)(((ki % 4) + 4) % 4);
-    if (want_cos) quad = (quad + 1) % 4;
-    const dd v = series(r, (quad % 2 == 0) ? 1 : 0);
-    return (quad >= 2) ? -v.hi : v.hi;
+    return quadrant(reduce(x, k), k, want_cos);
 }
 
 __host__ __device__ __forceinline__ double sin(double x) { return sincos_one(x, 0); }
