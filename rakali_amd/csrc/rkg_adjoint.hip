@@ -1373,14 +1373,17 @@ struct BwdPlan {
     int p;                      // parity of the replay
 };
 
+// Rows per workgroup of k_adj_y for a launch over `rows` rows of 64 columns:
+// about 2048 workgroups, two waves on each of the 1024 SIMDs (1024^2 basin,
+// us: 8 rows 48, 7 rows 57, 10 rows 56).
+int adj_y_rows(long long rows) { return (int)std::min<long long>(32, std::max<long long>(4, (rows + 2047) / 2048)); }
+
 int bwd_begin(rkg_adjoint* a, double loss_scale, int tile_rows, BwdPlan& pl) {
     if (!a->have_forward) { set_error("rkg_adjoint_backward before rkg_adjoint_forward"); return RKG_ERR_NOT_READY; }
     rkg_grid* g = a->g;
-    // rows per workgroup of k_adj_y: about 2048 workgroups, two waves on each
-    // of the 1024 SIMDs (1024^2 basin, us: 8 rows 48, 7 rows 57, 10 rows 56)
     const long long ny = g->cfg.ny;
     const long long ystrips = (g->cfg.nx + WAVE - 1) / WAVE;
-    if (tile_rows <= 0) tile_rows = (int)std::min<long long>(32, std::max<long long>(4, (ny * ystrips + 2047) / 2048));
+    if (tile_rows <= 0) tile_rows = adj_y_rows(ny * ystrips);
     if (tile_rows < 4 || tile_rows > 256) { set_error("tile_rows must lie in [4, 256]"); return RKG_ERR_RANGE; }
     pl.tile_rows = tile_rows;
     pl.nb = body_blocks(g);
@@ -1622,10 +1625,30 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
     const int nsteps = as[0]->nsteps, K = as[0]->K, nseg = as[0]->nseg;
     std::vector<BwdPlan> pl(n);
     int rc = RKG_OK;
-    for (int m = 0; m < n && !rc; ++m) rc = bwd_begin(as[m], loss_scale, 0, pl[m]);
+    // tile heights by the blocks of all members: a launch serves them
+    // together (eight grids of 128..512 cells, us: replay stages 66 / 70 with
+    // each grid's own rows, 44 / 47 with these; k_adj_y 47 and 41)
+    long long yrows = 0;
+    for (int m = 0; m < n; ++m) yrows += (long long)as[m]->g->cfg.ny * ((as[m]->g->cfg.nx + WAVE - 1) / WAVE);
+    const int adj_rows = adj_y_rows(yrows);
+    const int replay_rows = rows_for([=](int rows) {
+        long long t = 0;
+        for (int m = 0; m < n; ++m) t += grid_tiles(as[m]->g->cfg.nx, as[m]->g->cfg.ny, rows);
+        return t;
+    }, 1);
+    for (int m = 0; m < n && !rc; ++m) rc = bwd_begin(as[m], loss_scale, adj_rows, pl[m]);
     if (rc) return rc;
     for (int m = 0; m < n; ++m) use_set(as[m], 0);
     hipStream_t S = as[0]->g->stream;
+    // a member's replay descriptor; a height set by the caller stays
+    auto replay_desc = [&](rkg_adjoint* a, int k) {
+        GridDesc d = stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1));
+        if (a->g->ty == 0) {
+            d.ty = replay_rows;
+            d.nsegs = (d.ny + replay_rows - 1) / replay_rows;
+        }
+        return d;
+    };
 
     // block tables
     std::vector<BlockRef> tb, ty, tx, tseed;
@@ -1643,7 +1666,7 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
             const int sb = (as[m]->ncells + 255) / 256;
             for (int b = 0; b < sb; ++b) tseed.push_back(BlockRef{m, b, sb, 0});
         }
-        const GridDesc d0 = make_desc(g);
+        const GridDesc d0 = replay_desc(as[m], 0);
         const int ntiles = d0.nstrips * d0.nsegs;
         for (int t = 0; t < ntiles; ++t) {   // the single-grid kernel's tile order and leader
             RecTile r;
@@ -1700,7 +1723,7 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
             char* h = host + tab_bytes + step_bytes * (size_t)(s * K + k);
             for (int m = 0; m < n; ++m) {
                 rkg_adjoint* a = as[m];
-                GridDesc d1 = stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1));
+                GridDesc d1 = replay_desc(a, k);
                 d1.rec = wsD1(a, k);
                 d1.hist = a->hist + HIST * k;
                 GridDesc d2 = d1;
