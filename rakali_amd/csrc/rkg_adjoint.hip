@@ -684,19 +684,27 @@ __device__ __forceinline__ double spec_eta(const GaugeSpec& G, const double* h, 
 
 // Gauge misfit of one state: loss += sum_k (eta_k - target_k)^2, eta
 // recorded per gauge; a single workgroup, fixed summation order.
-__global__ __launch_bounds__(256) void k_gauge_loss(const double* __restrict__ h, const double* __restrict__ bed,
-                                                   long long pitch, GaugeSpec G, const double* __restrict__ tgt,
-                                                   double* __restrict__ eta_out, double* __restrict__ loss) {
+struct LossArgs {
+    const double* h;
+    const double* bed;
+    long long pitch;
+    GaugeSpec G;
+    const double* tgt;          // nsteps x ng
+    double* eta;                // nsteps x ng
+    double* loss;
+};
+
+__device__ __forceinline__ void gauge_loss(const LossArgs& A, int step) {
     __shared__ double red[256];
     double acc = 0.0;
-    const int ng = G.ng;
+    const int ng = A.G.ng;
+    const double* tgt = A.tgt + (long long)step * ng;
+    double* eta = A.eta + (long long)step * ng;
     for (int k = threadIdx.x; k < ng; k += 256) {
-        const double e = spec_eta(G, h, bed, pitch, k);
-        if (eta_out) eta_out[k] = e;
-        if (tgt) {
-            const double m = e - tgt[k];
-            acc = acc + m * m;
-        }
+        const double e = spec_eta(A.G, A.h, A.bed, A.pitch, k);
+        eta[k] = e;
+        const double m = e - tgt[k];
+        acc = acc + m * m;
     }
     red[threadIdx.x] = acc;
     __syncthreads();
@@ -704,8 +712,10 @@ __global__ __launch_bounds__(256) void k_gauge_loss(const double* __restrict__ h
         if (threadIdx.x < s) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *loss = *loss + red[0];
+    if (threadIdx.x == 0) *A.loss = *A.loss + red[0];
 }
+
+__global__ __launch_bounds__(256) void k_gauge_loss(LossArgs A, int step) { gauge_loss(A, step); }
 
 // Seeds d L / d U^{n+1} at the gauges.  One thread per distinct gauge cell
 // (cell_pos[u]) adds its taps (cell_gauges[q], weight cell_w[q] for q in
@@ -890,7 +900,7 @@ __device__ __forceinline__ void dt_rev(const DtArgs& A) {
 __global__ __launch_bounds__(1024) void k_dt_rev(DtArgs A) { dt_rev(A); }
 
 // ---------------------------------------------------------------------
-// One batched reverse sweep over several sessions: each kernel below is one
+// Batched runs and sweeps over several sessions: each kernel below is one
 // launch over the blocks of every member, in the members' own block
 // decomposition (a table entry names the member and its block), so that a
 // member's arithmetic and sums are exactly those of its single-session
@@ -912,13 +922,18 @@ struct RecTileOf {
     __device__ int3 operator()(const GridDesc&) const { return make_int3(t.strip, t.seg, t.leader); }
 };
 
-template <int STAGE, bool HLLC>
-__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_replay_batch(
+// REC: recording (the replay of a sweep), else a step of the forward run.
+template <int STAGE, bool HLLC, bool REC>
+__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_step_batch(
     const GridDesc* __restrict__ descs, const RecTile* __restrict__ tiles, const int* __restrict__ parity) {
     __shared__ TileRing ring;
     const RecTile t = tiles[blockIdx.x];
     const GridDesc& d = descs[t.member];
-    stage_tile<STAGE, HLLC, true, true, RecTileOf>(d, ring, parity[t.member], MODE_STEP, d.t_end, RecTileOf{t});
+    stage_tile<STAGE, HLLC, true, REC, RecTileOf>(d, ring, parity[t.member], MODE_STEP, d.t_end, RecTileOf{t});
+}
+
+__global__ __launch_bounds__(256) void k_gauge_loss_batch(const LossArgs* __restrict__ la, int step) {
+    gauge_loss(la[blockIdx.x], step);
 }
 
 __global__ __launch_bounds__(256) void k_gauge_seed_batch(const SeedArgs* __restrict__ sa,
@@ -994,6 +1009,9 @@ struct rkg_adjoint {
     int edge_len;
     double* loss_dev;
     double* loss_host;
+    char* batch_host;           // argument tables of batched calls that this session leads (pinned
+    char* batch_dev;            // and on the device), grown as needed
+    size_t batch_bytes;
     CtrlSlot end_ctrl[2];
     int end_parity;
     bool have_forward;
@@ -1258,6 +1276,8 @@ void rkg_adjoint_destroy(rkg_adjoint** pa) {
     for (hipEvent_t ev : a->seg_ev)
         if (ev) (void)hipEventDestroy(ev);
     if (a->loss_host) (void)hipHostFree(a->loss_host);
+    if (a->batch_host) (void)hipHostFree(a->batch_host);
+    if (a->batch_dev) (void)hipFree(a->batch_dev);
     if (a->ev[0]) (void)hipEventDestroy(a->ev[0]);
     if (a->ev[1]) (void)hipEventDestroy(a->ev[1]);
     rkg_grid* g = a->g;
@@ -1320,29 +1340,35 @@ int fwd_begin(rkg_adjoint* a) {
     return RKG_OK;
 }
 
+LossArgs loss_args(rkg_adjoint* a) {
+    rkg_grid* g = a->g;
+    return LossArgs{g->buf, g->buf + 6 * g->plane, (long long)g->pitch, gauge_spec(a), a->tgt, a->eta, a->loss_dev};
+}
+
+// The checkpoint of segment s, the state before step s K, on stream st.
+int fwd_checkpoint(rkg_adjoint* a, int s, hipStream_t st) {
+    rkg_grid* g = a->g;
+    const size_t Pl = g->plane;
+    HIP_TRY(hipMemcpyAsync(a->ckpt + (size_t)s * 3 * Pl, g->buf, 3 * Pl * sizeof(double), hipMemcpyDeviceToDevice, st));
+    HIP_TRY(hipMemcpyAsync(a->ckpt_ctrl + 2 * s, g->ctrl, 2 * sizeof(CtrlSlot), hipMemcpyDeviceToDevice, st));
+    a->ckpt_parity[s] = g->parity;
+    return RKG_OK;
+}
+
 // Step n of the forward run: the checkpoint at a segment start, the step,
 // the gauge misfit.
 int fwd_step(rkg_adjoint* a, int n) {
     rkg_grid* g = a->g;
-    const size_t Pl = g->plane;
+    int rc = RKG_OK;
     if (n % a->K == 0) {
-        const int s = n / a->K;
-        if (g->speed_stale) {   // make the control slot current before saving it
-            int rc = rkg_step(g, 0);
-            if (rc) return rc;
-        }
-        HIP_TRY(hipMemcpyAsync(a->ckpt + (size_t)s * 3 * Pl, g->buf, 3 * Pl * sizeof(double), hipMemcpyDeviceToDevice,
-                               g->stream));
-        HIP_TRY(hipMemcpyAsync(a->ckpt_ctrl + 2 * s, g->ctrl, 2 * sizeof(CtrlSlot), hipMemcpyDeviceToDevice,
-                               g->stream));
-        a->ckpt_parity[s] = g->parity;
+        if (g->speed_stale) rc = rkg_step(g, 0);   // make the control slot current before saving it
+        if (!rc) rc = fwd_checkpoint(a, n / a->K, g->stream);
+        if (rc) return rc;
     }
-    int rc = rkg_step(g, 1);
+    rc = rkg_step(g, 1);
     if (rc) return rc;
     if (a->ng > 0)
-        hipLaunchKernelGGL(k_gauge_loss, dim3(1), dim3(256), 0, g->stream, g->buf, g->buf + 6 * Pl,
-                           (long long)g->pitch, gauge_spec(a), a->tgt + (size_t)n * a->ng,
-                           a->eta + (size_t)n * a->ng, a->loss_dev);
+        hipLaunchKernelGGL(k_gauge_loss, dim3(1), dim3(256), 0, g->stream, loss_args(a), n);
     return RKG_OK;
 }
 
@@ -1611,6 +1637,145 @@ int bwd_finish(rkg_adjoint* a) {
     return RKG_OK;
 }
 
+size_t al256(size_t x) { return (x + 255) / 256 * 256; }
+
+// Room for `bytes` of argument tables with the batch's first session.  Every
+// batched call ends with its streams drained, so the last call's are free.
+int batch_tables(rkg_adjoint* a, size_t bytes) {
+    if (a->batch_bytes >= bytes) return RKG_OK;
+    if (a->batch_host) (void)hipHostFree(a->batch_host);
+    if (a->batch_dev) (void)hipFree(a->batch_dev);
+    a->batch_host = a->batch_dev = nullptr;
+    a->batch_bytes = 0;
+    hipError_t e = hipHostMalloc((void**)&a->batch_host, bytes, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc((void**)&a->batch_dev, bytes);
+    if (e != hipSuccess) {
+        if (a->batch_host) (void)hipHostFree(a->batch_host);
+        a->batch_host = nullptr;
+        a->batch_dev = nullptr;
+        set_error("batched adjoint: cannot allocate its %zu-byte argument tables: %s", bytes, hipGetErrorString(e));
+        return RKG_ERR_HIP;
+    }
+    a->batch_bytes = bytes;
+    return RKG_OK;
+}
+
+// Rows per stage tile by the tiles of all members: a launch serves them
+// together (eight grids of 128..512 cells, us: replay stages 66 / 70 with
+// each grid's own rows, 44 / 47 with these).
+int batch_rows(int n, rkg_adjoint* const* as) {
+    return rows_for([=](int rows) {
+        long long t = 0;
+        for (int m = 0; m < n; ++m) t += grid_tiles(as[m]->g->cfg.nx, as[m]->g->cfg.ny, rows);
+        return t;
+    }, 1);
+}
+
+// d with the batch's rows per tile; a height set by the caller stays.
+GridDesc batch_desc(const rkg_adjoint* a, GridDesc d, int rows) {
+    if (a->g->ty == 0) {
+        d.ty = rows;
+        d.nsegs = (d.ny + rows - 1) / rows;
+    }
+    return d;
+}
+
+// Member m's tiles, in the order and with the leader of its own launches.
+void batch_tiles(const GridDesc& d, int m, std::vector<RecTile>& t) {
+    for (int k = 0; k < d.nstrips * d.nsegs; ++k) t.push_back(RecTile{m, k % d.nstrips, k / d.nstrips, k == 0});
+}
+
+// The work of every stream before what the first stream queues next (to_first),
+// or the work of the first before what the others queue.
+hipError_t join_streams(int n, rkg_adjoint* const* as, hipEvent_t ev, bool to_first) {
+    hipStream_t S = as[0]->g->stream;
+    hipError_t e = hipSuccess;
+    if (!to_first) e = hipEventRecord(ev, S);
+    for (int m = 1; m < n && e == hipSuccess; ++m) {
+        if (to_first) {
+            e = hipEventRecord(ev, as[m]->g->stream);
+            if (e == hipSuccess) e = hipStreamWaitEvent(S, ev, 0);
+        } else {
+            e = hipStreamWaitEvent(as[m]->g->stream, ev, 0);
+        }
+    }
+    return e;
+}
+
+// Whether the forward runs of n sessions can go as one: one device, one
+// solver, and steps that launch the two stage kernels and nothing else.
+bool fwd_batchable(int n, rkg_adjoint* const* as) {
+    for (int m = 0; m < n; ++m) {
+        const rkg_grid* g = as[m]->g;
+        if (g->device != as[0]->g->device || (g->cfg.use_hllc != 0) != (as[0]->g->cfg.use_hllc != 0)) return false;
+        if (!g->nfield || g->mpart || g->gauges || g->prof) return false;
+    }
+    return n > 1;
+}
+
+// The forward runs of n sessions on the first session's stream: three
+// launches a step (both stages and the gauge misfits of every member)
+// instead of three per member, which the host could not issue as fast as the
+// GPU ran them.  Every member's arithmetic is that of its own run.
+int fwd_batched(int n, rkg_adjoint* const* as) {
+    const bool hllc = as[0]->g->cfg.use_hllc != 0;
+    const int nsteps = as[0]->nsteps, K = as[0]->K, rows = batch_rows(n, as);
+    hipStream_t S = as[0]->g->stream;
+    std::vector<GridDesc> d(n);
+    std::vector<RecTile> tiles;
+    std::vector<LossArgs> loss;
+    std::vector<int> par(2 * n);
+    int rc = RKG_OK;
+    for (int m = 0; m < n && !rc; ++m) {
+        rkg_grid* g = as[m]->g;
+        if (g->speed_stale) rc = rkg_step(g, 0);   // make the control slot current
+        d[m] = batch_desc(as[m], make_desc(g), rows);
+        batch_tiles(d[m], m, tiles);
+        if (as[m]->ng > 0) loss.push_back(loss_args(as[m]));
+        par[m] = g->parity;
+        par[n + m] = g->parity ^ 1;
+    }
+    if (rc) return rc;
+    const size_t oT = al256(n * sizeof(GridDesc)), oL = oT + al256(tiles.size() * sizeof(RecTile)),
+                 oP = oL + al256((loss.size() + 1) * sizeof(LossArgs)), total = oP + al256(2 * n * sizeof(int));
+    if ((rc = batch_tables(as[0], total))) return rc;
+    char *host = as[0]->batch_host, *dev = as[0]->batch_dev;
+    std::memcpy(host, d.data(), n * sizeof(GridDesc));
+    std::memcpy(host + oT, tiles.data(), tiles.size() * sizeof(RecTile));
+    if (!loss.empty()) std::memcpy(host + oL, loss.data(), loss.size() * sizeof(LossArgs));
+    std::memcpy(host + oP, par.data(), 2 * n * sizeof(int));
+    hipEvent_t join = nullptr;
+    HIP_TRY(hipEventCreateWithFlags(&join, hipEventDisableTiming));
+    hipError_t e = join_streams(n, as, join, true);
+    if (e == hipSuccess) e = hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, S);
+    const GridDesc* dd = (const GridDesc*)dev;
+    const RecTile* dt = (const RecTile*)(dev + oT);
+    const dim3 grid((unsigned)tiles.size()), block(WAVE);
+    for (int k = 0; k < nsteps && !rc && e == hipSuccess; ++k) {
+        if (k % K == 0)
+            for (int m = 0; m < n && !rc; ++m) rc = fwd_checkpoint(as[m], k / K, S);
+        const int* dp = (const int*)(dev + oP) + (k & 1) * n;
+        if (hllc) {
+            hipLaunchKernelGGL((k_step_batch<1, true, false>), grid, block, 0, S, dd, dt, dp);
+            hipLaunchKernelGGL((k_step_batch<2, true, false>), grid, block, 0, S, dd, dt, dp);
+        } else {
+            hipLaunchKernelGGL((k_step_batch<1, false, false>), grid, block, 0, S, dd, dt, dp);
+            hipLaunchKernelGGL((k_step_batch<2, false, false>), grid, block, 0, S, dd, dt, dp);
+        }
+        for (int m = 0; m < n; ++m) as[m]->g->parity ^= 1;
+        if (!loss.empty())
+            hipLaunchKernelGGL(k_gauge_loss_batch, dim3((unsigned)loss.size()), dim3(256), 0, S,
+                               (const LossArgs*)(dev + oL), k);
+    }
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = join_streams(n, as, join, false);
+    // the tables may be rewritten once every launch that reads them has finished
+    if (e != hipSuccess || rc) (void)hipStreamSynchronize(S);
+    (void)hipEventDestroy(join);
+    if (e != hipSuccess && !rc) { set_error("batched forward runs: %s", hipGetErrorString(e)); rc = RKG_ERR_HIP; }
+    return rc;
+}
+
 // The reverse sweeps of n sessions as one sweep on the first session's
 // stream: per replay step two launches (both stages of every member) and
 // per reverse step eight (gauge seeds, the two stages' bodies and faces, the
@@ -1625,29 +1790,16 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
     const int nsteps = as[0]->nsteps, K = as[0]->K, nseg = as[0]->nseg;
     std::vector<BwdPlan> pl(n);
     int rc = RKG_OK;
-    // tile heights by the blocks of all members: a launch serves them
-    // together (eight grids of 128..512 cells, us: replay stages 66 / 70 with
-    // each grid's own rows, 44 / 47 with these; k_adj_y 47 and 41)
+    // k_adj_y's rows too by the blocks of all members (us: 47 -> 41)
     long long yrows = 0;
     for (int m = 0; m < n; ++m) yrows += (long long)as[m]->g->cfg.ny * ((as[m]->g->cfg.nx + WAVE - 1) / WAVE);
-    const int adj_rows = adj_y_rows(yrows);
-    const int replay_rows = rows_for([=](int rows) {
-        long long t = 0;
-        for (int m = 0; m < n; ++m) t += grid_tiles(as[m]->g->cfg.nx, as[m]->g->cfg.ny, rows);
-        return t;
-    }, 1);
+    const int adj_rows = adj_y_rows(yrows), replay_rows = batch_rows(n, as);
     for (int m = 0; m < n && !rc; ++m) rc = bwd_begin(as[m], loss_scale, adj_rows, pl[m]);
     if (rc) return rc;
     for (int m = 0; m < n; ++m) use_set(as[m], 0);
     hipStream_t S = as[0]->g->stream;
-    // a member's replay descriptor; a height set by the caller stays
     auto replay_desc = [&](rkg_adjoint* a, int k) {
-        GridDesc d = stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1));
-        if (a->g->ty == 0) {
-            d.ty = replay_rows;
-            d.nsegs = (d.ny + replay_rows - 1) / replay_rows;
-        }
-        return d;
+        return batch_desc(a, stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1)), replay_rows);
     };
 
     // block tables
@@ -1666,21 +1818,12 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
             const int sb = (as[m]->ncells + 255) / 256;
             for (int b = 0; b < sb; ++b) tseed.push_back(BlockRef{m, b, sb, 0});
         }
-        const GridDesc d0 = replay_desc(as[m], 0);
-        const int ntiles = d0.nstrips * d0.nsegs;
-        for (int t = 0; t < ntiles; ++t) {   // the single-grid kernel's tile order and leader
-            RecTile r;
-            r.member = m;
-            r.strip = t % d0.nstrips;
-            r.seg = t / d0.nstrips;
-            r.leader = t == 0;
-            trec.push_back(r);
-        }
+        batch_tiles(replay_desc(as[m], 0), m, trec);
     }
     // per global step: replay descriptors (stage 1, 2), replay parities, and
     // the reverse arguments (stage 2, stage 1, seeds, dt), n of each
     const size_t szGD = sizeof(GridDesc), szAS = sizeof(AdjStage), szSA = sizeof(SeedArgs), szDA = sizeof(DtArgs);
-    auto al = [](size_t x) { return (x + 255) / 256 * 256; };
+    auto al = [](size_t x) { return al256(x); };
     const size_t oRec1 = 0, oRec2 = oRec1 + al(n * szGD), oPar = oRec2 + al(n * szGD), oSt2 = oPar + al(n * sizeof(int)),
                  oSt1 = oSt2 + al(n * szAS), oSeed = oSt1 + al(n * szAS), oDt = oSeed + al(n * szSA),
                  step_bytes = oDt + al(n * szDA);
@@ -1688,22 +1831,10 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
                              al(tx.size() * sizeof(BlockRef)) + al(std::max<size_t>(1, tseed.size()) * sizeof(BlockRef)) +
                              al(trec.size() * sizeof(RecTile));
     const size_t total = tab_bytes + step_bytes * (size_t)nsteps;
-    char* host = nullptr;
-    char* dev = nullptr;
+    if ((rc = batch_tables(as[0], total))) return rc;
+    char *host = as[0]->batch_host, *dev = as[0]->batch_dev;
     hipEvent_t join = nullptr;
-    auto cleanup = [&]() {
-        if (host) (void)hipHostFree(host);
-        if (dev) (void)hipFree(dev);
-        if (join) (void)hipEventDestroy(join);
-    };
-    hipError_t e = hipHostMalloc((void**)&host, total, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc((void**)&dev, total);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
-    if (e != hipSuccess) {
-        cleanup();
-        set_error("batched adjoint sweep: cannot allocate its %zu-byte argument tables: %s", total, hipGetErrorString(e));
-        return RKG_ERR_HIP;
-    }
+    HIP_TRY(hipEventCreateWithFlags(&join, hipEventDisableTiming));
     size_t off = 0;
     auto put = [&](const void* src, size_t bytes) {
         const size_t o = off;
@@ -1745,13 +1876,10 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
         }
     }
     // the sweep starts after every member's queued work (bwd_begin's clears)
-    for (int m = 1; m < n && e == hipSuccess; ++m) {
-        e = hipEventRecord(join, as[m]->g->stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(S, join, 0);
-    }
+    hipError_t e = join_streams(n, as, join, true);
     if (e == hipSuccess) e = hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, S);
     if (e != hipSuccess) {
-        cleanup();
+        (void)hipEventDestroy(join);
         set_error("batched adjoint sweep: %s", hipGetErrorString(e));
         return RKG_ERR_HIP;
     }
@@ -1766,11 +1894,11 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
             const GridDesc* r2 = (const GridDesc*)(d + oRec2);
             const int* par = (const int*)(d + oPar);
             if (hllc) {
-                hipLaunchKernelGGL((k_replay_batch<1, true>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
-                hipLaunchKernelGGL((k_replay_batch<2, true>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
+                hipLaunchKernelGGL((k_step_batch<1, true, true>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
+                hipLaunchKernelGGL((k_step_batch<2, true, true>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
             } else {
-                hipLaunchKernelGGL((k_replay_batch<1, false>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
-                hipLaunchKernelGGL((k_replay_batch<2, false>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
+                hipLaunchKernelGGL((k_step_batch<1, false, true>), dim3(nrec), dim3(WAVE), 0, S, r1, dTr, par);
+                hipLaunchKernelGGL((k_step_batch<2, false, true>), dim3(nrec), dim3(WAVE), 0, S, r2, dTr, par);
             }
         }
         for (int k = Ks - 1; k >= 0; --k) {
@@ -1801,13 +1929,12 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
     }
     if (!rc) e = hipGetLastError();
     // every member's stream continues after the sweep
-    if (!rc && e == hipSuccess) e = hipEventRecord(join, S);
-    for (int m = 1; m < n && !rc && e == hipSuccess; ++m) e = hipStreamWaitEvent(as[m]->g->stream, join, 0);
+    if (!rc && e == hipSuccess) e = join_streams(n, as, join, false);
     if (!rc && e != hipSuccess) { set_error("batched adjoint sweep: %s", hipGetErrorString(e)); rc = RKG_ERR_HIP; }
     for (int m = 0; m < n && !rc; ++m) rc = bwd_end(as[m]);
-    // the tables are freed once every launch that reads them has finished
+    // the tables may be rewritten once every launch that reads them has finished
     for (int m = 0; m < n; ++m) (void)hipStreamSynchronize(as[m]->g->stream);
-    cleanup();
+    (void)hipEventDestroy(join);
     if (rc) return rc;
     for (int m = 0; m < n && !rc; ++m) rc = bwd_finish(as[m]);
     return rc;
@@ -1875,14 +2002,19 @@ int rkg_adjoint_backward(rkg_adjoint* a, double loss_scale, int tile_rows) {
     return bwd_finish(a);
 }
 
-// The forward runs of n sessions (one grid and stream each), queued step
-// by step across the sessions so that their kernels overlap.
+// The forward runs of n sessions (one grid and stream each): as one run
+// where they can (fwd_batchable), else queued step by step across the
+// sessions so that their kernels overlap.
 int rkg_adjoint_forward_many(int n, rkg_adjoint* const* as, double* losses) {
     int rc = check_batch(n, as);
     if (rc) return rc;
     for (int m = 0; m < n && !rc; ++m) rc = fwd_begin(as[m]);
-    for (int k = 0; k < as[0]->nsteps && !rc; ++k)
-        for (int m = 0; m < n && !rc; ++m) rc = fwd_step(as[m], k);
+    if (!rc && fwd_batchable(n, as)) {
+        rc = fwd_batched(n, as);
+    } else {
+        for (int k = 0; k < as[0]->nsteps && !rc; ++k)
+            for (int m = 0; m < n && !rc; ++m) rc = fwd_step(as[m], k);
+    }
     for (int m = 0; m < n && !rc; ++m) rc = fwd_end(as[m]);
     if (rc) return rc;
     for (int m = 0; m < n; ++m) HIP_TRY(hipStreamSynchronize(as[m]->g->stream));

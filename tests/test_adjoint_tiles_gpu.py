@@ -44,3 +44,51 @@ def test_face_reverses_at_tile_edges(ref, nx, ny, bc):
         assert np.abs(got - want[k]).max() <= 1e-9 * np.abs(want[k]).max(), k
     sess.close()
     g.close()
+
+
+@pytest.mark.parametrize("hllc", [True, False])
+@pytest.mark.parametrize("rows", [0, 5])
+def test_batched_forward_runs_equal_single_runs(hllc, rows):
+    """One launch for all members: uneven sizes down to two cells, a member
+    without gauges, an odd start parity, a second batch of another size."""
+    from rakali_amd.adjoint import GaugeMisfit, backward_many, forward_many
+    sizes, steps, K = [(2, 2), (61, 33), (130, 70), (200, 9), (3, 40)], 7, 3
+    grids, sess, states = [], [], []
+    for m, (nx, ny) in enumerate(sizes):
+        rng, b, n, h, hu, hv = generic_state(nx, ny, 90 + m)
+        g = gpu_grid(nx, ny, dict(CFG, dt=0.0), hllc, EDGES[m % 4], 1e-3 * (m % 2))
+        g.tile_rows = rows
+        k = 0 if m == 3 else 6
+        gauges = [(int(rng.integers(0, nx)), int(rng.integers(0, ny))) for _ in range(k)]
+        sess.append(GaugeMisfit(g, steps, K, gauges, rng.normal(0.0, 0.05, (steps, k))))
+        grids.append(g)
+        states.append((b, n, h, hu, hv))
+
+    def start(m):
+        load(grids[m], *states[m])
+        if m == 1:
+            grids[m].step(1)
+
+    def result(m):
+        return ({k: grids[m].get_field(k) for k in ("h", "hu", "hv")}, grids[m].clock, sess[m].gauge_eta(),
+                {k: sess[m].gradient(k) for k in ("b", "n", "h")})
+
+    for batch in ([0, 1, 2, 3, 4], [4, 2], [3, 0, 1, 2]):
+        print(f"[batched forward] {batch} hllc={hllc} rows={rows}", flush=True)
+        for m in batch:
+            start(m)
+        losses = forward_many([sess[m] for m in batch])
+        backward_many([sess[m] for m in batch])
+        many = [result(m) for m in batch]
+        for i, m in enumerate(batch):
+            start(m)
+            assert sess[m].forward() == losses[i]
+            sess[m].backward()
+            f, clock, eta, grad = result(m)
+            assert clock == many[i][1] and np.array_equal(eta, many[i][2])
+            assert all(np.array_equal(f[k], many[i][0][k]) for k in f)
+            assert all(np.array_equal(grad[k], many[i][3][k]) for k in grad)
+    for s in sess:
+        s.close()
+    for g in grids:
+        g.close()
