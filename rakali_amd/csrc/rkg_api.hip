@@ -101,14 +101,7 @@ bool valid(const rkg_grid* g) { return g != nullptr && g->magic == GRID_MAGIC; }
 
 int refresh_speed(rkg_grid* g) {
     GridDesc d = make_desc(g);
-    const CtrlSlot& cur = g->ctrl_host[g->parity];
-    (void)cur;
-    // keep t / dt / step_count of the current slot, clear its speed max
-    HIP_TRY(hipMemcpyAsync(g->ctrl_host, g->ctrl, 2 * sizeof(CtrlSlot), hipMemcpyDeviceToHost, g->stream));
-    HIP_TRY(hipStreamSynchronize(g->stream));
-    const CtrlSlot c = g->ctrl_host[g->parity];
-    hipLaunchKernelGGL(k_ctrl_reset, dim3(1), dim3(64), 0, g->stream, g->ctrl, g->parity, c.t, c.dt,
-                       c.step_count, c.mass_out, c.mass_src);
+    hipLaunchKernelGGL(k_speed_reset, dim3(1), dim3(64), 0, g->stream, g->ctrl, g->parity);
     hipLaunchKernelGGL(k_init_speed, dim3(sweep_blocks((long long)g->cfg.nx * g->cfg.ny)), dim3(256), 0, g->stream, d, g->parity);
     HIP_TRY(hipGetLastError());
     g->speed_stale = false;

@@ -172,17 +172,10 @@ int build_tables(rkg_ensemble* e) {
 }
 
 int refresh_speeds(rkg_ensemble* e) {
-    bool any = false;
-    for (int m = 0; m < e->n; ++m) any = any || e->speed_stale[m];
-    if (!any) return RKG_OK;
-    HIP_TRY(hipMemcpyAsync(e->ctrl_host, e->ctrl, 2 * e->n * sizeof(CtrlSlot), hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
     for (int m = 0; m < e->n; ++m) {
         if (!e->speed_stale[m]) continue;
         const GridDesc d = ens_desc(e, m);
-        const CtrlSlot c = e->ctrl_host[2 * m + e->parity];
-        hipLaunchKernelGGL(k_ctrl_reset, dim3(1), dim3(64), 0, e->stream, d.ctrl, e->parity, c.t, c.dt,
-                           c.step_count, c.mass_out, c.mass_src);
+        hipLaunchKernelGGL(k_speed_reset, dim3(1), dim3(64), 0, e->stream, d.ctrl, e->parity);
         hipLaunchKernelGGL(k_init_speed, dim3(sweep_blocks((long long)d.nx * d.ny)), dim3(256), 0, e->stream, d, e->parity);
         e->speed_stale[m] = 0;
     }

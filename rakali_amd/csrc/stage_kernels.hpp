@@ -240,6 +240,15 @@ __global__ void k_ctrl_reset(CtrlSlot* ctrl, int p, double t, double dt, long lo
     }
 }
 
+// k_ctrl_reset to the slot's own clock and budget.
+__global__ void k_speed_reset(CtrlSlot* ctrl, int p) {
+    if (threadIdx.x < SPEED_WAYS) ctrl[p].speed[threadIdx.x * SPEED_STRIDE] = 0ull;
+    if (threadIdx.x == 0) {
+        ctrl[p].active = 1;
+        ctrl[p].t_bc = ctrl[p].t;
+    }
+}
+
 // Boundary mass budget of one SSP-RK2 step (rki_solver.F90:507-537, called
 // after each stage's flux at :769 and :796): mass_out -= 0.5 dt sum(flux_h)
 // area per stage.  The per-tile sums of both stages are added in a fixed
