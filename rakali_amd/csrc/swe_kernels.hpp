@@ -544,16 +544,18 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
             else if (two_op) divergence<DIV_TWO_OP>(g, d.sdx, fxl, fxr, y, fh, fhu, fhv);
             else divergence<DIV_SHARED>(g, d.sdx, fxl, fxr, y, fh, fhu, fhv);
         };
+        // Row j+3, needed at the end of the row, before the faces (4096^2, three
+        // grids: 937 us a step, 948 with the loads after them; its eight registers
+        // fit without spills).  The loads are unconditional (the last row of the
+        // halo again, a cell of the grid): under a condition the compiler waits
+        // for everything in flight where the paths join.
+        const int jn = min(j + 3, j1 + 1);
+        const Cell src = row_source<EDGE>(d, s, lsrc, jn);
+        __builtin_amdgcn_sched_barrier(0);
         if (__builtin_expect(plain_row, 0)) faces(ExactTag<true>{});
         else faces(ExactTag<false>{});
 
-        // Row j+3 and U^n at (c, j), both needed at the end of the row: the
-        // cell update hides them, and the faces keep their registers.  The
-        // loads are unconditional (the last row of the halo again, a cell of
-        // the grid): under a condition the compiler waits for everything in
-        // flight where the paths join.
-        const int jn = min(j + 3, j1 + 1);
-        const Cell src = row_source<EDGE>(d, s, lsrc, jn);
+        // U^n at (c, j): the cell update hides it, and the faces keep their registers
         Cell un{0.0, 0.0, 0.0, 0.0};
         if (read_un) {
             const long long k = (long long)max(j, 0) * pitch + c_in;
