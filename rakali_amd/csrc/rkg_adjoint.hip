@@ -57,15 +57,15 @@ struct AdjStage {
     double* part_dt;            // per body workgroup: sum of d L / d dt of its cells
     double* pval;               // stage 1 with the CFL dt: per body workgroup, max CFL speed of
     long long* pidx;            // the stage input and its first cell (x fastest), else null
-    double* edge_lg;            // adjoint (h, normal momentum) of every tidal ghost cell, see edge_slot
+    double* edge_eta;           // d L / d eta through every tidal ghost cell, see edge_slot
     int edge_len;               // max(nx, ny)
     int ty;                     // rows per tile of k_adj_y
 };
 
 // Slot of ghost layer kk (0 = next to the edge) at position p along edge e
-// (0 W, 1 E, 2 S, 3 N) in edge_lg (two doubles per slot).
+// (0 W, 1 E, 2 S, 3 N) in edge_eta.
 __host__ __device__ __forceinline__ long long edge_slot(int e, int kk, int p, int len) {
-    return ((long long)(e * 2 + kk) * len + p) * 2;
+    return (long long)(e * 2 + kk) * len + p;
 }
 
 constexpr int HIST = 3;         // doubles per step in hist
@@ -225,10 +225,11 @@ __device__ __forceinline__ Cell side_ghost(const GridDesc& d, int side, double e
 
 // Adjoint of the row-y ghost at column x onto interior cells (x-direction
 // ghosts: normal momentum hu); cell(col) gives the row's interior cells.
-// Returns the contributions for the mirror and first-interior columns.
+// Returns the contributions for the mirror and first-interior columns, and in
+// leta that for the tide.
 template <class CELL>
 __device__ __forceinline__ void ghost_x_rev(const GridDesc& d, double eta, int x, CELL cell, const adj::C4& lg, int& mcol,
-                                            int& icol, adj::C4& lm, adj::C4& li) {
+                                            int& icol, adj::C4& lm, adj::C4& li, double* leta) {
     const bool west = x < 0;
     const int kk = west ? (-x - 1) : (x - d.nx);
     mcol = west ? kk : (d.nx - 1 - kk);
@@ -236,11 +237,11 @@ __device__ __forceinline__ void ghost_x_rev(const GridDesc& d, double eta, int x
     lm = adj::C4{0, 0, 0, 0};
     li = adj::C4{0, 0, 0, 0};
     adj::ghost_rev(d.bc[west ? 0 : 1], d.g, eta, d.inflow_velocity, d.clamped_elevation, cell(mcol), cell(icol),
-                   west ? -1.0 : 1.0, true, lg, lm, li);
+                   west ? -1.0 : 1.0, true, lg, lm, li, leta);
 }
 
 __device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, int x, int y, const adj::C4& lg, int& mrow,
-                                            int& irow, adj::C4& lm, adj::C4& li) {
+                                            int& irow, adj::C4& lm, adj::C4& li, double* leta) {
     const bool south = y < 0;
     const int kk = south ? (-y - 1) : (y - d.ny);
     mrow = south ? kk : (d.ny - 1 - kk);
@@ -250,7 +251,7 @@ __device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, int x
     lm = adj::C4{0, 0, 0, 0};
     li = adj::C4{0, 0, 0, 0};
     adj::ghost_rev(d.bc[south ? 2 : 3], d.g, eta, d.inflow_velocity, d.clamped_elevation, mir, in0,
-                   south ? -1.0 : 1.0, false, lg, lm, li);
+                   south ? -1.0 : 1.0, false, lg, lm, li, leta);
 }
 
 // Two LDS rows of the 11 planes over 64 columns (the twelfth is a spare: two
@@ -269,7 +270,8 @@ struct YRows {
 // r and r+1 and the y slope of row r, which completes row r-1.  A ghost row's
 // adjoint is added to its source rows when row 0 is complete (south), or with
 // the last row (north, row ny-2 waiting for it).  TY: a south or north edge is
-// tidal, and the adjoints of its ghost cells are kept in edge_lg for k_dt_rev.
+// tidal, and what its ghost cells give the tide is kept in edge_eta for
+// k_dt_rev.
 //
 // Bound by latency with two wavefronts on a SIMD (face_rev's live values leave
 // no room for a third): what iteration r + 1 needs is loaded into LDS during
@@ -352,13 +354,11 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
     // Adjoint lg of ghost row rho onto rows mrow and irow.
     auto fold = [&](int rho, const Acc& ghost, int& mrow, int& irow, adj::C4& lm, adj::C4& li) {
         const adj::C4 lg = c4(ghost);
-        ghost_y_rev(d, eta, xs, rho, lg, mrow, irow, lm, li);
+        double leta = 0.0;
+        ghost_y_rev(d, eta, xs, rho, lg, mrow, irow, lm, li, &leta);
         const int e = rho < 0 ? 2 : 3;
-        if (TY && xin && d.bc[e] == BC_TIDAL) {
-            const long long o = edge_slot(e, rho < 0 ? -rho - 1 : rho - ny, x, a.edge_len);
-            a.edge_lg[o] = lg.h;
-            a.edge_lg[o + 1] = lg.hv;
-        }
+        if (TY && xin && d.bc[e] == BC_TIDAL)
+            a.edge_eta[edge_slot(e, rho < 0 ? -rho - 1 : rho - ny, x, a.edge_len)] = leta;
     };
 
     for (int r = rs; r <= re; ++r) {
@@ -571,14 +571,12 @@ __device__ __forceinline__ void adj_x(const AdjStage& a, XRows& rows, int blk) {
             adj::C4 gm{0, 0, 0, 0}, gi{0, 0, 0, 0};
             int mcol = -100, icol = -100;
             if (x == -1 || x == -2 || x == d.nx || x == d.nx + 1) {
-                ghost_x_rev(d, eta, x, [&](int c) { return cell_at(c - cb); }, mine, mcol, icol, gm, gi);
+                double leta = 0.0;
+                ghost_x_rev(d, eta, x, [&](int c) { return cell_at(c - cb); }, mine, mcol, icol, gm, gi, &leta);
                 const int e = x < 0 ? 0 : 1;
                 // kept once, by the tile holding the edge column
-                if (TX && (x < 0 ? c0 == 0 : c1 == d.nx) && d.bc[e] == BC_TIDAL) {
-                    const long long o = edge_slot(e, x < 0 ? -x - 1 : x - d.nx, r, a.edge_len);
-                    a.edge_lg[o] = mine.h;
-                    a.edge_lg[o + 1] = mine.hu;
-                }
+                if (TX && (x < 0 ? c0 == 0 : c1 == d.nx) && d.bc[e] == BC_TIDAL)
+                    a.edge_eta[edge_slot(e, x < 0 ? -x - 1 : x - d.nx, r, a.edge_len)] = leta;
             }
             // lanes holding columns -2, -1, nx, nx + 1 (when inside the wavefront)
             const int srcs[4] = {-c0, 1 - c0, d.nx - c0 + 2, d.nx - c0 + 3};
@@ -609,54 +607,18 @@ __global__ __launch_bounds__(WAVE) void k_adj_x(AdjStage a) {
     adj_x<HLLC, STAGE, TX>(a, rows, blockIdx.x);
 }
 
-// d L / d eta_tidal from one tidal ghost cell (adjoints lg0 of h and lg1
-// of the normal momentum; in0 its source cell of the stage input): the
-// eta_ext terms of bc_flather_edge (rki_boundary.F90:331-343),
-// h_g = max(eta_ext - b_g, 0) and the radiation term.
-__device__ double eta_rev_one(const GridDesc& d, double eta, const Cell& in0, double lg0, double lg1, double sgn,
-                              bool xe) {
-    adj::C4 lg{lg0, 0.0, 0.0, 0.0};
-    if (xe) lg.hu = lg1;
-    else lg.hv = lg1;
-    adj::C4 lm{0, 0, 0, 0}, li{0, 0, 0, 0};
-    double le = 0.0;
-    adj::ghost_rev(BC_TIDAL, d.g, eta, d.inflow_velocity, d.clamped_elevation, in0, in0, sgn, xe, lg, lm, li, &le);
-    return le;
-}
-
-// This thread's share for both stages at once (stage 1: input d.ah at
-// eta1, ghost adjoints lg1; stage 2: input in2 at eta2, lg2).  Items
-// i = threadIdx.x + q blockDim.x go two at a time, their loads issued
-// together; each stage's sum keeps the item order.
-__device__ void eta_parts(const GridDesc& d, double eta1, double eta2, const double* in2, const double* lg1,
-                          const double* lg2, int len, double* acc1, double* acc2) {
+// This thread's share of d L / d eta of both stages (eta1, eta2: their
+// edge_eta), edge by edge, each stage's sum in item order.
+__device__ void eta_parts(const GridDesc& d, const double* eta1, const double* eta2, int len, double* acc1, double* acc2) {
     double s1 = 0.0, s2 = 0.0;
     for (int e = 0; e < 4; ++e) {
         if (d.bc[e] != BC_TIDAL) continue;
-        const bool xe = e < 2;
-        const int n = xe ? d.ny : d.nx;
-        const double sgn = (e == 0 || e == 2) ? -1.0 : 1.0;
-        for (int i0 = threadIdx.x; i0 < 2 * n; i0 += 2 * blockDim.x) {
-            Cell c1[2], c2[2];
-            double g[2][4];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int i = u == 0 ? i0 : min(i0 + (int)blockDim.x, 2 * n - 1);
-                const int kk = i / n, p = i % n;
-                const int ci = xe ? (e == 0 ? 0 : d.nx - 1) : p;
-                const int cj = xe ? p : (e == 2 ? 0 : d.ny - 1);
-                c1[u] = load_direct(d.ah, d.ahu, d.ahv, d.bed, d.pitch, ci, cj);
-                c2[u] = load_direct(in2, in2 + d.plane, in2 + 2 * d.plane, d.bed, d.pitch, ci, cj);
-                const long long o = edge_slot(e, kk, p, len);
-                g[u][0] = lg1[o]; g[u][1] = lg1[o + 1];
-                g[u][2] = lg2[o]; g[u][3] = lg2[o + 1];
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                if (u == 1 && i0 + (int)blockDim.x >= 2 * n) break;
-                s1 = s1 + eta_rev_one(d, eta1, c1[u], g[u][0], g[u][1], sgn, xe);
-                s2 = s2 + eta_rev_one(d, eta2, c2[u], g[u][2], g[u][3], sgn, xe);
-            }
+        const int n = e < 2 ? d.ny : d.nx;
+#pragma unroll 4
+        for (int i = threadIdx.x; i < 2 * n; i += 1024) {
+            const long long o = edge_slot(e, i >= n, i >= n ? i - n : i, len);
+            s1 = s1 + eta1[o];
+            s2 = s2 + eta2[o];
         }
     }
     *acc1 = s1;
@@ -781,8 +743,7 @@ struct DtArgs {
     const double* hist;
     const double* part_dt;      // 2 x nbody partial sums of d L / d dt
     int nbody;
-    const double* in2;          // U* (the stage-2 input)
-    const double* edge_lg;
+    const double* edge_eta;     // of stage 1, then of stage 2
     int edge_len;
     const double* pval;
     const long long* pidx;
@@ -796,8 +757,7 @@ __device__ __forceinline__ void dt_rev(const DtArgs& A) {
     const double* hist = A.hist;
     const double* part_dt = A.part_dt;
     const int nbody = A.nbody;
-    const double* in2 = A.in2;
-    const double* edge_lg = A.edge_lg;
+    const double* edge_eta = A.edge_eta;
     const int edge_len = A.edge_len;
     const double* pval = A.pval;
     const long long* pidx = A.pidx;
@@ -807,7 +767,7 @@ __device__ __forceinline__ void dt_rev(const DtArgs& A) {
     __shared__ double red[3][1024];
     __shared__ double sv[1024];
     __shared__ long long si[1024];
-    __shared__ double tide[4];   // eta(t), eta(t + dt), eta'(t), eta'(t + dt)
+    __shared__ double tide[2];   // eta'(t), eta'(t + dt)
     const double t = hist[0], dt = hist[1];
     // The kernel is bound by dependent memory round trips: each loop below
     // issues four elements' loads before it waits, and adds or compares them
@@ -843,45 +803,56 @@ __device__ __forceinline__ void dt_rev(const DtArgs& A) {
     sv[threadIdx.x] = best;
     si[threadIdx.x] = bi;
     const int w = threadIdx.x / WAVE;
-    if (w < 4) {
-        const double tw = (w & 1) ? t + dt : t;
-        const double v = w < 2 ? tidal_eta(d, tw) : adj::tidal_deta(d, tw);
+    if (w < 2) {
+        const double v = adj::tidal_deta(d, w ? t + dt : t);
         if (threadIdx.x % WAVE == 0) tide[w] = v;
     }
+    // d L / d eta_tidal of stage 1 (at t) and of stage 2 (at t + dt)
+    eta_parts(d, edge_eta, edge_eta + edge_slot(4, 0, 0, edge_len), edge_len, &red[1][threadIdx.x], &red[2][threadIdx.x]);
     __syncthreads();
-    // d L / d eta_tidal of stage 1 (input A = d.ah, at t) and stage 2 (input B = in2, at t + dt)
-    eta_parts(d, tide[0], tide[1], in2, edge_lg, edge_lg + edge_slot(4, 0, 0, edge_len), edge_len, &red[1][threadIdx.x],
-              &red[2][threadIdx.x]);
-    __syncthreads();
-    for (int s = 512; s > 0; s >>= 1) {
+    // a tree over the workgroup: its upper levels in LDS, the last wavefront's
+    // by lane shuffles
+    auto later = [](double v, long long x, double& best, long long& bi) {
+        if (v > best || (v == best && x >= 0 && (bi < 0 || x < bi))) {
+            best = v;
+            bi = x;
+        }
+    };
+    for (int s = 512; s >= WAVE; s >>= 1) {
         if (threadIdx.x < s) {
             for (int q = 0; q < 3; ++q) red[q][threadIdx.x] = red[q][threadIdx.x] + red[q][threadIdx.x + s];
-            const double v = sv[threadIdx.x + s];
-            const long long x = si[threadIdx.x + s];
-            if (v > sv[threadIdx.x] || (v == sv[threadIdx.x] && x >= 0 && (si[threadIdx.x] < 0 || x < si[threadIdx.x]))) {
-                sv[threadIdx.x] = v;
-                si[threadIdx.x] = x;
-            }
+            later(sv[threadIdx.x + s], si[threadIdx.x + s], sv[threadIdx.x], si[threadIdx.x]);
         }
         __syncthreads();
     }
+    if (threadIdx.x >= WAVE) return;
+    double r0 = red[0][threadIdx.x], r1 = red[1][threadIdx.x], r2 = red[2][threadIdx.x];
+    double ms = sv[threadIdx.x];
+    long long mi = si[threadIdx.x];
+    for (int s = WAVE / 2; s > 0; s >>= 1) {
+        r0 = r0 + __shfl_down(r0, s, WAVE);
+        r1 = r1 + __shfl_down(r1, s, WAVE);
+        r2 = r2 + __shfl_down(r2, s, WAVE);
+        const double v = __shfl_down(ms, s, WAVE);
+        const long long x = __shfl_down(mi, s, WAVE);
+        later(v, x, ms, mi);
+    }
     if (threadIdx.x != 0) return;
     const bool recomputed = hist[2] != 0.0;
-    const double lam_t1 = scal[0] + red[2][0] * tide[3];   // stage 2 ran at t + dt
-    const double gdt = red[0][0] + lam_t1 + scal[1];
-    double lam_t = lam_t1 + red[1][0] * tide[2];
+    const double lam_t1 = scal[0] + r2 * tide[1];   // stage 2 ran at t + dt
+    const double gdt = r0 + lam_t1 + scal[1];
+    double lam_t = lam_t1 + r1 * tide[0];
     double carry = 0.0;
     const double dt_max = d.t_end - t;
     if (d.dt_fixed > 0.0) {
         if (!(d.dt_fixed < dt_max)) lam_t -= gdt;           // dt = t_end - t
     } else if (recomputed) {
-        const double ms = sv[0];
         double dc = ms > 0.0 ? d.cfl / ms : d.cfl * dmin(d.dx, d.dy) / sqrt(d.g * DRY_TOLERANCE);
         dc = dc * d.ssp_coeff;
         if (!(dc < dt_max)) {
             lam_t -= gdt;                                    // dt = t_end - t
-        } else if (ms > 0.0 && si[0] >= 0) {                 // dt = cfl ssp / max speed
-            const long long idx = si[0];
+        } else if (ms > 0.0 && mi >= 0) {                    // dt = cfl ssp / max speed
+            const long long idx = mi;
             const long long k = (idx / d.nx) * d.pitch + idx % d.nx;
             const double l0 = lam[k], l1 = lam[d.plane + k], l2 = lam[2 * d.plane + k];
             const double lms = gdt * (-(d.cfl * d.ssp_coeff) / (ms * ms));
@@ -1005,7 +976,7 @@ struct rkg_adjoint {
     double* part;               // part_dt (2 x body blocks), argmax values
     long long* part_idx;        // argmax cells
     double* scal;               // adjoint of the clock and of a reused dt
-    double* edge_lg;            // tidal ghost adjoints of stage 1, then stage 2 (edge_slot)
+    double* edge_eta;           // edge_eta of stage 1, then of stage 2 (edge_slot)
     int edge_len;
     double* loss_dev;
     double* loss_host;
@@ -1200,8 +1171,8 @@ int create_session(rkg_grid* g, int nsteps, int K, int ng, const int* gauge_i, c
     a->edge_len = std::max(g->cfg.nx, g->cfg.ny);
     if (e == hipSuccess)
         e = hipMalloc((void**)&a->part, (size_t)(3 * body_blocks(g)) * sizeof(double));   // part_dt, argmax values
-    if (e == hipSuccess) e = hipMalloc((void**)&a->edge_lg, 2 * (size_t)edge_slot(4, 0, 0, a->edge_len) * sizeof(double));
-    if (e == hipSuccess) e = hipMemset(a->edge_lg, 0, 2 * (size_t)edge_slot(4, 0, 0, a->edge_len) * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc((void**)&a->edge_eta, 2 * (size_t)edge_slot(4, 0, 0, a->edge_len) * sizeof(double));
+    if (e == hipSuccess) e = hipMemset(a->edge_eta, 0, 2 * (size_t)edge_slot(4, 0, 0, a->edge_len) * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&a->part_idx, (size_t)body_blocks(g) * sizeof(long long));
     if (e == hipSuccess) e = hipMalloc((void**)&a->scal, 2 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&a->loss_dev, sizeof(double));
@@ -1270,7 +1241,7 @@ void rkg_adjoint_destroy(rkg_adjoint** pa) {
     for (void* p : {(void*)a->gi, (void*)a->gj, (void*)a->gw, (void*)a->cell_start, (void*)a->cell_gauges,
                     (void*)a->cell_w, (void*)a->cell_pos, (void*)a->tgt, (void*)a->eta, (void*)a->ckpt, (void*)a->ckpt_ctrl,
                     (void*)a->ws, (void*)a->lam, (void*)a->hist, (void*)a->loss_dev, (void*)a->part,
-                    (void*)a->part_idx, (void*)a->scal, (void*)a->edge_lg, (void*)a->ws_alt, (void*)a->hist_alt})
+                    (void*)a->part_idx, (void*)a->scal, (void*)a->edge_eta, (void*)a->ws_alt, (void*)a->hist_alt})
         if (p) (void)hipFree(p);
     if (a->rstream) (void)hipStreamDestroy(a->rstream);
     for (hipEvent_t ev : a->seg_ev)
@@ -1535,7 +1506,7 @@ AdjStage stage_args(rkg_adjoint* a, int k, int stage, const BwdPlan& pl) {
         st.part_dt = a->part + nb;
         st.pval = nullptr;
         st.pidx = nullptr;
-        st.edge_lg = a->edge_lg + pl.edge_size;
+        st.edge_eta = a->edge_eta + pl.edge_size;
     } else {            // input U^n (A_k)
         st.d = stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1));
         st.un = nullptr;
@@ -1545,7 +1516,7 @@ AdjStage stage_args(rkg_adjoint* a, int k, int stage, const BwdPlan& pl) {
         st.part_dt = a->part;
         st.pval = pl.cfl_dt ? a->part + 2 * nb : nullptr;
         st.pidx = pl.cfl_dt ? a->part_idx : nullptr;
-        st.edge_lg = a->edge_lg;
+        st.edge_eta = a->edge_eta;
     }
     return st;
 }
@@ -1556,8 +1527,7 @@ DtArgs dt_args(rkg_adjoint* a, int k, const AdjStage& st1, const BwdPlan& pl) {
     A.hist = st1.hist;
     A.part_dt = a->part;
     A.nbody = pl.nb;
-    A.in2 = wsB(a, k);
-    A.edge_lg = a->edge_lg;
+    A.edge_eta = a->edge_eta;
     A.edge_len = a->edge_len;
     A.pval = a->part + 2 * pl.nb;
     A.pidx = a->part_idx;
