@@ -192,10 +192,7 @@ int launch_generic(rkg_grid* g, int n, int mode, double tlim) {
             hipLaunchKernelGGL(k_euler_finish, dim3(sweep_blocks((long long)d.nx * d.ny)), dim3(256), 0, g->stream, d, g->parity);
         }
         g->parity ^= 1;
-        if (g->gauges) {
-            int rc = gauges_after_step(g, g->parity);
-            if (rc) return rc;
-        }
+        gauges_after_step(g, g->parity, BudgetArgs{});
     }
     HIP_TRY(hipGetLastError());
     return RKG_OK;
@@ -260,14 +257,10 @@ int launch_steps_now(rkg_grid* g, int n, int mode, double tlim) {
         launch_stage<1>(g, d, ntiles, mode, tlim);
         if (g->prof) HIP_TRY(hipEventRecord(g->ev[1], g->stream));
         launch_stage<2>(g, d, ntiles, mode, tlim);
-        if (d.mpart)
-            hipLaunchKernelGGL(k_budget, dim3(1), dim3(256), 0, g->stream, g->ctrl, g->parity, d.mpart, ntiles, area,
-                               rain, d.spart);
+        const BudgetArgs budget{g->ctrl, g->parity, d.mpart, ntiles, area, rain, d.spart};
         g->parity ^= 1;
-        if (g->gauges) {
-            int rc = gauges_after_step(g, g->parity);
-            if (rc) return rc;
-        }
+        if (!gauges_after_step(g, g->parity, budget) && d.mpart)
+            hipLaunchKernelGGL(k_budget, dim3(1), dim3(256), 0, g->stream, budget);
         if (g->prof) {
             float a = 0.f, b = 0.f;
             HIP_TRY(hipEventRecord(g->ev[2], g->stream));

@@ -11,6 +11,7 @@
 #include "../../include/rakali_amd.h"
 #include "gauge_eval.hpp"
 #include "rkg_internal.hpp"
+#include "stage_kernels.hpp"
 
 namespace rk {
 
@@ -73,31 +74,41 @@ __global__ __launch_bounds__(256) void k_gauges_now(GridDesc d, GaugeTable t, do
 
 // After a step: slot p holds the state's clock.  A record is appended when
 // the step ran and (interval <= 0 or t >= next), and next advances by the
-// interval (write_gauges, rki_driver.F90:777-800).  One workgroup: thread 0
-// decides, then all threads write the record.
+// interval (write_gauges, rki_driver.F90:777-800).  Workgroup 0: thread 0
+// decides, then all threads write the record.  Workgroup 1, where the run keeps
+// a mass budget, adds the step's (701x515 forced, us a step: 10.4 as two
+// launches, 8 as one): it updates the budget of slot p, of which the record
+// reads only the clock.
 __global__ __launch_bounds__(256) void k_gauges_record(GridDesc d, GaugeTable t, const CtrlSlot* ctrl, int p,
                                                        double interval, double* series, int* count, double* next,
-                                                       int cap) {
+                                                       int cap, BudgetArgs budget) {
+    if (blockIdx.x == 1) {
+        step_budget(budget);
+        return;
+    }
     __shared__ int slot;
+    // the first 256 stations are evaluated while thread 0 waits for its loads
+    double e = 0.0, u = 0.0, v = 0.0;
+    if ((int)threadIdx.x < t.n) gauge_value(d, t, threadIdx.x, e, u, v);
     if (threadIdx.x == 0) {
         slot = -1;
-        const CtrlSlot c = ctrl[p];
-        if (c.active && (interval <= 0.0 || c.t >= *next)) {
-            const int k = *count;
+        const CtrlClock c = ctrl[p];
+        const double due = *next;
+        const int k = *count;
+        if (c.active && (interval <= 0.0 || c.t >= due)) {
             if (k < cap) {   // the host drains before the buffer can fill
                 slot = k;
                 *count = k + 1;
                 series[(long long)k * (1 + 3 * t.n)] = c.t;
             }
-            if (interval > 0.0) *next = *next + interval;
+            if (interval > 0.0) *next = due + interval;
         }
     }
     __syncthreads();
     if (slot < 0) return;
     double* rec = series + (long long)slot * (1 + 3 * t.n) + 1;
     for (int g = threadIdx.x; g < t.n; g += 256) {
-        double e, u, v;
-        gauge_value(d, t, g, e, u, v);
+        if (g >= 256) gauge_value(d, t, g, e, u, v);
         rec[g] = e;
         rec[t.n + g] = u;
         rec[2 * t.n + g] = v;
@@ -183,14 +194,14 @@ int gauges_drain(rkg_grid* g) {
     return RKG_OK;
 }
 
-int gauges_after_step(rkg_grid* g, int p) {
+bool gauges_after_step(rkg_grid* g, int p, const BudgetArgs& budget) {
     GaugeState* s = g->gauges;
-    if (!s->recording || s->n_local == 0) return RKG_OK;
+    if (!s || !s->recording || s->n_local == 0) return false;
     const GridDesc d = make_desc(g);
-    hipLaunchKernelGGL(k_gauges_record, dim3(1), dim3(256), 0, g->stream, d, table_of(s), g->ctrl, p, s->interval,
-                       s->d_series, s->d_count, s->d_next, s->cap);
+    hipLaunchKernelGGL(k_gauges_record, dim3(budget.mpart ? 2 : 1), dim3(256), 0, g->stream, d, table_of(s), g->ctrl, p,
+                       s->interval, s->d_series, s->d_count, s->d_next, s->cap, budget);
     s->pending += 1;
-    return RKG_OK;
+    return true;
 }
 
 void gauges_free(rkg_grid* g) {

@@ -113,7 +113,9 @@ bool station_weights(const rkg_config& c, double x, double y, int* c0, int* j0, 
 
 long long gauges_room(const rkg_grid* g);
 int gauges_drain(rkg_grid* g);
-int gauges_after_step(rkg_grid* g, int p);
+// The record after a step together with its mass budget (if it has one);
+// false when no gauges are recorded and nothing was launched.
+bool gauges_after_step(rkg_grid* g, int p, const BudgetArgs& budget);
 void gauges_free(rkg_grid* g);
 
 inline double* field_ptr(rkg_grid* g, int field) {

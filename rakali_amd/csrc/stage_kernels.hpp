@@ -259,11 +259,15 @@ __global__ void k_speed_reset(CtrlSlot* ctrl, int p) {
 // sponge on, `spart` holds the per-tile sums of its change of h and
 // mass_src += 0.5 sum area (accumulate_sponge_mass_src, :608-657, at :787
 // and :814).  Slot 1-p is the step's result.
-__global__ __launch_bounds__(256) void k_budget(CtrlSlot* ctrl, int p, const double* mpart, int ntiles,
-                                                double area, const double* rain, const double* spart) {
+__device__ __forceinline__ void step_budget(const BudgetArgs& b) {
     __shared__ double red[4][256];
+    CtrlSlot* ctrl = b.ctrl;
+    const int p = b.p, ntiles = b.ntiles;
+    const double *mpart = b.mpart, *rain = b.rain, *spart = b.spart;
+    const double area = b.area;
     if (!ctrl[1 - p].active) return;
     double a[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
     for (int i = threadIdx.x; i < ntiles; i += 256) {
         a[0] = a[0] + mpart[i];
         a[1] = a[1] + mpart[ntiles + i];
@@ -294,6 +298,8 @@ __global__ __launch_bounds__(256) void k_budget(CtrlSlot* ctrl, int p, const dou
         q->mass_src = src;
     }
 }
+
+__global__ __launch_bounds__(256) void k_budget(BudgetArgs b) { step_budget(b); }
 
 // Max CFL speed over all cells, whose states load(offset, h, hu, hv) gives;
 // the result is valid in thread 0.  Workgroups of 256 threads, cell after cell

@@ -41,6 +41,17 @@ struct alignas(128) CtrlSlot : CtrlClock {
     alignas(128) unsigned long long speed[SPEED_WAYS * SPEED_STRIDE];
 };
 
+// Arguments of a step's mass budget (k_budget); mpart null: none.
+struct BudgetArgs {
+    CtrlSlot* ctrl;
+    int p;
+    const double* mpart;
+    int ntiles;
+    double area;
+    const double* rain;
+    const double* spart;
+};
+
 // Optional source terms of the stage kernels (template bit mask).
 constexpr int FEAT_FORCING = 1;   // surface forcing, rki_kernel_fused.F90:268-289
 constexpr int FEAT_SPONGE = 2;    // sponge relaxation, rki_kernel_sponge.F90:16-88
