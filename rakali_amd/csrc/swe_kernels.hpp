@@ -363,12 +363,14 @@ constexpr int OWN = WAVE - 2 * HALO;
 // last block holding at least two cells: the halo of the block before it
 // then ends inside the grid, so a ghost cell (which may depend on what the
 // edge's own tile overwrites, see chapman_ghost) is read by the edge's own
-// tile only.  With w = 1 the block before the last one is empty.
+// tile only.  Blocks of one cell, which grids with such edges do not use, stay
+// that (a last block of two would last as long as two rows: 130x97, 25 us a
+// step, 21 so).
 __host__ __device__ __forceinline__ void tile_range(int n, int w, int s, int& lo, int& hi) {
     const int nb = (n + w - 1) / w;
     lo = s * w;
     hi = lo + w < n ? lo + w : n;
-    if (nb >= 2 && n - (nb - 1) * w == 1) {
+    if (w >= 2 && nb >= 2 && n - (nb - 1) * w == 1) {
         if (s == nb - 1) lo = n - 2;
         if (s == nb - 2) hi = n - 2;
     }
