@@ -477,7 +477,7 @@ struct XRows {
 // TX: a west or east edge is tidal (see k_adj_y's TY).
 //
 // Bound by latency, as adj_y: the next row is loaded into LDS while a row is
-// computed.  1024^2: 78 us when each row loaded its own, 54 now,
+// computed.  1024^2: 78 us when each row loaded its own, 50 now,
 // of which its 138 MB take 30; 4096 x 1024: 144 us, at 3.8 TB/s.
 template <bool HLLC, int STAGE, bool TX>
 __device__ __forceinline__ void adj_x(const AdjStage& a, XRows& rows, int blk) {

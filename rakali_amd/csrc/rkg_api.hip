@@ -100,6 +100,8 @@ namespace {
 bool valid(const rkg_grid* g) { return g != nullptr && g->magic == GRID_MAGIC; }
 
 int refresh_speed(rkg_grid* g) {
+    const int rc = refuse_capture(g->stream);
+    if (rc) return rc;
     GridDesc d = make_desc(g);
     hipLaunchKernelGGL(k_speed_reset, dim3(1), dim3(64), 0, g->stream, g->ctrl, g->parity);
     hipLaunchKernelGGL(k_init_speed, dim3(sweep_blocks((long long)g->cfg.nx * g->cfg.ny)), dim3(256), 0, g->stream, d, g->parity);
@@ -389,6 +391,14 @@ hipError_t rk::plane_from_host(HostStage& st, double* plane, size_t pitch, const
             e = hipMemcpy2DAsync(plane + j * pitch, pitch * W, half, nx * W, nx * W, n, hipMemcpyHostToDevice, stream);
     }
     return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+}
+
+int rk::refuse_capture(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(stream, &st));
+    if (st == hipStreamCaptureStatusNone) return RKG_OK;
+    set_error("the first step after an upload cannot be captured");
+    return RKG_ERR_HIP;
 }
 
 int rk::validate_config(const rkg_config* c) { return check_config(c); }

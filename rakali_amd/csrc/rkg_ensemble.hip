@@ -174,6 +174,8 @@ int build_tables(rkg_ensemble* e) {
 int refresh_speeds(rkg_ensemble* e) {
     for (int m = 0; m < e->n; ++m) {
         if (!e->speed_stale[m]) continue;
+        const int rc = refuse_capture(e->stream);
+        if (rc) return rc;
         const GridDesc d = ens_desc(e, m);
         hipLaunchKernelGGL(k_speed_reset, dim3(1), dim3(64), 0, e->stream, d.ctrl, e->parity);
         hipLaunchKernelGGL(k_init_speed, dim3(sweep_blocks((long long)d.nx * d.ny)), dim3(256), 0, e->stream, d, e->parity);

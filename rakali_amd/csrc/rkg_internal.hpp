@@ -100,6 +100,11 @@ void grid_release(rkg_grid* g);
 // RKG_OK or an error code with the message set.
 int validate_config(const rkg_config* c);
 
+// RKG_ERR_HIP (with the message set) while `stream` is being captured: the
+// speed maximum of an uploaded state is taken once, when the host sees the
+// upload, and would otherwise be left to the captured graph's launch.
+int refuse_capture(hipStream_t stream);
+
 inline double* plane_ptr(rkg_grid* g, int k) { return g->buf + (size_t)k * g->plane; }
 
 // Gauge recording around the step launches (rkg_gauges.hip): the steps one

@@ -56,3 +56,27 @@ def test_ensemble_members_share_the_stage():
         e.set_field(m, "hv", w)
     for m, w in reversed(list(enumerate(want))):
         assert np.array_equal(e.get_field(m, "hv"), w)
+
+
+def test_first_step_after_an_upload_is_not_captured():
+    """Refused under capture, before anything is queued, and run as ever
+    afterwards; a later step may be captured and replayed."""
+    import torch
+    from conftest import make_grid
+    from rakali_amd import scenarios as S
+    from rakali_amd._lib import RkgError
+    scn = S.wetdry_islands(nx=75, ny=33, steps=4)
+    want = make_grid(scn)
+    want.step(4)
+    s = torch.cuda.Stream()
+    g = make_grid(scn, stream=s.cuda_stream)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        torch.zeros(1, device="cuda")
+        with pytest.raises(RkgError):
+            g.step(1)
+    g.step(4)
+    for k in ("h", "hu", "hv"):
+        assert np.array_equal(g.get_field(k), want.get_field(k))
+    assert g.clock == want.clock
