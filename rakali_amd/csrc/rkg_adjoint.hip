@@ -477,14 +477,19 @@ struct XRows {
 // TX: a west or east edge is tidal (see k_adj_y's TY).
 //
 // Bound by latency, as adj_y: the next row is loaded into LDS while a row is
-// computed.  1024^2: 78 us when each row loaded its own, 50 now,
+// computed.  1024^2: 78 us when each row loaded its own, 44 now,
 // of which its 138 MB take 30; 4096 x 1024: 144 us, at 3.8 TB/s.
 template <bool HLLC, int STAGE, bool TX>
 __device__ __forceinline__ void adj_x(const AdjStage& a, XRows& rows, int blk) {
     const GridDesc& d = a.d;
     const int lane = threadIdx.x;
-    const int nstr = (d.nx + AW - 1) / AW;
-    const int sx = blk % nstr, sy = blk / nstr;
+    const int nstr = (d.nx + AW - 1) / AW, nrow = (d.ny + XROWS - 1) / XROWS;
+    // the edge strips, whose ghost columns take longer, first (1024^2: 45 us, 49
+    // in the order of the columns)
+    int sx, sy;
+    if (nstr < 3) { sx = blk % nstr; sy = blk / nstr; }
+    else if (blk < 2 * nrow) { sx = blk & 1 ? nstr - 1 : 0; sy = blk >> 1; }
+    else { const int q = blk - 2 * nrow; sx = 1 + q % (nstr - 2); sy = q / (nstr - 2); }
     int c0, c1;
     tile_range(d.nx, AW, sx, c0, c1);
     const int r0 = sy * XROWS, r1 = min(r0 + XROWS, d.ny);
@@ -898,7 +903,7 @@ template <int STAGE, bool HLLC, bool REC>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_step_batch(
     const GridDesc* __restrict__ descs, const RecTile* __restrict__ tiles, const int* __restrict__ parity) {
     __shared__ TileRing ring;
-    const RecTile t = tiles[blockIdx.x];
+    const RecTile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
     const GridDesc& d = descs[t.member];
     stage_tile<STAGE, HLLC, true, REC, RecTileOf>(d, ring, parity[t.member], MODE_STEP, d.t_end, RecTileOf{t});
 }
@@ -926,7 +931,7 @@ template <bool HLLC, int STAGE>
 __global__ __launch_bounds__(WAVE) void k_adj_y_batch(const AdjStage* __restrict__ as,
                                                      const BlockRef* __restrict__ tab) {
     __shared__ alignas(16) YRows rows;
-    const BlockRef r = tab[blockIdx.x];
+    const BlockRef r = tab[xcd_tile(blockIdx.x, gridDim.x)];
     adj_y<HLLC, STAGE, true>(as[r.member], rows, r.blk);
 }
 
@@ -1045,6 +1050,10 @@ void launch_rec(rkg_grid* g, const GridDesc& d, int p, hipStream_t st) {
         hipLaunchKernelGGL((k_stage<STAGE, false, true, true>), dim3(ntiles), dim3(WAVE), 0, st, d, p, MODE_STEP, tlim);
 }
 
+// Workgroups of k_adj_x, and how many of them, the first, hold an edge strip.
+int x_blocks(int nx, int ny) { return ((nx + AW - 1) / AW) * ((ny + XROWS - 1) / XROWS); }
+int x_edge_blocks(int nx, int ny) { return std::min(x_blocks(nx, ny), 2 * ((ny + XROWS - 1) / XROWS)); }
+
 // The stage's face reverse: k_adj_y then k_adj_x (both add into lam_in and
 // grad_b).
 template <bool HLLC, int STAGE>
@@ -1053,7 +1062,7 @@ void launch_faces(rkg_grid* g, const AdjStage& st) {
     const bool tx = bc[0] == BC_TIDAL || bc[1] == BC_TIDAL, ty = bc[2] == BC_TIDAL || bc[3] == BC_TIDAL;
     const int nx = g->cfg.nx, ny = g->cfg.ny;
     const int yblocks = ((nx + WAVE - 1) / WAVE) * ((ny + st.ty - 1) / st.ty);
-    const int xblocks = ((nx + AW - 1) / AW) * ((ny + XROWS - 1) / XROWS);
+    const int xblocks = x_blocks(nx, ny);
     if (ty)
         hipLaunchKernelGGL((k_adj_y<HLLC, STAGE, true>), dim3(yblocks), dim3(WAVE), 0, g->stream, st);
     else
@@ -1773,7 +1782,7 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
     };
 
     // block tables
-    std::vector<BlockRef> tb, ty, tx, tseed;
+    std::vector<BlockRef> tb, ty, tx, txr, tseed;
     std::vector<RecTile> trec;
     for (int m = 0; m < n; ++m) {
         rkg_grid* g = as[m]->g;
@@ -1782,14 +1791,16 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
         for (int b = 0; b < nb; ++b) tb.push_back(BlockRef{m, b, nb, 0});
         const int yb = ((nx + WAVE - 1) / WAVE) * ((ny + pl[m].tile_rows - 1) / pl[m].tile_rows);
         for (int b = 0; b < yb; ++b) ty.push_back(BlockRef{m, b, yb, 0});
-        const int xb = ((nx + AW - 1) / AW) * ((ny + XROWS - 1) / XROWS);
-        for (int b = 0; b < xb; ++b) tx.push_back(BlockRef{m, b, xb, 0});
+        // the edge strips of all members first (see adj_x)
+        const int xb = x_blocks(nx, ny), xe = x_edge_blocks(nx, ny);
+        for (int b = 0; b < xb; ++b) (b < xe ? tx : txr).push_back(BlockRef{m, b, xb, 0});
         if (as[m]->ng > 0) {
             const int sb = (as[m]->ncells + 255) / 256;
             for (int b = 0; b < sb; ++b) tseed.push_back(BlockRef{m, b, sb, 0});
         }
         batch_tiles(replay_desc(as[m], 0), m, trec);
     }
+    tx.insert(tx.end(), txr.begin(), txr.end());
     // per global step: replay descriptors (stage 1, 2), replay parities, and
     // the reverse arguments (stage 2, stage 1, seeds, dt), n of each
     const size_t szGD = sizeof(GridDesc), szAS = sizeof(AdjStage), szSA = sizeof(SeedArgs), szDA = sizeof(DtArgs);
