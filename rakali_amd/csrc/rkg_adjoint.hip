@@ -240,14 +240,8 @@ __device__ __forceinline__ void ghost_x_rev(const GridDesc& d, double eta, int x
                    west ? -1.0 : 1.0, true, lg, lm, li, leta);
 }
 
-__device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, int x, int y, const adj::C4& lg, int& mrow,
-                                            int& irow, adj::C4& lm, adj::C4& li, double* leta) {
-    const bool south = y < 0;
-    const int kk = south ? (-y - 1) : (y - d.ny);
-    mrow = south ? kk : (d.ny - 1 - kk);
-    irow = south ? 0 : (d.ny - 1);
-    const Cell mir = load_direct(d.ah, d.ahu, d.ahv, d.bed, d.pitch, x, mrow);
-    const Cell in0 = load_direct(d.ah, d.ahu, d.ahv, d.bed, d.pitch, x, irow);
+__device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, bool south, const Cell& mir, const Cell& in0,
+                                            const adj::C4& lg, adj::C4& lm, adj::C4& li, double* leta) {
     lm = adj::C4{0, 0, 0, 0};
     li = adj::C4{0, 0, 0, 0};
     adj::ghost_rev(d.bc[south ? 2 : 3], d.g, eta, d.inflow_velocity, d.clamped_elevation, mir, in0,
@@ -255,11 +249,11 @@ __device__ __forceinline__ void ghost_y_rev(const GridDesc& d, double eta, int x
 }
 
 // Two LDS rows of the 11 planes over 64 columns (the twelfth is a spare: two
-// planes make one load), and two accumulators that wait for their ghost rows:
-// the south ghost rows', then row ny-2's with its old values.
+// planes make one load), and what waits for ghost rows: the south ghost rows'
+// accumulators, then row ny-2's old values, accumulator and cell.
 struct YRows {
     double v[2][ADJ_PLANES + 1][WAVE];
-    double kept[8][WAVE];
+    double kept[12][WAVE];
 };
 
 // Reverse of the y faces and y slopes of one stage (and the south / north
@@ -351,11 +345,12 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
     adj::states_fwd(v0, v1, v2, lo_tmp, hi_r);
     adj::S3 llo_r{0.0, 0.0, 0.0};        // adjoint of the y lo-state of row r (from face r - 1/2)
 
-    // Adjoint lg of ghost row rho onto rows mrow and irow.
-    auto fold = [&](int rho, const Acc& ghost, int& mrow, int& irow, adj::C4& lm, adj::C4& li) {
+    // Adjoint of ghost row rho onto its mirror row (cell mir) and the first
+    // interior row (cell in0).
+    auto fold = [&](int rho, const Acc& ghost, const Cell& mir, const Cell& in0, adj::C4& lm, adj::C4& li) {
         const adj::C4 lg = c4(ghost);
         double leta = 0.0;
-        ghost_y_rev(d, eta, xs, rho, lg, mrow, irow, lm, li, &leta);
+        ghost_y_rev(d, eta, rho < 0, mir, in0, lg, lm, li, &leta);
         const int e = rho < 0 ? 2 : 3;
         if (TY && xin && d.bc[e] == BC_TIDAL)
             a.edge_eta[edge_slot(e, rho < 0 ? -rho - 1 : rho - ny, x, a.edge_len)] = leta;
@@ -400,15 +395,14 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
             return Acc{rows.kept[q][lane], rows.kept[q + 1][lane], rows.kept[q + 2][lane], rows.kept[q + 3][lane]};
         };
         adj::C4 lm, li;
-        int mrow, irow;
         if (j0 == 0 && r <= 1) {
             if (r == -1 || r == 0) {   // row -2, -1 complete
                 keep(4 * (r + 1), acc[0].h, acc[0].hu, acc[0].hv, acc[0].b);
-            } else if (r == 1) {       // acc[0], acc[1] are rows 0 and 1
-                fold(-2, kept(0), mrow, irow, lm, li);
+            } else if (r == 1) {       // acc[0], acc[1] and v0, v1 are rows 0 and 1
+                fold(-2, kept(0), v1, v0, lm, li);
                 add(acc[1], lm);       // the mirror row is 1, the first row 0
                 add(acc[0], li);
-                fold(-1, kept(4), mrow, irow, lm, li);
+                fold(-1, kept(4), v0, v0, lm, li);
                 add(acc[0], lm);
                 add(acc[0], li);
             }
@@ -425,13 +419,15 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
         if (waits) {
             keep(0, old.h, old.hu, old.hv, old.b);
             keep(4, acc[0].h, acc[0].hu, acc[0].hv, acc[0].b);
+            keep(8, v0.h, v0.hu, v0.hv, v0.b);
         }
-        if (j1 == ny && r == ny) {   // acc[0..2] are rows ny-1, ny, ny+1
+        if (j1 == ny && r == ny) {   // acc[0..2] are rows ny-1, ny, ny+1, v0 is row ny-1
             Acc last = kept(4);      // row ny-2
-            fold(ny, acc[1], mrow, irow, lm, li);
+            const Acc cell = kept(8);
+            fold(ny, acc[1], v0, v0, lm, li);
             add(acc[0], lm);
             add(acc[0], li);
-            fold(ny + 1, acc[2], mrow, irow, lm, li);
+            fold(ny + 1, acc[2], Cell{cell.h, cell.hu, cell.hv, cell.b}, v0, lm, li);
             add(last, lm);
             add(acc[0], li);
             if (xin) put(ny - 2, c4(kept(0)), last);
