@@ -356,6 +356,7 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
             a.edge_eta[edge_slot(e, rho < 0 ? -rho - 1 : rho - ny, x, a.edge_len)] = leta;
     };
 
+    wait_loads();   // the rows of the first iteration
     for (int r = rs; r <= re; ++r) {
         // v0..v2 are rows r-1 .. r+1
         const double(*in)[WAVE] = rows.v[(r - rs) & 1];
@@ -521,6 +522,7 @@ __device__ __forceinline__ void adj_x(const AdjStage& a, XRows& rows, int blk) {
     const LaneSource l1 = edge_tile ? lane_source<true>(d, x) : lane_source<false>(d, x);
     const LaneSource l2 = edge_tile ? lane_source<true>(d, lane == 0 ? x - 1 : x + 1) : l1;
     const int i1 = min(max(l1.c - cb, 0), XCOLS - 1), i2 = min(max(l2.c - cb, 0), XCOLS - 1);
+    wait_loads();   // the first row
     for (int r = r0; r < r1; ++r) {
         const double* row = rows.v[(r - r0) & 1];
         auto cell_at = [&](int i) { return Cell{row[i], row[XCOLS + i], row[2 * XCOLS + i], row[3 * XCOLS + i]}; };

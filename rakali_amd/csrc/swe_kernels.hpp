@@ -215,6 +215,16 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// Orders the LDS writes of one wavefront's lanes before the reads of its other
+// lanes (and those reads before the next writes).  A wavefront's LDS accesses
+// are performed in order, so it is no instruction; it keeps the compiler from
+// moving them, which per lane it may (the addresses of two lanes differ).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Three rows of the march, (h + b, hu, hv, b, h) of the wavefront's 64
 // columns, and what the row below hands up: its high y state (h, hu, hv), the
 // part of its upper face that the row above takes (fh, fhu, fhv, a) and the
@@ -511,6 +521,7 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
         put(0, rc);
         put(1, rn);
         put(2, rnn);
+        wave_lds_order();
         hand_up(hi, Face{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, surf(1, lane) - surf(0, lane));
     }
     // a column of the grid for the lanes that own none: their loads of U^n are not used
@@ -659,7 +670,9 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
             }
             in_hbm(s.oh)[k] = h; in_hbm(s.ohu)[k] = hu; in_hbm(s.ohv)[k] = hv;
         }
+        wave_lds_order();
         put(sc, nxt);   // row j+3 takes the place of row j
+        wave_lds_order();
         const int free_slot = sc;
         sc = sn; sn = snn; snn = free_slot;
     }
