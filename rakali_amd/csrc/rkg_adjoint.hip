@@ -279,7 +279,7 @@ __device__ __forceinline__ void adj_y(const AdjStage& a, YRows& rows, int blk) {
     const int sx = blk % nstr, sy = blk / nstr;
     const int c0 = sx * WAVE;
     int j0, j1;
-    tile_range(d.ny, a.ty, sy, j0, j1);
+    tile_range(d.ny, a.ty, (d.ny + a.ty - 1) / a.ty, sy, j0, j1);
     const int x = c0 + lane;
     const bool xin = x < d.nx;   // lanes past the edge compute on the rows' padding, unwritten
     const int xs = xin ? x : d.nx - 1;
@@ -488,7 +488,7 @@ __device__ __forceinline__ void adj_x(const AdjStage& a, XRows& rows, int blk) {
     else if (blk < 2 * nrow) { sx = blk & 1 ? nstr - 1 : 0; sy = blk >> 1; }
     else { const int q = blk - 2 * nrow; sx = 1 + q % (nstr - 2); sy = q / (nstr - 2); }
     int c0, c1;
-    tile_range(d.nx, AW, sx, c0, c1);
+    tile_range(d.nx, AW, nstr, sx, c0, c1);
     const int r0 = sy * XROWS, r1 = min(r0 + XROWS, d.ny);
     const int x = c0 - 2 + lane;
     const bool own_col = x >= c0 && x < c1;
@@ -886,24 +886,14 @@ struct BlockRef {
     int member, blk, nblk, pad;
 };
 
-// A replay tile of one member (strip, segment, leader of its launch).
-struct RecTile {
-    int member, strip, seg, leader;
-};
-
-struct RecTileOf {
-    RecTile t;
-    __device__ int3 operator()(const GridDesc&) const { return make_int3(t.strip, t.seg, t.leader); }
-};
-
 // REC: recording (the replay of a sweep), else a step of the forward run.
 template <int STAGE, bool HLLC, bool REC>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(RKG_WAVES_PER_EU, 8))) void k_step_batch(
-    const GridDesc* __restrict__ descs, const RecTile* __restrict__ tiles, const int* __restrict__ parity) {
+    const GridDesc* __restrict__ descs, const BatchTile* __restrict__ tiles, const int* __restrict__ parity) {
     __shared__ TileRing ring;
-    const RecTile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
+    const BatchTile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
     const GridDesc& d = descs[t.member];
-    stage_tile<STAGE, HLLC, true, REC, RecTileOf>(d, ring, parity[t.member], MODE_STEP, d.t_end, RecTileOf{t});
+    stage_tile<STAGE, HLLC, true, REC, BatchTile>(d, ring, parity[t.member], MODE_STEP, d.t_end, t);
 }
 
 __global__ __launch_bounds__(256) void k_gauge_loss_batch(const LossArgs* __restrict__ la, int step) {
@@ -1040,7 +1030,7 @@ GridDesc stage_desc(rkg_adjoint* a, double* in, double* in2, double* out2) {
 
 template <int STAGE>
 void launch_rec(rkg_grid* g, const GridDesc& d, int p, hipStream_t st) {
-    const int ntiles = d.nstrips * d.nsegs;
+    const int ntiles = d.ntiles;
     const double tlim = g->cfg.t_end;
     if (g->cfg.use_hllc)
         hipLaunchKernelGGL((k_stage<STAGE, true, true, true>), dim3(ntiles), dim3(WAVE), 0, st, d, p, MODE_STEP, tlim);
@@ -1639,27 +1629,16 @@ int batch_tables(rkg_adjoint* a, size_t bytes) {
 
 // Rows per stage tile by the tiles of all members: a launch serves them
 // together (eight grids of 128..512 cells, us: replay stages 66 / 70 with
-// each grid's own rows, 44 / 47 with these).
-int batch_rows(int n, rkg_adjoint* const* as) {
-    return rows_for([=](int rows) {
+// each grid's own rows, 44 / 47 with these).  A height set by the caller stays.
+void set_batch_tiles(int n, rkg_adjoint* const* as, GridDesc* d) {
+    const int rows = rows_for([=](int r) {
         long long t = 0;
-        for (int m = 0; m < n; ++m) t += grid_tiles(as[m]->g->cfg.nx, as[m]->g->cfg.ny, rows);
+        for (int m = 0; m < n; ++m) t += grid_tiles(as[m]->g->cfg.nx, as[m]->g->cfg.ny, r);
         return t;
     }, 1);
-}
-
-// d with the batch's rows per tile; a height set by the caller stays.
-GridDesc batch_desc(const rkg_adjoint* a, GridDesc d, int rows) {
-    if (a->g->ty == 0) {
-        d.ty = rows;
-        d.nsegs = (d.ny + rows - 1) / rows;
-    }
-    return d;
-}
-
-// Member m's tiles, in the order and with the leader of its own launches.
-void batch_tiles(const GridDesc& d, int m, std::vector<RecTile>& t) {
-    for (int k = 0; k < d.nstrips * d.nsegs; ++k) t.push_back(RecTile{m, k % d.nstrips, k / d.nstrips, k == 0});
+    std::vector<int> ty(n);
+    for (int m = 0; m < n; ++m) ty[m] = as[m]->g->ty == 0 ? rows : d[m].ty;
+    set_launch_tiles(d, n, ty.data());
 }
 
 // The work of every stream before what the first stream queues next (to_first),
@@ -1696,29 +1675,30 @@ bool fwd_batchable(int n, rkg_adjoint* const* as) {
 // GPU ran them.  Every member's arithmetic is that of its own run.
 int fwd_batched(int n, rkg_adjoint* const* as) {
     const bool hllc = as[0]->g->cfg.use_hllc != 0;
-    const int nsteps = as[0]->nsteps, K = as[0]->K, rows = batch_rows(n, as);
+    const int nsteps = as[0]->nsteps, K = as[0]->K;
     hipStream_t S = as[0]->g->stream;
     std::vector<GridDesc> d(n);
-    std::vector<RecTile> tiles;
+    std::vector<BatchTile> tiles;
     std::vector<LossArgs> loss;
     std::vector<int> par(2 * n);
     int rc = RKG_OK;
     for (int m = 0; m < n && !rc; ++m) {
         rkg_grid* g = as[m]->g;
         if (g->speed_stale) rc = rkg_step(g, 0);   // make the control slot current
-        d[m] = batch_desc(as[m], make_desc(g), rows);
-        batch_tiles(d[m], m, tiles);
+        d[m] = make_desc(g);
         if (as[m]->ng > 0) loss.push_back(loss_args(as[m]));
         par[m] = g->parity;
         par[n + m] = g->parity ^ 1;
     }
     if (rc) return rc;
-    const size_t oT = al256(n * sizeof(GridDesc)), oL = oT + al256(tiles.size() * sizeof(RecTile)),
+    set_batch_tiles(n, as, d.data());
+    for (int m = 0; m < n; ++m) batch_tiles(d[m], m, tiles);
+    const size_t oT = al256(n * sizeof(GridDesc)), oL = oT + al256(tiles.size() * sizeof(BatchTile)),
                  oP = oL + al256((loss.size() + 1) * sizeof(LossArgs)), total = oP + al256(2 * n * sizeof(int));
     if ((rc = batch_tables(as[0], total))) return rc;
     char *host = as[0]->batch_host, *dev = as[0]->batch_dev;
     std::memcpy(host, d.data(), n * sizeof(GridDesc));
-    std::memcpy(host + oT, tiles.data(), tiles.size() * sizeof(RecTile));
+    std::memcpy(host + oT, tiles.data(), tiles.size() * sizeof(BatchTile));
     if (!loss.empty()) std::memcpy(host + oL, loss.data(), loss.size() * sizeof(LossArgs));
     std::memcpy(host + oP, par.data(), 2 * n * sizeof(int));
     hipEvent_t join = nullptr;
@@ -1726,7 +1706,7 @@ int fwd_batched(int n, rkg_adjoint* const* as) {
     hipError_t e = join_streams(n, as, join, true);
     if (e == hipSuccess) e = hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, S);
     const GridDesc* dd = (const GridDesc*)dev;
-    const RecTile* dt = (const RecTile*)(dev + oT);
+    const BatchTile* dt = (const BatchTile*)(dev + oT);
     const dim3 grid((unsigned)tiles.size()), block(WAVE);
     for (int k = 0; k < nsteps && !rc && e == hipSuccess; ++k) {
         if (k % K == 0)
@@ -1770,18 +1750,19 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
     // k_adj_y's rows too by the blocks of all members (us: 47 -> 41)
     long long yrows = 0;
     for (int m = 0; m < n; ++m) yrows += (long long)as[m]->g->cfg.ny * ((as[m]->g->cfg.nx + WAVE - 1) / WAVE);
-    const int adj_rows = adj_y_rows(yrows), replay_rows = batch_rows(n, as);
+    const int adj_rows = adj_y_rows(yrows);
     for (int m = 0; m < n && !rc; ++m) rc = bwd_begin(as[m], loss_scale, adj_rows, pl[m]);
     if (rc) return rc;
     for (int m = 0; m < n; ++m) use_set(as[m], 0);
     hipStream_t S = as[0]->g->stream;
-    auto replay_desc = [&](rkg_adjoint* a, int k) {
-        return batch_desc(a, stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1)), replay_rows);
-    };
+    // every step's replay has the tiles of these
+    std::vector<GridDesc> rec;
+    for (int m = 0; m < n; ++m) rec.push_back(make_desc(as[m]->g));
+    set_batch_tiles(n, as, rec.data());
 
     // block tables
     std::vector<BlockRef> tb, ty, tx, txr, tseed;
-    std::vector<RecTile> trec;
+    std::vector<BatchTile> trec;
     for (int m = 0; m < n; ++m) {
         rkg_grid* g = as[m]->g;
         const int nx = g->cfg.nx, ny = g->cfg.ny;
@@ -1796,7 +1777,7 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
             const int sb = (as[m]->ncells + 255) / 256;
             for (int b = 0; b < sb; ++b) tseed.push_back(BlockRef{m, b, sb, 0});
         }
-        batch_tiles(replay_desc(as[m], 0), m, trec);
+        batch_tiles(rec[m], m, trec);
     }
     tx.insert(tx.end(), txr.begin(), txr.end());
     // per global step: replay descriptors (stage 1, 2), replay parities, and
@@ -1808,7 +1789,7 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
                  step_bytes = oDt + al(n * szDA);
     const size_t tab_bytes = al(tb.size() * sizeof(BlockRef)) + al(ty.size() * sizeof(BlockRef)) +
                              al(tx.size() * sizeof(BlockRef)) + al(std::max<size_t>(1, tseed.size()) * sizeof(BlockRef)) +
-                             al(trec.size() * sizeof(RecTile));
+                             al(trec.size() * sizeof(BatchTile));
     const size_t total = tab_bytes + step_bytes * (size_t)nsteps;
     if ((rc = batch_tables(as[0], total))) return rc;
     char *host = as[0]->batch_host, *dev = as[0]->batch_dev;
@@ -1826,14 +1807,15 @@ int bwd_batched(int n, rkg_adjoint* const* as, double loss_scale) {
     const BlockRef* dTx = (const BlockRef*)put(tx.data(), tx.size() * sizeof(BlockRef));
     const BlockRef* dTs = (const BlockRef*)put(tseed.data(), tseed.size() * sizeof(BlockRef));
     if (tseed.empty()) off += 256;
-    const RecTile* dTr = (const RecTile*)put(trec.data(), trec.size() * sizeof(RecTile));
+    const BatchTile* dTr = (const BatchTile*)put(trec.data(), trec.size() * sizeof(BatchTile));
     off = tab_bytes;
     for (int s = 0; s < nseg; ++s) {
         for (int k = 0; k < seg_steps(as[0], s); ++k) {
             char* h = host + tab_bytes + step_bytes * (size_t)(s * K + k);
             for (int m = 0; m < n; ++m) {
                 rkg_adjoint* a = as[m];
-                GridDesc d1 = replay_desc(a, k);
+                GridDesc d1 = stage_desc(a, wsA(a, k), wsB(a, k), wsA(a, k + 1));
+                copy_tiles(d1, rec[m]);
                 d1.rec = wsD1(a, k);
                 d1.hist = a->hist + HIST * k;
                 GridDesc d2 = d1;

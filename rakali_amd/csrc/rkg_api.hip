@@ -167,7 +167,7 @@ int launch_generic(rkg_grid* g, int n, int mode, double tlim) {
     GridDesc d = make_desc(g);
     d.mpart = nullptr;  // the generic path keeps no mass budget (as the reference)
     d.spart = nullptr;
-    const int ntiles = d.nstrips * d.nsegs;
+    const int ntiles = d.ntiles;
     const SchemeTab T = scheme_tab(g->scheme);
     double* A = plane_ptr(g, 0);
     double* B = plane_ptr(g, 3);
@@ -241,7 +241,7 @@ int launch_steps_now(rkg_grid* g, int n, int mode, double tlim) {
     }
     if (g->scheme != RKG_TIME_RK2) return launch_generic(g, n, mode, tlim);
     GridDesc d = make_desc(g);
-    const int ntiles = d.nstrips * d.nsegs;
+    const int ntiles = d.ntiles;
     const double area = d.dx * d.dy;
     // Interior sum of the precipitation rate for the surface mass source
     // (fixed over the call: the planes change only between calls).
@@ -259,7 +259,7 @@ int launch_steps_now(rkg_grid* g, int n, int mode, double tlim) {
         launch_stage<1>(g, d, ntiles, mode, tlim);
         if (g->prof) HIP_TRY(hipEventRecord(g->ev[1], g->stream));
         launch_stage<2>(g, d, ntiles, mode, tlim);
-        const BudgetArgs budget{g->ctrl, g->parity, d.mpart, ntiles, area, rain, d.spart};
+        const BudgetArgs budget{g->ctrl, g->parity, d.mpart, d.nstrips * d.nsegs, area, rain, d.spart};
         g->parity ^= 1;
         if (!gauges_after_step(g, g->parity, budget) && d.mpart)
             hipLaunchKernelGGL(k_budget, dim3(1), dim3(256), 0, g->stream, budget);

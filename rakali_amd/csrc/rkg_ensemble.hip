@@ -31,16 +31,6 @@ namespace {
 constexpr unsigned ENS_MAGIC = 0x72616B45u;  // 'rakE'
 constexpr unsigned ENS_DEAD = 0xDEADBEEFu;
 
-struct BatchTile {
-    int member, strip, seg, leader;
-};
-
-// The tile of a table entry, as stage_tile asks for it.
-struct TileOf {
-    BatchTile bt;
-    __device__ int3 operator()(const GridDesc&) const { return make_int3(bt.strip, bt.seg, bt.leader); }
-};
-
 // The tile loop of the persistent variant needs about 250 VGPRs to keep
 // the tile body free of spills, so it runs at two waves per SIMD.
 template <int STAGE, bool HLLC, bool PERSISTENT>
@@ -51,8 +41,8 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(PERSISTENT
     if (!PERSISTENT) {
         const int t = xcd_tile(blockIdx.x, ntiles);
         const BatchTile bt = tiles[t];
-        stage_tile<STAGE, HLLC, false, false, TileOf>(descs[bt.member], ring, p, MODE_STEP,
-                                                      descs[bt.member].t_end, TileOf{bt});
+        stage_tile<STAGE, HLLC, false, false, BatchTile>(descs[bt.member], ring, p, MODE_STEP,
+                                                      descs[bt.member].t_end, bt);
         return;
     }
     // The other stage's counter is idle during this launch: clear it for
@@ -65,8 +55,8 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(PERSISTENT
         const int t = __builtin_amdgcn_readfirstlane((int)slot);
         if (t >= ntiles) break;
         const BatchTile bt = tiles[t];
-        stage_tile<STAGE, HLLC, false, false, TileOf>(descs[bt.member], ring, p, MODE_STEP,
-                                                      descs[bt.member].t_end, TileOf{bt});
+        stage_tile<STAGE, HLLC, false, false, BatchTile>(descs[bt.member], ring, p, MODE_STEP,
+                                                      descs[bt.member].t_end, bt);
         __syncthreads();   // the next tile rewrites the slot
     }
 }
@@ -135,9 +125,7 @@ GridDesc ens_desc(rkg_ensemble* e, int m) {
     d.clamped_elevation = c.clamped_elevation;
     d.dt_fixed = c.dt_fixed; d.t_end = c.t_end;
     d.cfl_interval = c.cfl_interval;
-    d.ty = e->ty;
-    d.nstrips = (c.nx + OWN - 1) / OWN;
-    d.nsegs = (c.ny + e->ty - 1) / e->ty;
+    set_tiles(d, e->ty, false);
     d.ctrl = e->ctrl + 2 * m;
     d.ssp_coeff = 1.0;  // ensembles run SSP-RK2
     return d;
@@ -152,12 +140,9 @@ void drop_graph(rkg_ensemble* e) {
 int build_tables(rkg_ensemble* e) {
     std::vector<GridDesc> d(e->n);
     std::vector<BatchTile> t;
-    for (int m = 0; m < e->n; ++m) {
-        d[m] = ens_desc(e, m);
-        for (int seg = 0; seg < d[m].nsegs; ++seg)
-            for (int strip = 0; strip < d[m].nstrips; ++strip)
-                t.push_back(BatchTile{m, strip, seg, (strip == 0 && seg == 0) ? 1 : 0});
-    }
+    for (int m = 0; m < e->n; ++m) d[m] = ens_desc(e, m);
+    set_launch_tiles(d.data(), e->n, std::vector<int>(e->n, e->ty).data());
+    for (int m = 0; m < e->n; ++m) batch_tiles(d[m], m, t);
     HIP_TRY(hipStreamSynchronize(e->stream));
     if (e->tiles) HIP_TRY(hipFree(e->tiles));
     e->tiles = nullptr;

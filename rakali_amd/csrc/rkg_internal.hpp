@@ -200,6 +200,32 @@ inline long long grid_tiles(int nx, int ny, int rows) {
     return (long long)((nx + OWN - 1) / OWN) * ((ny + rows - 1) / rows);
 }
 
+// Whether a launch packs the segments of its narrow last strips (tile_at):
+// `tiles` wavefronts without, `packed` with.  It pays where the launch is more
+// than the chip's 3072 slots, or where it leaves the fullest of the 1024 SIMDs a
+// wavefront less to run; with as many there a shared wavefront, which reads
+// `pack` rows at a time, is the slower one.  us per step, unpacked / packed:
+//   64x262144 1821 / 1112,  128x131072 1286 / 1053,  256x8192  180 / 162,
+//   128x8192   123 / 102,   64x3000      47 / 39,    2x100000  383 / 81;
+//   as many on a SIMD: 128x2048 41 / 45, 500x1000 51 / 55, 256x1024 41 / 43;
+//   ensembles of 64 x 256^2 302 / 275, 256 x 128^2 358 / 302, 256 x 64^2 185 / 132
+inline bool pack_pays(long long tiles, long long packed) {
+    auto fullest = [](long long n) { return (n + 1023) / 1024; };
+    return tiles > 3 * 1024 || fullest(packed) < fullest(tiles);
+}
+
+// The tiles of the n members of a launch.
+inline void set_launch_tiles(GridDesc* d, int n, const int* ty) {
+    long long tiles = 0, packed = 0;
+    for (int m = 0; m < n; ++m) {
+        set_tiles(d[m], ty[m], true);
+        tiles += (long long)d[m].nstrips * d[m].nsegs;
+        packed += d[m].ntiles;
+    }
+    if (pack_pays(tiles, packed)) return;
+    for (int m = 0; m < n; ++m) set_tiles(d[m], ty[m], false);
+}
+
 inline int default_tile_rows(int nx, int ny) {
     return rows_for([=](int rows) { return grid_tiles(nx, ny, rows); }, 1);
 }
@@ -243,9 +269,7 @@ inline GridDesc desc_of_config(const rkg_config& c, long long pitch, int ty) {
     d.clamped_elevation = c.clamped_elevation;
     d.dt_fixed = c.dt_fixed; d.t_end = c.t_end;
     d.cfl_interval = c.cfl_interval;
-    d.ty = ty;
-    d.nstrips = (c.nx + OWN - 1) / OWN;
-    d.nsegs = (c.ny + d.ty - 1) / d.ty;
+    set_launch_tiles(&d, 1, &ty);
     d.ssp_coeff = 1.0;
     return d;
 }

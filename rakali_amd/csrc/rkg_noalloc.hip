@@ -101,7 +101,7 @@ extern "C" int rkg_step_noalloc(const rkg_config* cfg, double* h, double* hu, do
     d.bhu = d.bh + cells;
     d.bhv = d.bhu + cells;
     d.ctrl = reinterpret_cast<CtrlSlot*>(s);
-    const int ntiles = d.nstrips * d.nsegs;
+    const int ntiles = d.ntiles;
     const bool hllc = cfg->use_hllc != 0;
 
     // Slot 0 starts from the caller's clock (a kernel writes it: no memset

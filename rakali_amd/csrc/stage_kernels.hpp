@@ -4,6 +4,8 @@
 // that launches them holds its own copy.
 #pragma once
 
+#include <vector>
+
 #include "swe_kernels.hpp"
 
 #ifndef RKG_WAVES_PER_EU
@@ -83,19 +85,18 @@ __device__ __forceinline__ SourceTerms make_src(const GridDesc& d, double dt) {
     return s;
 }
 
-// One tile of one stage of one grid.  `where(d)` gives the tile as
-// (strip, segment, leader); the leader is the single tile per grid and
-// launch that advances the control slot.  STAGE 1 and 2 are the fused
+// One tile of one stage of one grid.  `where(d, leader)` gives the tile; the
+// leader is the single tile per grid and launch that advances the control slot.  STAGE 1 and 2 are the fused
 // SSP-RK2 stages; STAGE 3 is one stage `gs` of a generic SSP scheme.
 template <int STAGE, bool HLLC, bool NF, bool REC, class Where, int FEAT = 0>
 __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, int p, int mode, double tlim, Where where, const GenStage& gs = GenStage{}) {
-    const int3 w = where(d);
-    const bool leader = w.z != 0;
-    const int strip = w.x, seg = w.y;
+    bool leader;
+    const TileAt w = where(d, leader);
+    const int strip = w.strip, seg = w.seg;
     StageCtx s;
     int x0, x1;
-    tile_range(d.nx, OWN, strip, x0, x1);
-    tile_range(d.ny, d.ty, seg, s.row0, s.row1);
+    tile_range(d.nx, OWN, d.nstrips, strip, x0, x1);
+    tile_range(d.ny, d.ty, d.nsegs, seg, s.row0, s.row1);   // of several segments, those of the first
     const bool west = x0 < HALO, east = x0 + OWN + HALO > d.nx;
     const bool south = s.row0 < HALO, north = s.row1 + HALO > d.ny;
     const bool edge = west || east || south || north;
@@ -103,9 +104,8 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, in
     if (STAGE == 1) { s.ih = d.ah; s.ihu = d.ahu; s.ihv = d.ahv; }
     else if (STAGE == 2) { s.ih = d.bh; s.ihu = d.bhu; s.ihv = d.bhv; }
     else { s.ih = gs.ih; s.ihu = gs.ihu; s.ihv = gs.ihv; }
-    const int c = x0 - HALO + (int)threadIdx.x;
-    const LaneSource lsrc = edge ? lane_source<true>(d, c) : lane_source<false>(d, c);
-    const FirstRows first = edge ? first_rows<true>(d, s, lsrc, s.row0) : first_rows<false>(d, s, lsrc, s.row0);
+    const TileLane lane = edge ? tile_lane<true>(d, w, x0, x1, threadIdx.x) : tile_lane<false>(d, w, x0, x1, threadIdx.x);
+    const FirstRows first = edge ? first_rows<true>(d, s, lane, s.row0) : first_rows<false>(d, s, lane, s.row0);
     s.alpha = 0.0; s.a_prev = 1.0;
     s.blend = false; s.first = false; s.last = false;
     s.radiate = false; s.prev_h = nullptr; s.bc_dt = 0.0;
@@ -177,38 +177,57 @@ __device__ __forceinline__ void stage_tile(const GridDesc& d, TileRing& ring, in
     s.src = make_src(d, s.dt);
     double smax, fsum, ssum;
     if (!edge) {
-        smax = process_tile<STAGE, HLLC, false, NF, REC, FEAT>(d, s, ring, lsrc, first, x0, x1, s.row0, s.row1, fsum, ssum);
+        const TileLane inner = tile_lane<false>(d, w, x0, x1, threadIdx.x);   // again, not kept through the clock's code
+        smax = process_tile<STAGE, HLLC, false, NF, REC, FEAT>(d, s, ring, inner, first, s.row0, s.row1, fsum, ssum);
     } else {
         // the tide (a correctly rounded sine, a long dependent chain) only
         // where the tile reads ghost cells of a tidal edge
         if ((west && d.bc[0] == BC_TIDAL) || (east && d.bc[1] == BC_TIDAL) || (south && d.bc[2] == BC_TIDAL) ||
             (north && d.bc[3] == BC_TIDAL))
             s.eta_tidal = tidal_eta(d, t_tide);
-        smax = process_tile<STAGE, HLLC, true, NF, REC, FEAT>(d, s, ring, lsrc, first, x0, x1, s.row0, s.row1, fsum, ssum);
+        smax = process_tile<STAGE, HLLC, true, NF, REC, FEAT>(d, s, ring, lane, first, s.row0, s.row1, fsum, ssum);
     }
     if (STAGE == 2 || STAGE == 3) {
         smax = wave_max(smax);
         if (threadIdx.x == 0 && smax > 0.0) speed_add(d.ctrl[1 - p], (unsigned)(strip + seg * d.nstrips), smax);
     }
+    // the sums of a tile go to its first segment's slot, zeros to the other segments'
+    const int slots = d.nstrips * d.nsegs;
+    const long long slot = (long long)(STAGE - 1) * slots + (long long)(seg + (int)threadIdx.x) * d.nstrips + strip;
     if (STAGE != 3 && d.mpart != nullptr) {  // accumulate_boundary_mass_out's sum, per tile
         fsum = wave_sum(fsum);
-        if (threadIdx.x == 0)
-            d.mpart[(long long)(STAGE - 1) * d.nstrips * d.nsegs + (long long)seg * d.nstrips + strip] = fsum;
+        if ((int)threadIdx.x < w.count) d.mpart[slot] = threadIdx.x == 0 ? fsum : 0.0;
     }
     if ((FEAT & FEAT_SPONGE) && STAGE != 3 && d.spart != nullptr) {  // accumulate_sponge_mass_src
         ssum = wave_sum(ssum);
-        if (threadIdx.x == 0)
-            d.spart[(long long)(STAGE - 1) * d.nstrips * d.nsegs + (long long)seg * d.nstrips + strip] = ssum;
+        if ((int)threadIdx.x < w.count) d.spart[slot] = threadIdx.x == 0 ? ssum : 0.0;
     }
 }
 
 // Single grid: one workgroup (one wavefront) per tile.
 struct SingleGridTile {
-    __device__ int3 operator()(const GridDesc& g) const {
-        const int tile = xcd_tile(blockIdx.x, g.nstrips * g.nsegs);
-        return make_int3(tile % g.nstrips, tile / g.nstrips, blockIdx.x == 0);
+    __device__ TileAt operator()(const GridDesc& g, bool& leader) const {
+        leader = blockIdx.x == 0;
+        return tile_at(g, xcd_tile(blockIdx.x, g.ntiles));
     }
 };
+
+// A tile of one member of a batch, as the tables list them.
+struct BatchTile {
+    int member, strip, seg, count;   // count negative: the leader
+    __device__ TileAt operator()(const GridDesc&, bool& leader) const {
+        leader = count < 0;
+        return TileAt{strip, seg, leader ? -count : count};
+    }
+};
+
+// Member m's tiles, in the order and with the leader of its own launches.
+inline void batch_tiles(const GridDesc& d, int m, std::vector<BatchTile>& t) {
+    for (int k = 0; k < d.ntiles; ++k) {
+        const TileAt w = tile_at(d, k);
+        t.push_back(BatchTile{m, w.strip, w.seg, k == 0 ? -w.count : w.count});
+    }
+}
 
 // FEAT: FEAT_FORCING / FEAT_SPONGE / FEAT_CHAPMAN source terms.
 template <int STAGE, bool HLLC, bool NF, bool REC, int FEAT = 0>

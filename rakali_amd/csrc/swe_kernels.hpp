@@ -91,6 +91,10 @@ struct GridDesc {
     int ty;                       // rows per tile segment (<= 64)
     int plain_rows;               // every row with plain divisions (rkg_set_fast_path(-1))
     int nstrips, nsegs;
+    int ntiles;                   // wavefronts of a launch, see tile_at
+    unsigned strips_inv;          // 2^32 / nstrips, rounded up (0 for one strip)
+    int pack, pack_seg, pack_n;   // segments of the last strip that share a wavefront (1: none); the
+                                  // first and the number of the segments that do
     CtrlSlot* ctrl;               // [2]
 };
 
@@ -244,7 +248,7 @@ struct StageCtx {
     // Chapman edges (FEAT_CHAPMAN): whether this boundary call radiates
     // (its state differs from the previous call's), the previous call's
     // state prev_h (its eta_old = prev_h + b at the first interior cell),
-    // the step's dt (bc%dt) and the tile's own rows
+    // the step's dt (bc%dt) and the own rows of the tile's first segment
     bool radiate;
     const double* prev_h;
     double bc_dt;
@@ -280,10 +284,10 @@ struct GenStage {
 //   the generic schemes, with the step's dt; the outer layer again sees
 //   eta_old = its interior eta.
 // The bed ghost is the first interior bed (fill_bathymetry_ghosts_array).
-// x-edge ghosts of rows outside the tile's own are never used (the y
+// x-edge ghosts of rows outside the tile's own (own_row) are never used (the y
 // pipeline loads them for lanes past the grid); they skip the radiation,
 // whose eta_old the owning tile may be overwriting in place.
-__device__ __forceinline__ Cell chapman_ghost(const GridDesc& d, const StageCtx& s, int side, int c, int j) {
+__device__ __forceinline__ Cell chapman_ghost(const GridDesc& d, const StageCtx& s, int side, int c, int j, bool own_row) {
     const bool xedge = side < 2, lo = (side & 1) == 0;
     const int kk = xedge ? (lo ? -c - 1 : c - d.nx) : (lo ? -j - 1 : j - d.ny);
     Cell g;
@@ -298,8 +302,7 @@ __device__ __forceinline__ Cell chapman_ghost(const GridDesc& d, const StageCtx&
     const double hmax = dmax(h_int, 1.0e-6);
     const double speed = sqrt(d.g * hmax);
     double eta_g = eta_int;
-    const bool own_row = !xedge || (j >= s.row0 && j < s.row1);
-    if (kk == 0 && s.radiate && s.bc_dt > 0.0 && own_row) {
+    if (kk == 0 && s.radiate && s.bc_dt > 0.0 && (own_row || !xedge)) {
         const long long k0 = (long long)ji * d.pitch + ci;
         const long long k2 = (long long)j2 * d.pitch + c2;
         const double dd = xedge ? d.dx : d.dy;
@@ -330,10 +333,10 @@ struct LaneSource {
     int side;   // 0 W, 1 E: a ghost column; -1: a column of the grid; -2: beyond the ghosts
 };
 
-__device__ __forceinline__ bool mirrors(int tag) { return tag == BC_WALL || tag == BC_SPONGE; }
+__host__ __device__ __forceinline__ bool mirrors(int tag) { return tag == BC_WALL || tag == BC_SPONGE; }
 
 template <bool EDGE>
-__device__ __forceinline__ LaneSource lane_source(const GridDesc& d, int c) {
+__host__ __device__ __forceinline__ LaneSource lane_source(const GridDesc& d, int c) {
     if (!EDGE || ((unsigned)c < (unsigned)d.nx)) return LaneSource{c, -1};
     const bool west = c < 0;
     const int kk = west ? -c - 1 : c - d.nx;
@@ -342,21 +345,33 @@ __device__ __forceinline__ LaneSource lane_source(const GridDesc& d, int c) {
     return LaneSource{west ? in : d.nx - 1 - in, west ? 0 : 1};
 }
 
+// A lane of a tile: its column c, the rows `row` by which its segment lies
+// above the tile's first one (tiles that hold several, see tile_at), and `at`,
+// the offset of its source column in the tile's row 0 of a plane (of its own
+// column where it owns one).  own: its cells are the tile's; use_x: its
+// right face is used.
+struct TileLane {
+    int c, row, side;             // side as in LaneSource
+    long long at;
+    bool own, use_x;
+};
+
 // The cells that row j of the march is made from: those of row j, or of the
 // source row of a ghost row.
 template <bool EDGE>
-__device__ __forceinline__ Cell row_source(const GridDesc& d, const StageCtx& s, const LaneSource& l, int j) {
+__device__ __forceinline__ Cell row_source(const GridDesc& d, const StageCtx& s, const TileLane& l, int j) {
     int js = j;
     if (EDGE) {
         if (j < 0) js = mirrors(d.bc[2]) ? -j - 1 : 0;
         else if (j >= d.ny) js = mirrors(d.bc[3]) ? 2 * d.ny - 1 - j : d.ny - 1;
     }
-    return load_direct(s.ih, s.ihu, s.ihv, d.bed, d.pitch, l.c, js);
+    const long long k = (long long)js * d.pitch + l.at;
+    return Cell{in_hbm(s.ih)[k], in_hbm(s.ihu)[k], in_hbm(s.ihv)[k], in_hbm(d.bed)[k]};
 }
 
 // Row j of the march at the lane's column from its source cell.
 template <bool EDGE, int FEAT>
-__device__ __forceinline__ Cell row_cell(const GridDesc& d, const StageCtx& s, const LaneSource& l, int c, int j,
+__device__ __forceinline__ Cell row_cell(const GridDesc& d, const StageCtx& s, const TileLane& l, int j,
                                          const Cell& src) {
     if (!EDGE) return src;
     const int rs = j < 0 ? 2 : (j >= d.ny ? 3 : -1);
@@ -365,7 +380,7 @@ __device__ __forceinline__ Cell row_cell(const GridDesc& d, const StageCtx& s, c
     const int side = rs >= 0 ? (l.side == -1 ? rs : -2) : l.side;
     if (side < 0) return Cell{0.0, 0.0, 0.0, 0.0};
     if constexpr ((FEAT & FEAT_CHAPMAN) != 0)
-        if (d.bc[side] == BC_CHAPMAN) return chapman_ghost(d, s, side, c, j);
+        if (d.bc[side] == BC_CHAPMAN) return chapman_ghost(d, s, side, l.c, j + l.row, j >= s.row0 && j < s.row1);
     return ghost_from(d, d.bc[side], s.eta_tidal, src, src, (side & 1) ? 1.0 : -1.0, side < 2);
 }
 
@@ -379,15 +394,14 @@ struct ExactTag {
 constexpr int HALO = 2;
 constexpr int OWN = WAVE - 2 * HALO;
 
-// Own range [lo, hi) of block s when [0, n) is cut into blocks of w, the
+// Own range [lo, hi) of block s when [0, n) is cut into nb blocks of w, the
 // last block holding at least two cells: the halo of the block before it
 // then ends inside the grid, so a ghost cell (which may depend on what the
 // edge's own tile overwrites, see chapman_ghost) is read by the edge's own
 // tile only.  Blocks of one cell, which grids with such edges do not use, stay
 // that (a last block of two would last as long as two rows: 130x97, 25 us a
 // step, 21 so).
-__host__ __device__ __forceinline__ void tile_range(int n, int w, int s, int& lo, int& hi) {
-    const int nb = (n + w - 1) / w;
+__host__ __device__ __forceinline__ void tile_range(int n, int w, int nb, int s, int& lo, int& hi) {
     lo = s * w;
     hi = lo + w < n ? lo + w : n;
     if (w >= 2 && nb >= 2 && n - (nb - 1) * w == 1) {
@@ -402,8 +416,84 @@ struct FirstRows {
     Cell r[4];
 };
 
+// The tile `t` of a launch: `count` segments from `seg` of a strip.
+struct TileAt {
+    int strip, seg, count;
+};
+
+// A last strip of w <= 28 columns would leave most lanes of its wavefronts
+// idle: 64 columns took the time of 120.  There `pack` = 64 / (w + 4) segments
+// that lie above each other share a wavefront, each with its own halo lanes;
+// they march together, so they must be of one height and touch neither the
+// south nor the north ghost rows (segments pack_seg .. pack_seg + pack_n).  The
+// order stays by rows, a shared wavefront after the strips beside it: at the
+// end of the launch they were one XCD's alone.
+__host__ __device__ __forceinline__ TileAt tile_at(const GridDesc& d, unsigned t) {
+    const unsigned strips = d.nstrips, full = strips - 1, below = d.pack_seg * strips;
+    unsigned seg0 = 0;
+    if (__builtin_expect(d.pack > 1, 0) && t >= below) {
+        t -= below;
+        const unsigned per = d.pack * full + 1, group = t / per, r = t - group * per;
+        const int seg = d.pack_seg + (int)group * d.pack;
+        const int left = d.pack_n - (int)group * d.pack, count = left < d.pack ? left : d.pack;
+        if (count > 0) {
+            if (r == count * full) return TileAt{(int)full, seg, count};
+            if (r < count * full) return TileAt{(int)(r % full), seg + (int)(r / full), 1};
+        }
+        t -= d.pack_n * full + (d.pack_n + d.pack - 1) / d.pack;
+        seg0 = d.pack_seg + d.pack_n;
+    }
+    // t / strips without a division, which every wavefront would wait for before
+    // its first load: the quotient, or one more
+    unsigned q = d.strips_inv == 0 ? t : (unsigned)((unsigned long long)t * d.strips_inv >> 32);
+    if (q * strips > t) --q;
+    return TileAt{(int)(t - q * strips), (int)(seg0 + q), 1};
+}
+
+// The tiles of `ty` rows of a descriptor, narrow last strips packed or not.
+inline void set_tiles(GridDesc& d, int ty, bool pack) {
+    d.ty = ty;
+    d.nstrips = (d.nx + OWN - 1) / OWN;
+    d.nsegs = (d.ny + ty - 1) / ty;
+    d.strips_inv = d.nstrips == 1 ? 0 : (unsigned)(((1ull << 32) + d.nstrips - 1) / d.nstrips);
+    int lo, hi;
+    tile_range(d.nx, OWN, d.nstrips, d.nstrips - 1, lo, hi);
+    d.pack = pack ? WAVE / (hi - lo + 2 * HALO) : 1;
+    d.pack_seg = (HALO + ty - 1) / ty;
+    d.pack_n = (d.ny - HALO) / ty - d.pack_seg;
+    if (d.pack_n < 2 || d.pack < 2) { d.pack = 1; d.pack_n = 0; }
+    d.ntiles = d.nstrips * d.nsegs - d.pack_n + (d.pack_n + d.pack - 1) / d.pack;
+}
+
+// Gives d the tiles of another descriptor of the grid.
+inline void copy_tiles(GridDesc& d, const GridDesc& of) {
+    d.ty = of.ty; d.nstrips = of.nstrips; d.nsegs = of.nsegs; d.ntiles = of.ntiles;
+    d.strips_inv = of.strips_inv;
+    d.pack = of.pack; d.pack_seg = of.pack_seg; d.pack_n = of.pack_n;
+}
+
+// Lane `lane` of tile w, whose columns are [x0, x1).
 template <bool EDGE>
-__device__ __forceinline__ FirstRows first_rows(const GridDesc& d, const StageCtx& s, const LaneSource& l, int j0) {
+__host__ __device__ __forceinline__ TileLane tile_lane(const GridDesc& d, const TileAt& w, int x0, int x1, int lane) {
+    int i = lane, k = 0;
+    if (EDGE && w.count > 1) {
+        const int span = x1 - x0 + 2 * HALO;
+        k = lane / span;
+        i = lane - k * span;
+    }
+    TileLane l;
+    l.c = x0 - HALO + i;
+    l.own = i >= HALO && l.c < x1 && k < w.count;
+    l.use_x = i >= HALO - 1 && l.c < x1 && k < w.count;
+    const LaneSource src = lane_source<EDGE>(d, l.c);
+    l.side = src.side;
+    l.row = EDGE ? (k < w.count ? k : w.count - 1) * d.ty : 0;
+    l.at = src.c + l.row * d.pitch;
+    return l;
+}
+
+template <bool EDGE>
+__device__ __forceinline__ FirstRows first_rows(const GridDesc& d, const StageCtx& s, const TileLane& l, int j0) {
     FirstRows f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) f.r[q] = row_source<EDGE>(d, s, l, j0 - 2 + q);
@@ -434,10 +524,11 @@ __device__ __forceinline__ void sponge_cell(const GridDesc& d, double dt, int c,
     }
 }
 
-// One tile of one RK stage: a strip of at most 60 owned columns x d.ty rows,
-// processed by one wavefront marching down the rows; lane l holds column
-// x0 - 2 + l, so the two columns each side that the stencil needs are lanes
-// of the same wavefront, and no column is treated apart.
+// One tile of one RK stage: a strip of at most 60 owned columns x d.ty rows
+// (or several such segments of a narrow strip), processed by one wavefront
+// marching down the rows; lane l holds column x0 - 2 + l, so the two columns
+// each side that the stencil needs are lanes of the same wavefront, and no
+// column is treated apart.
 // Row j: the y-slope of row j+1 is formed from the raw rows j, j+1, j+2
 // held in registers, giving the face above row j together with the top
 // state of row j carried from the previous row; the march starts one row
@@ -459,14 +550,12 @@ __device__ __forceinline__ void sponge_cell(const GridDesc& d, double dt, int c,
 // and writes U^{n+1} over A, returning the lane's max CFL speed.
 template <int STAGE, bool HLLC, bool EDGE, bool NF, bool REC, int FEAT = 0>
 __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx& s, TileRing& ring,
-                                               const LaneSource& lsrc, const FirstRows& first, int x0, int x1, int j0,
-                                               int j1, double& fsum, double& ssum) {
+                                               const TileLane& l, const FirstRows& first, int j0, int j1, double& fsum,
+                                               double& ssum) {
     constexpr bool FRC = (FEAT & FEAT_FORCING) != 0;
     constexpr bool SPG = (FEAT & FEAT_SPONGE) != 0;
     const int lane = threadIdx.x;
-    const int c = x0 - HALO + lane;
-    const bool own = lane >= HALO && c < x1;
-    const bool use_x = lane >= HALO - 1 && c < x1;   // lanes whose right face is used
+    const bool own = l.own, use_x = l.use_x;
     const double g = d.g;
     const long long pitch = d.pitch;
     // the row path's ranges assume a gravity and a friction of ordinary size
@@ -482,9 +571,9 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
     // the rows j, j+1 and j+2 of the march, in LDS; a lane's neighbours by
     // their lane, the wavefront's ends repeating themselves (unused)
     const int lane_m = max(lane - 1, 0), lane_p = min(lane + 1, WAVE - 1);
-    auto surf = [&](int slot, int l) { return Surf{ring.v[slot][0][l], ring.v[slot][1][l], ring.v[slot][2][l]}; };
-    auto cell = [&](int slot, int l) {
-        return Cell{ring.v[slot][4][l], ring.v[slot][1][l], ring.v[slot][2][l], ring.v[slot][3][l]};
+    auto surf = [&](int slot, int i) { return Surf{ring.v[slot][0][i], ring.v[slot][1][i], ring.v[slot][2][i]}; };
+    auto cell = [&](int slot, int i) {
+        return Cell{ring.v[slot][4][i], ring.v[slot][1][i], ring.v[slot][2][i], ring.v[slot][3][i]};
     };
     auto put = [&](int slot, const Cell& x) {
         ring.v[slot][0][lane] = x.h + x.b; ring.v[slot][1][lane] = x.hu; ring.v[slot][2][lane] = x.hv;
@@ -508,10 +597,10 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
     bool odd_prev;
     RowBits bc, bn, bnn;
     {
-        const Cell a = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0 - 2, first.r[0]);
-        const Cell rc = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0 - 1, first.r[1]);
-        const Cell rn = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0, first.r[2]);
-        const Cell rnn = row_cell<EDGE, FEAT>(d, s, lsrc, c, j0 + 1, first.r[3]);
+        const Cell a = row_cell<EDGE, FEAT>(d, s, l, j0 - 2, first.r[0]);
+        const Cell rc = row_cell<EDGE, FEAT>(d, s, l, j0 - 1, first.r[1]);
+        const Cell rn = row_cell<EDGE, FEAT>(d, s, l, j0, first.r[2]);
+        const Cell rnn = row_cell<EDGE, FEAT>(d, s, l, j0 + 1, first.r[3]);
         FState lo, hi;
         cell_states(a, rc, rn, lo, hi);
         odd_prev = __any(unbounded(a));
@@ -524,8 +613,6 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
         wave_lds_order();
         hand_up(hi, Face{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, surf(1, lane) - surf(0, lane));
     }
-    // a column of the grid for the lanes that own none: their loads of U^n are not used
-    const int c_in = min(max(c, 0), d.nx - 1);
 
     for (int j = j0 - 1; j < j1; ++j) {
         const bool inner = j >= j0;   // the row before the first only gives its upper face
@@ -584,21 +671,22 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
         // halo again, a cell of the grid): under a condition the compiler waits
         // for everything in flight where the paths join.
         const int jn = min(j + 3, j1 + 1);
-        const Cell src = row_source<EDGE>(d, s, lsrc, jn);
+        const Cell src = row_source<EDGE>(d, s, l, jn);
         __builtin_amdgcn_sched_barrier(0);
         if (__builtin_expect(plain_row, 0)) faces(ExactTag<true>{});
         else faces(ExactTag<false>{});
 
-        // U^n at (c, j): the cell update hides it, and the faces keep their registers
+        // U^n of the cell (lanes that own none load their source cell's): the cell
+        // update hides it, and the faces keep their registers
         Cell un{0.0, 0.0, 0.0, 0.0};
         if (read_un) {
-            const long long k = (long long)max(j, 0) * pitch + c_in;
+            const long long k = (long long)max(j, 0) * pitch + l.at;
             un.h = in_hbm(d.ah)[k]; un.hu = in_hbm(d.ahu)[k]; un.hv = in_hbm(d.ahv)[k];
         }
 
         double h = 0.0, hu = 0.0, hv = 0.0;   // the row's result
         if (inner && own) {
-            const long long k = (long long)j * pitch + c;
+            const long long k = (long long)j * pitch + l.at;
             if (REC) {
                 in_hbm(d.rec)[k] = fh; in_hbm(d.rec)[d.plane + k] = fhu; in_hbm(d.rec)[2 * d.plane + k] = fhv;
             }
@@ -620,7 +708,7 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
                 if (EX) stage_body<NF, FRC>(s.src, s.dt, fh, fhu, fhv, h, hu, hv, n_cell, fr);
                 else if (stage_body_row<NF, FRC>(s.src, s.dt, fh, fhu, fhv, h, hu, hv, n_cell, fr)) return true;
                 // the sponge follows each fused stage (rki_solver.F90:787,814)
-                if (STAGE == 1 && SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, relax);
+                if (STAGE == 1 && SPG) sponge_cell(d, s.dt, l.c, j + l.row, h, hu, hv, relax);
                 if (STAGE == 2) {
                     // rki_kernel_fused.F90:435-463
                     h = 0.5 * (un.h + h);
@@ -637,7 +725,7 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
                     else if (clamp_row(g, h, hu, hv)) return true;
                 }
                 // :919-920, at beta_i dt in the generic schemes
-                if (STAGE != 1 && SPG) sponge_cell(d, s.dt, c, j, h, hu, hv, relax);
+                if (STAGE != 1 && SPG) sponge_cell(d, s.dt, l.c, j + l.row, h, hu, hv, relax);
                 if (STAGE == 2 || (STAGE == 3 && s.last)) {
                     if (EX) cfl_plain(g, h, hu, hv, smax);
                     else cfl_row(g, same, h, hu, hv, smax);
@@ -658,12 +746,12 @@ __device__ __forceinline__ double process_tile(const GridDesc& d, const StageCtx
         bc = bn;
         bn = bnn;
         if (j + 1 < j1) {
-            nxt = row_cell<EDGE, FEAT>(d, s, lsrc, c, jn, src);
+            nxt = row_cell<EDGE, FEAT>(d, s, l, jn, src);
             bnn = bits(nxt);
         }
         __builtin_amdgcn_sched_barrier(0);
         if (inner && own) {
-            const long long k = (long long)j * pitch + c;
+            const long long k = (long long)j * pitch + l.at;
             if ((STAGE == 1 || (STAGE == 3 && s.first)) && d.sh != nullptr) {
                 // h0, hu0, hv0 (rki_kernel_fused.F90:224-226, rki_solver.F90:879-881)
                 in_hbm(d.sh)[k] = ring.v[sc][4][lane]; in_hbm(d.shu)[k] = ring.v[sc][1][lane]; in_hbm(d.shv)[k] = ring.v[sc][2][lane];
