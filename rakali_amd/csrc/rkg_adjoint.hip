@@ -1658,15 +1658,27 @@ hipError_t join_streams(int n, rkg_adjoint* const* as, hipEvent_t ev, bool to_fi
     return e;
 }
 
-// Whether the forward runs of n sessions can go as one: one device, one
-// solver, and steps that launch the two stage kernels and nothing else.
+// Whether the forward runs of n sessions go as one: one device, one solver,
+// and steps that launch the two stage kernels and nothing else; and launches
+// that gain by it.  The host issues a member's step in about 16 us.  Runs of up
+// to three members, and of up to six whose common launches would be of half a
+// round to a round and a half of tiles, keep the chip busier on streams of their
+// own, where one member's stage fills the others' tails.  us a step, streams of
+// their own / as one:
+//   2 x 700x600   90 / 125,  3 x 512^2    89 / 126,  3 x 1024^2  215 / 279,
+//   4 x 512^2    142 / 162,  6 x 700x600 233 / 270;
+//   4 x 128^2     76 /  62,  4 x 1024^2  361 / 337,  8 x 512^2   262 / 262,
+//   16 x 400x300 389 / 313,  32 x 256^2  686 / 501
 bool fwd_batchable(int n, rkg_adjoint* const* as) {
+    long long tiles = 0;   // of 10 rows
+    for (int m = 0; m < n; ++m) tiles += grid_tiles(as[m]->g->cfg.nx, as[m]->g->cfg.ny, 10);
+    if (n <= 3 || (n <= 6 && tiles >= 1536 && tiles <= 3 * 1536)) return false;
     for (int m = 0; m < n; ++m) {
         const rkg_grid* g = as[m]->g;
         if (g->device != as[0]->g->device || (g->cfg.use_hllc != 0) != (as[0]->g->cfg.use_hllc != 0)) return false;
         if (!g->nfield || g->mpart || g->gauges || g->prof) return false;
     }
-    return n > 1;
+    return true;
 }
 
 // The forward runs of n sessions on the first session's stream: three
