@@ -315,15 +315,23 @@ rk::HostStage::~HostStage() {
 
 namespace {
 
+// Rows of a plane that go through the stage at a time: all of a plane of up to
+// half a piece, else at most half of them, so that one piece is in transfer while
+// the host copies another.
+size_t piece_rows(size_t row, size_t ny) {
+    if (row * ny <= HostStage::PIECE / 2) return ny;
+    return std::max<size_t>(1, std::min(HostStage::PIECE / row, ny / 2));
+}
+
 // Whether this host memory goes through the stage: pageable memory, more than
-// one row (a single row is one transfer anyway), rows that fit a piece; and
-// the stage has room for two pieces, or for the plane.
-bool staged(HostStage& st, const void* host, size_t row, size_t ny) {
-    if (ny < 2 || row > HostStage::PIECE) return false;
+// one row (a single row is one transfer anyway), rows of at most `widest` bytes;
+// and the stage has room for the plane, or for two pieces.
+bool staged(HostStage& st, const void* host, size_t row, size_t ny, size_t widest) {
+    if (ny < 2 || row > widest) return false;
     hipPointerAttribute_t a;
     if (hipPointerGetAttributes(&a, host) != hipSuccess) { (void)hipGetLastError(); return false; }
     if (a.type != hipMemoryTypeUnregistered) return false;
-    const size_t whole = row * ny, need = whole <= HostStage::PIECE ? whole : 2 * HostStage::PIECE;
+    const size_t need = piece_rows(row, ny) == ny ? row * ny : 2 * HostStage::PIECE;
     if (st.bytes < need) {
         // an allocation does not disturb a capture on another thread
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -351,11 +359,11 @@ hipError_t rk::plane_to_host(HostStage& st, double* dst, size_t ld, const double
     const size_t W = sizeof(double);
     std::lock_guard<std::mutex> hold(st.lock);
     hipError_t e = hipSuccess;
-    if (!staged(st, dst, nx * W, ny)) {
+    if (!staged(st, dst, nx * W, ny, HostStage::PIECE)) {
         e = hipMemcpy2DAsync(dst, ld * W, plane, pitch * W, nx * W, ny, hipMemcpyDeviceToHost, stream);
         return e == hipSuccess ? hipStreamSynchronize(stream) : e;
     }
-    const size_t rows = HostStage::PIECE / (nx * W);   // per piece
+    const size_t rows = piece_rows(nx * W, ny);
     auto rows_of = [&](size_t j) { return std::min(rows, ny - j); };
     auto half = [&](size_t k) { return st.mem + (k & 1) * (HostStage::PIECE / W); };
     auto fetch = [&](size_t k) {
@@ -376,11 +384,11 @@ hipError_t rk::plane_from_host(HostStage& st, double* plane, size_t pitch, const
     const size_t W = sizeof(double);
     std::lock_guard<std::mutex> hold(st.lock);
     hipError_t e = hipSuccess;
-    if (!staged(st, src, nx * W, ny)) {
+    if (!staged(st, src, nx * W, ny, HostStage::WIDEST_UP)) {
         e = hipMemcpy2DAsync(plane, pitch * W, src, ld * W, nx * W, ny, hipMemcpyHostToDevice, stream);
         return e == hipSuccess ? hipStreamSynchronize(stream) : e;
     }
-    const size_t rows = HostStage::PIECE / (nx * W);
+    const size_t rows = piece_rows(nx * W, ny);
     for (size_t k = 0, j = 0; j < ny && e == hipSuccess; ++k, j += rows) {
         // the half's previous piece, two before, has left: the last wait was for it
         double* half = st.mem + (k & 1) * (HostStage::PIECE / W);

@@ -25,10 +25,13 @@ struct GaugeState;   // gauge stations and their time series (rkg_gauges.hip)
 // each (768 x 700: 4.9 ms down, 6.5 ms up); to pinned memory it is one
 // transfer at the link's rate (83 us) plus a copy in host memory (55 us).  A
 // plane goes through in pieces, one in transfer while the host copies the
-// other.  Made on first use, at most 2 * PIECE bytes, freed with its owner;
-// calls from several threads take turns.
+// other.  Uploads of wide rows go directly: the runtime takes a row of pageable
+// memory faster than the host copies it (us, directly / through the stage: rows
+// of 160 KB x 32 380 / 209, 320 KB x 4 68 / 76, 800 KB x 32 757 / 956; downloads
+// of 800 KB x 32 1507 / 983).  Made on first use, at most 2 * PIECE bytes, freed
+// with its owner; calls from several threads take turns.
 struct HostStage {
-    static constexpr size_t PIECE = (size_t)2 << 20;
+    static constexpr size_t PIECE = (size_t)2 << 20, WIDEST_UP = (size_t)1 << 19;
     std::mutex lock;
     double* mem = nullptr;
     size_t bytes = 0;     // of mem

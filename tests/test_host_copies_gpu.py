@@ -80,3 +80,10 @@ def test_first_step_after_an_upload_is_not_captured():
     for k in ("h", "hu", "hv"):
         assert np.array_equal(g.get_field(k), want.get_field(k))
     assert g.clock == want.clock
+
+
+@pytest.mark.parametrize("nx,ny", [(65536, 3), (65537, 3), (PIECE // 4, 2), (PIECE // 4 + 1, 2), (PIECE // 4 + 1, 3),
+                                   (PIECE // 2, 2), (PIECE // 2 + 1, 3), (361, 363), (363, 362)])
+def test_planes_at_the_limits_of_the_pieces(nx, ny):
+    """Rows of just 512 KiB and planes of just 1 MiB, and one value more."""
+    test_grid_planes(nx, ny)
