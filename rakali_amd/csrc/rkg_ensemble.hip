@@ -494,16 +494,21 @@ int rkg_ensemble_autotune(rkg_ensemble* e, int steps, double* best_ms_per_step) 
     const int graph0 = e->use_graph ? 1 : 0;
     const int base_blocks = 4 * e->cus;   // one workgroup per SIMD
     struct Cand { int sched, ty, blocks; };
-    std::vector<Cand> cands;
-    for (int ty : {8, 16, 32, 64}) {
-        cands.push_back({0, ty, 0});
+    // What the ensemble came with first and, in case the first timing was a cold
+    // one, last; then heights from the default rule's least to tall tiles (us a
+    // step at 4 / 8 / 20 / 64 rows: 4 of 64..200 39 / 59 / 122 / 358, 64 of
+    // 128..2048 2123 / 1970 / 1875 / 1911).
+    const Cand entry = {e->schedule, e->ty, e->persistent_blocks};
+    std::vector<Cand> cands{entry};
+    for (int ty : {4, 8, 10, 16, 20, 32, 64}) cands.push_back({0, ty, 0});
+    for (int ty : {8, 16, 32, 64})
         for (int mult : {1, 2}) cands.push_back({1, ty, base_blocks * mult});
-    }
+    cands.push_back(entry);
     hipEvent_t a, b;
     HIP_TRY(hipEventCreate(&a));
     HIP_TRY(hipEventCreate(&b));
     double best = 1e300;
-    Cand win = {e->schedule, e->ty, e->persistent_blocks};
+    Cand win = entry;
     for (const Cand& c : cands) {
         if ((rc = rkg_ensemble_set_schedule(e, c.sched, c.ty, c.blocks, 0))) break;
         ens_steps(e, 1);   // warm-up
@@ -528,7 +533,7 @@ int rkg_ensemble_autotune(rkg_ensemble* e, int steps, double* best_ms_per_step) 
     (void)hipFree(backup);
     (void)hipFree(ctrl_backup);
     if (rc) return rc;
-    rc = rkg_ensemble_set_schedule(e, win.sched, win.ty, win.sched == 1 ? win.blocks : 0, graph0);
+    rc = rkg_ensemble_set_schedule(e, win.sched, win.ty, win.blocks, graph0);
     if (best_ms_per_step) *best_ms_per_step = best;
     return rc;
 }
