@@ -1369,7 +1369,10 @@ struct BwdPlan {
 
 // Rows per workgroup of k_adj_y for a launch over `rows` rows of 64 columns:
 // about 2048 workgroups, two waves on each of the 1024 SIMDs (1024^2 basin,
-// us: 8 rows 48, 7 rows 57, 10 rows 56).
+// us: 8 rows 48, 7 rows 57, 10 rows 56).  The remainder tiles of the strips may
+// make it a few more; a row more per tile, to stay within 2048, is slower
+// (897x1773, 13 rows and 2055 workgroups 70, 14 rows 73; 1947x1453, 22 rows and
+// 2077 workgroups 112, 23 rows 114).
 int adj_y_rows(long long rows) { return (int)std::min<long long>(32, std::max<long long>(4, (rows + 2047) / 2048)); }
 
 int bwd_begin(rkg_adjoint* a, double loss_scale, int tile_rows, BwdPlan& pl) {
