@@ -65,23 +65,24 @@ __device__ __forceinline__ double pow4(double x) { return ((x * x) * x) * x; }
 // Recip keeps the refined reciprocal, so each further quotient by the same
 // denominator costs a product and two fmas and returns the same bits as
 // `n / d`.  The residual is formed as -fma(d, q0, -n) so that zero
-// numerators keep their sign.  The refinement is one cubic step, an fma
-// fewer than two Newton steps: v_rcp_f64 is within 2^-24.3 (measured over
-// 6e9 operands), so y0 (1 + e + e^2) is 1 / d within 2^-72 before its
-// rounding, as close as two steps come in effect; the quotients agreed with
-// the division on all of those operands.  The unscaled sequence equals the
-// IEEE quotient while |n| >= 2^-969 (or n = 0) and the denominator is far
-// from the exponent extremes; callers guarantee the numerator bound by
-// running a row with EXACT = true (plain division) whenever a cell of its
-// stencil holds a value that is unbounded().
+// numerators keep their sign.  Two Newton steps, as the division takes.  One cubic
+// step from v_rcp is an fma less, but leaves 1 / d within 2^-72 before its rounding
+// and so the wrong one of two doubles where 1 / d lies that close to the middle
+// between them: 113 of the 9e6 operands that can tell gave another quotient than
+// the division then (tests/quotients.hip enumerates them).  (The division itself
+// misrounds three of them, all with d of the form 2^k (1 - 5, 11 or 13 2^-53).)
+// The unscaled sequence equals the IEEE quotient while |n| >= 2^-969 (or n = 0)
+// and the denominator is far from the exponent extremes; callers guarantee the
+// numerator bound by running a row with EXACT = true (plain division) whenever a
+// cell of its stencil holds a value that is unbounded().
 struct Recip {
     double d, y;
 };
 
 __device__ __forceinline__ Recip recip(double d) {
     const double y0 = __builtin_amdgcn_rcp(d);
-    const double e = fma(-d, y0, 1.0);
-    return Recip{d, fma(y0, fma(e, e, e), y0)};
+    const double y1 = fma(y0, fma(-d, y0, 1.0), y0);
+    return Recip{d, fma(y1, fma(-d, y1, 1.0), y1)};
 }
 
 template <bool EXACT>
