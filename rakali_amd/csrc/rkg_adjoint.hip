@@ -1634,6 +1634,7 @@ int batch_tables(rkg_adjoint* a, size_t bytes) {
     hipError_t e = hipHostMalloc((void**)&a->batch_host, bytes, hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc((void**)&a->batch_dev, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         if (a->batch_host) (void)hipHostFree(a->batch_host);
         a->batch_host = nullptr;
         a->batch_dev = nullptr;
@@ -1701,8 +1702,9 @@ bool fwd_batchable(int n, rkg_adjoint* const* as) {
 // The forward runs of n sessions on the first session's stream: three
 // launches a step (both stages and the gauge misfits of every member)
 // instead of three per member, which the host could not issue as fast as the
-// GPU ran them.  Every member's arithmetic is that of its own run.
-int fwd_batched(int n, rkg_adjoint* const* as) {
+// GPU ran them.  Every member's arithmetic is that of its own run.  `ran` is false,
+// and nothing has been queued, where there is no memory for the tables.
+int fwd_batched(int n, rkg_adjoint* const* as, bool& ran) {
     const bool hllc = as[0]->g->cfg.use_hllc != 0;
     const int nsteps = as[0]->nsteps, K = as[0]->K;
     hipStream_t S = as[0]->g->stream;
@@ -1724,7 +1726,8 @@ int fwd_batched(int n, rkg_adjoint* const* as) {
     for (int m = 0; m < n; ++m) batch_tiles(d[m], m, tiles);
     const size_t oT = al256(n * sizeof(GridDesc)), oL = oT + al256(tiles.size() * sizeof(BatchTile)),
                  oP = oL + al256((loss.size() + 1) * sizeof(LossArgs)), total = oP + al256(2 * n * sizeof(int));
-    if ((rc = batch_tables(as[0], total))) return rc;
+    if (batch_tables(as[0], total)) return RKG_OK;
+    ran = true;
     char *host = as[0]->batch_host, *dev = as[0]->batch_dev;
     std::memcpy(host, d.data(), n * sizeof(GridDesc));
     std::memcpy(host + oT, tiles.data(), tiles.size() * sizeof(BatchTile));
@@ -2000,12 +2003,10 @@ int rkg_adjoint_forward_many(int n, rkg_adjoint* const* as, double* losses) {
     int rc = check_batch(n, as);
     if (rc) return rc;
     for (int m = 0; m < n && !rc; ++m) rc = fwd_begin(as[m]);
-    if (!rc && fwd_batchable(n, as)) {
-        rc = fwd_batched(n, as);
-    } else {
-        for (int k = 0; k < as[0]->nsteps && !rc; ++k)
-            for (int m = 0; m < n && !rc; ++m) rc = fwd_step(as[m], k);
-    }
+    bool ran = false;
+    if (!rc && fwd_batchable(n, as)) rc = fwd_batched(n, as, ran);
+    for (int k = 0; k < as[0]->nsteps && !rc && !ran; ++k)
+        for (int m = 0; m < n && !rc; ++m) rc = fwd_step(as[m], k);
     for (int m = 0; m < n && !rc; ++m) rc = fwd_end(as[m]);
     if (rc) return rc;
     for (int m = 0; m < n; ++m) HIP_TRY(hipStreamSynchronize(as[m]->g->stream));
