@@ -98,11 +98,6 @@ struct GridDesc {
     CtrlSlot* ctrl;               // [2]
 };
 
-// Boundary data resolved once per launch.
-struct EdgeEta {
-    double tidal;                 // tidal surface at this stage's time
-};
-
 // Tidal surface, rki_boundary.F90:92-101.
 __host__ __device__ __forceinline__ double tidal_eta(const GridDesc& d, double time) {
     double e = 0.0;
