@@ -177,19 +177,21 @@ inline double* field_ptr(rkg_grid* g, int field) {
 // and 20 once there are 8192 tiles of 16, where the uneven end of a launch no
 // longer matters.  Measured (us per step, one grid / each of three grids on
 // their own streams):
-//   200x100    1 row  29 / 11,   3 rows  35 / 14,   6 rows 51 / 19
-//   400x300    1 row  33 / 15,   3 rows  37 / 16,   6 rows 52 / 22
-//   512x512    2 rows 42 / 22,   1 row   50 / 30,   5 rows 48 / 24
-//   701x515    3 rows 47 / 29,   7 rows  60 / 29,  10 rows 76 / 34
-//   800x800    6 rows 72 / 41,   3 rows  73 / 46,  10 rows 90 / 43
-//   1024x1024  10 rows 103 / 60, 5 rows 101 / 65,  19 rows 129 / 69
-//   3000x2000  10 rows 380 / 345, 16 rows 403 / 339
-//   4096x4096  20 rows 976 / 924, 10 rows 1004 / 960, 32 rows 998 / 912
-// and for ensembles (their tiles have 4 rows at least):
-//   4 of 64..200      4 rows 45, 8 rows 65, 32 rows 192
-//   12 of 200..400    10 rows 108, 4 rows 117, 32 rows 204
-//   16 of 128..768    10 rows 250, 20 rows 286, 32 rows 278
-//   32 of 512..1024   20 rows 1207, 10 rows 1301, 32 rows 1208
+//   200x100    1 row  23 / 9,    3 rows  32 / 13,   6 rows 49 / 19
+//   400x300    1 row  31 / 15,   3 rows  33 / 15,   6 rows 49 / 21
+//   512x512    2 rows 42 / 23,   1 row   48 / 31,   5 rows 46 / 23
+//   701x515    3 rows 48 / 27,   7 rows  58 / 28,  10 rows 73 / 33
+//   800x800    6 rows 70 / 40,   3 rows  71 / 45,  10 rows 92 / 43
+//   1024x1024  10 rows 101 / 60, 5 rows  98 / 62,  20 rows 130 / 71
+//   3000x2000  10 rows 370 / 345, 16 rows 403 / 338
+//   4096x4096  20 rows 970 / 914, 10 rows 983 / 950, 32 rows 987 / 908
+// and for ensembles (their tiles have 4 rows at least; nx and ny log-uniform):
+//   4 of 64..200      4 rows 39, 8 rows 60, 32 rows 190
+//   12 of 200..400    10 rows 127, 4 rows 111, 32 rows 203
+//   16 of 128..768    10 rows 196, 20 rows 230, 32 rows 272
+//   64 of 256x256     10 rows 279, 4 rows 291, 32 rows 350
+//   32 of 512..1024   20 rows 1154, 10 rows 1175, 32 rows 1174
+//   64 of 128..2048   20 rows 1926, 10 rows 1979, 32 rows 1931
 template <class TILES>
 int rows_for(TILES tiles, int least) {
     for (int rows = least; rows <= 3; ++rows)
@@ -208,10 +210,10 @@ inline long long grid_tiles(int nx, int ny, int rows) {
 // than the chip's 3072 slots, or where it leaves the fullest of the 1024 SIMDs a
 // wavefront less to run; with as many there a shared wavefront, which reads
 // `pack` rows at a time, is the slower one.  us per step, unpacked / packed:
-//   64x262144 1821 / 1112,  128x131072 1286 / 1053,  256x8192  180 / 162,
-//   128x8192   123 / 102,   64x3000      47 / 39,    2x100000  383 / 81;
+//   64x262144 1821 / 1104,  128x131072 1286 / 1038,  256x8192  180 / 164,
+//   128x8192   123 / 104,   64x3000      47 / 39,    2x100000  383 / 82;
 //   as many on a SIMD: 128x2048 41 / 45, 500x1000 51 / 55, 256x1024 41 / 43;
-//   ensembles of 64 x 256^2 302 / 275, 256 x 128^2 358 / 302, 256 x 64^2 185 / 132
+//   ensembles of 64 x 256^2 302 / 275, 256 x 128^2 358 / 302, 256 x 64^2 185 / 134
 inline bool pack_pays(long long tiles, long long packed) {
     auto fullest = [](long long n) { return (n + 1023) / 1024; };
     return tiles > 3 * 1024 || fullest(packed) < fullest(tiles);
